@@ -132,6 +132,19 @@ OMO_API int omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit(const void* input, i
                                                     const int32_t* scale_offsets, int64_t num_splits,
                                                     int64_t max_split_len, float eps, void* stream);
 
+/* The grouped variant for split lengths the host knows, splits back to back
+ * (split i's rows follow split i - 1's, and so do its output block and scale
+ * rows): m_splits is a HOST array of num_splits lengths summing to rows,
+ * copied into the launch's arguments, so no metadata is copied to the device
+ * and nothing waits for the stream. output_s: sum of ceil(m_splits[i]/128)
+ * rows of N. Outputs equal the device-metadata entry point's. Up to 128
+ * splits, N % 32 == 0, input 16-byte aligned; OMO_ERR_UNSUPPORTED otherwise.
+ * A captured launch keeps the lengths of the capture. */
+OMO_API int omo_hip_Mxfp4RowToBf16ToFp8Col_splits(const void* input, int64_t rows, int64_t row_bytes,
+                                          const void* input_s, int64_t input_s_bytes, void* output_q,
+                                          int64_t output_q_bytes, void* output_s, int64_t output_s_elems,
+                                          const int64_t* m_splits, int64_t num_splits, float eps, void* stream);
+
 /* Fused dual-layout BF16 -> MXFP4 quantize: rowwise codes [rows, cols/2] +
  * scales [rows, cols/32] and columnwise codes [cols, rows/2] + scales
  * [cols, rows/32], the latter equal to the rowwise quantize of the transpose.

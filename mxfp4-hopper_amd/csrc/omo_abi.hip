@@ -300,6 +300,41 @@ int omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit(const void* input, int64_t r
                   fn);
 }
 
+int omo_hip_Mxfp4RowToBf16ToFp8Col_splits(const void* input, int64_t rows, int64_t row_bytes, const void* input_s,
+                                          int64_t input_s_bytes, void* output_q, int64_t output_q_bytes,
+                                          void* output_s, int64_t output_s_elems, const int64_t* m_splits,
+                                          int64_t num_splits, float eps, void* stream) {
+  const char* fn = "omo_Mxfp4RowToBf16ToFp8Col_splits";
+  REQUIRE(rows >= 0 && row_bytes >= 0 && num_splits >= 0, "%s: negative shape", fn);
+  REQUIRE(!std::isnan(eps), "%s: eps is NaN", fn);
+  REQUIRE(row_bytes <= kMaxSize / 2 && size_mul(rows, 2 * row_bytes) >= 0, "%s: shape too large", fn);
+  const int64_t M = rows, N = row_bytes * 2;
+  REQUIRE(num_splits == 0 || m_splits != nullptr, "%s: null split lengths", fn);
+  int64_t total = 0, scale_rows = 0;
+  for (int64_t i = 0; i < num_splits; i++) {
+    REQUIRE(m_splits[i] >= 0 && m_splits[i] <= M - total, "%s: split %lld does not fit the rows", fn, (long long)i);
+    total += m_splits[i];
+    scale_rows += (m_splits[i] + 127) / 128;
+  }
+  REQUIRE(total == M, "%s: the splits sum to %lld of %lld rows", fn, (long long)total, (long long)M);
+  REQUIRE_BUF("input", input, M * row_bytes, M * row_bytes);
+  const int64_t s_need = M == 0 || N == 0 ? 0 : (M - 1) * (N / 32) + (N - 1) / 32 + 1;
+  REQUIRE_BUF("input_s", input_s, input_s_bytes, s_need);
+  REQUIRE_BUF("output_q", output_q, output_q_bytes, M * N);
+  const int64_t out_s_need = size_mul(scale_rows, N);
+  REQUIRE(out_s_need >= 0, "%s: shape too large", fn);
+  REQUIRE_BUF("output_s", output_s, output_s_elems, out_s_need);
+  REQUIRE(aligned(output_s, 4), "%s: misaligned buffer", fn);
+  if (M == 0 || N == 0) return ok();
+  if (!omo_hip::row_to_fp8_col_splits_ok(input, M, N, num_splits))
+    return fail(OMO_ERR_UNSUPPORTED,
+                "%s: takes up to 128 splits of rows of N %% 32 == 0 elements with 16-byte aligned codes; pass device "
+                "metadata to omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit instead", fn);
+  return from_hip(omo_hip::launch_row_to_fp8_col_splits(input, input_s, output_q, static_cast<float*>(output_s), M, N,
+                                                        m_splits, num_splits, scale_rows, eps, as_stream(stream)),
+                  fn);
+}
+
 int omo_hip_quant_mxfp4_dual(const void* input, int64_t rows, int64_t cols, void* row_q, int64_t row_q_bytes,
                              void* row_s, int64_t row_s_bytes, void* col_q, int64_t col_q_bytes, void* col_s,
                              int64_t col_s_bytes, float eps, void* stream) {

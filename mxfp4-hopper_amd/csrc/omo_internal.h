@@ -46,6 +46,14 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
                                         int64_t nsplits, int64_t max_split_len, int64_t out_capacity,
                                         int64_t out_s_rows, float eps, hipStream_t stream);
 
+// Splits back to back with host-known lengths; only for the forms
+// row_to_fp8_col_splits_ok accepts (at most 128 splits, N % 32 == 0, 16 B
+// aligned codes, a grid within the launch limits).
+bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, int64_t nsplits);
+hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,
+                                        int64_t N, const int64_t* lens, int64_t nsplits, int64_t out_s_rows, float eps,
+                                        hipStream_t stream);
+
 // Row-strided variants (bytes between consecutive rows of codes / scales).
 hipError_t launch_quant_rows(const void* x, void* q, int64_t q_stride, void* s, int64_t s_stride, int64_t rows,
                              int64_t K, float eps, hipStream_t stream);

@@ -944,27 +944,65 @@ __device__ __forceinline__ bool band_walk_tile(int xcd, int j, int S, int T, int
   return true;
 }
 
+// Where a wave of the flat grid reads the splits from. load() gives lane l
+// the length, first row and first scale row of splits l + 64k.
+//  * DeviceSplits: three int32 device arrays, any offsets.
+//  * ValueSplits: lengths the host knows, passed by value in the kernel
+//    arguments, the splits back to back: the lane reads one word per split
+//    and two wave sums give the first rows. No device copy of the metadata is
+//    made, which otherwise makes the host wait for everything queued on the
+//    stream before it can enqueue the conversion. 16431 x 7168 in 8 ragged
+//    splits: the kernel 42.4 us against 43.2 with device arrays (kernel
+//    trace), the whole wrapper call 41.0 against 63.9 us back to back.
+struct DeviceSplits {
+  const int32_t* __restrict__ lens;
+  const int32_t* __restrict__ offs;
+  const int32_t* __restrict__ soffs;
+  template <int CHUNKS>
+  __device__ __forceinline__ void load(int nsplits, int (&len)[CHUNKS], int (&start)[CHUNKS],
+                                       int (&sstart)[CHUNKS]) const {
+#pragma unroll
+    for (int k = 0; k < CHUNKS; k++) {
+      const int i = (int)(threadIdx.x & 63) + 64 * k;
+      len[k] = start[k] = sstart[k] = 0;
+      if (i < nsplits) {
+        len[k] = lens[i];
+        start[k] = offs[i];
+        sstart[k] = soffs[i];
+      }
+    }
+  }
+};
+
+struct ValueSplits {
+  int32_t lens[kFlatMaxSplits];  // entries past the last split are 0
+  template <int CHUNKS>
+  __device__ __forceinline__ void load(int, int (&len)[CHUNKS], int (&start)[CHUNKS], int (&sstart)[CHUNKS]) const {
+    int row = 0, srow = 0;  // first rows of chunk k
+#pragma unroll
+    for (int k = 0; k < CHUNKS; k++) len[k] = lens[(threadIdx.x & 63) + 64 * k];
+#pragma unroll
+    for (int k = 0; k < CHUNKS; k++) {
+      const int tiles = (len[k] + kTile - 1) / kTile;
+      const int incl = wave_inclusive_sum(len[k]), tincl = wave_inclusive_sum(tiles);
+      start[k] = row + incl - len[k];
+      sstart[k] = srow + tincl - tiles;
+      row += __builtin_amdgcn_readlane(incl, 63);
+      srow += __builtin_amdgcn_readlane(tincl, 63);
+    }
+  }
+};
+
 // The tile of this workgroup on the flat grid: split, row tile bm and band
 // bn, or false past the last tile (uniform over the workgroup).
 template <int CHUNKS,  // splits per lane: 1 (up to 64 splits) or 2 (up to 128)
-          bool WALK>   // band walk, else ranges
-__device__ __forceinline__ bool flat_split_tile(const int32_t* __restrict__ lens, const int32_t* __restrict__ offs,
-                                                const int32_t* __restrict__ soffs, int nsplits, int tm, int bands,
-                                                int64_t* len, int64_t* start, int64_t* sstart, int64_t* bm,
-                                                int64_t* bn) {
-  const int lane = (int)(threadIdx.x & 63);
+          bool WALK,   // band walk, else ranges
+          typename Splits>
+__device__ __forceinline__ bool flat_split_tile(const Splits& splits, int nsplits, int tm, int bands, int64_t* len,
+                                                int64_t* start, int64_t* sstart, int64_t* bm, int64_t* bn) {
   const int xcd = (int)(blockIdx.x & 7u);
   int len_l[CHUNKS], start_l[CHUNKS], sstart_l[CHUNKS];
-#pragma unroll
-  for (int k = 0; k < CHUNKS; k++) {
-    const int i = lane + 64 * k;
-    len_l[k] = start_l[k] = sstart_l[k] = 0;
-    if (i < nsplits) {
-      len_l[k] = lens[i];
-      start_l[k] = offs[i];
-      sstart_l[k] = soffs[i];
-    }
-  }
+  splits.load(nsplits, len_l, start_l, sstart_l);
   // Each split's share of the numbering, in split order (chunk k's splits
   // follow those of chunks 0 .. k-1): ranges count whole splits' row tiles
   // (times bands below), band walk this XCD's tiles of each split.
@@ -1020,14 +1058,14 @@ __device__ __forceinline__ bool flat_split_tile(const int32_t* __restrict__ lens
   return true;
 }
 
-template <int CHUNKS, bool WALK, bool NARROWN>
+template <int CHUNKS, bool WALK, bool NARROWN, typename Splits>
 __global__ __launch_bounds__(256, 4) void row_to_fp8_col_msplit_flat_kernel(
     const uint8_t* __restrict__ q, const uint8_t* __restrict__ s, uint8_t* __restrict__ out, float* __restrict__ out_s,
-    const int32_t* __restrict__ lens, const int32_t* __restrict__ offs, const int32_t* __restrict__ soffs,
-    int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool out_line, int nsplits, int tm, int bands) {
+    const Splits splits, int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool out_line, int nsplits,
+    int tm, int bands) {
   __shared__ WideSmem sm;
   int64_t len, start, sstart, bm, bn;
-  if (!flat_split_tile<CHUNKS, WALK>(lens, offs, soffs, nsplits, tm, bands, &len, &start, &sstart, &bm, &bn)) return;
+  if (!flat_split_tile<CHUNKS, WALK>(splits, nsplits, tm, bands, &len, &start, &sstart, &bm, &bn)) return;
   msplit_wide_tile<NARROWN>(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, out_line);
 }
 
@@ -1085,11 +1123,11 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_kernel(
 template <int CHUNKS>
 __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_narrow_flat_kernel(
     const uint8_t* __restrict__ q, const uint8_t* __restrict__ s, uint8_t* __restrict__ out, float* __restrict__ out_s,
-    const int32_t* __restrict__ lens, const int32_t* __restrict__ offs, const int32_t* __restrict__ soffs,
-    int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vin, bool vs, int nsplits, int tm, int bands) {
+    const DeviceSplits splits, int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vin, bool vs,
+    int nsplits, int tm, int bands) {
   __shared__ RowColSmem sm;
   int64_t len, start, sstart, bm, bn;
-  if (!flat_split_tile<CHUNKS, false>(lens, offs, soffs, nsplits, tm, bands, &len, &start, &sstart, &bm, &bn)) return;
+  if (!flat_split_tile<CHUNKS, false>(splits, nsplits, tm, bands, &len, &start, &sstart, &bm, &bn)) return;
   msplit_narrow_tile(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, vin, vs);
 }
 
@@ -1124,6 +1162,63 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
                      eps, vin, vs);
 }
 
+// Dynamic LDS, unused, that caps the wide per-split kernel's residency at 4
+// workgroups per CU (6 by its own LDS and registers): fewer tiles' partial
+// output lines wait in L2 at once. Ragged cfg5 splits: 49.6 us against 51.0,
+// and 59.8 against 62.8 right after a 512 MB fill (dirty caches, as in a
+// layer step).
+static size_t split_lds_reserve() {
+  const int per_wg = current_device_caps().lds_per_workgroup / 4 - 2560;
+  return per_wg > (int)sizeof(WideSmem) ? (size_t)(per_wg - (int)sizeof(WideSmem)) : 0;
+}
+
+// The wide flat kernel's form for a split count and width: band walk up to
+// 64 splits on rows of more than 16 bands, else contiguous ranges.
+static bool split_walk(int64_t nsplits, int64_t bands) { return nsplits <= 64 && bands > 16; }
+
+template <typename Splits>
+static auto split_flat_kernel(int64_t nsplits, int64_t bands, bool narrow_n) {
+  const bool walk = split_walk(nsplits, bands);
+  return narrow_n ? (nsplits > 64 ? row_to_fp8_col_msplit_flat_kernel<2, false, true, Splits>
+                     : walk      ? row_to_fp8_col_msplit_flat_kernel<1, true, true, Splits>
+                                 : row_to_fp8_col_msplit_flat_kernel<1, false, true, Splits>)
+                  : (nsplits > 64 ? row_to_fp8_col_msplit_flat_kernel<2, false, false, Splits>
+                     : walk      ? row_to_fp8_col_msplit_flat_kernel<1, true, false, Splits>
+                                 : row_to_fp8_col_msplit_flat_kernel<1, false, false, Splits>);
+}
+
+bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, int64_t nsplits) {
+  return nsplits <= kFlatMaxSplits && N % 32 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0 &&
+         total_rows <= INT32_MAX && total_rows / kTile + nsplits < (int64_t)UINT32_MAX / 256 / (N / kWideCols + 1) - 8;
+}
+
+// Splits back to back with lengths known to the host, in the forms that
+// row_to_fp8_col_splits_ok accepts. The grid holds exactly the tiles there
+// are (device lengths need nsplits times the longest split's).
+hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,
+                                        int64_t N, const int64_t* lens, int64_t nsplits, int64_t out_s_rows, float eps,
+                                        hipStream_t stream) {
+  ValueSplits v;
+  memset(&v, 0, sizeof(v));
+  const int64_t bands = (N + kWideCols - 1) / kWideCols;
+  const bool walk = split_walk(nsplits, bands);
+  int64_t row_tiles = 0, per_xcd = 0;
+  for (int64_t i = 0; i < nsplits; i++) {
+    const int64_t tiles = (lens[i] + kTile - 1) / kTile;
+    v.lens[i] = (int32_t)lens[i];
+    row_tiles += tiles;
+    per_xcd += (tiles * bands + 7) / 8;  // XCD 0 has the largest share of every split
+  }
+  const int64_t grid = walk ? 8 * per_xcd : row_tiles * bands;
+  if (grid == 0) return hipSuccess;
+  const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
+  const bool out_line = (reinterpret_cast<uintptr_t>(out) & 127) == 0;
+  return launch(split_flat_kernel<ValueSplits>(nsplits, bands, narrow_n), dim3((unsigned)grid), dim3(256),
+                split_lds_reserve(), stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
+                static_cast<uint8_t*>(out), out_s, v, total_rows, N, out_s_rows, eps, out_line, (int)nsplits,
+                (int)row_tiles, (int)bands);
+}
+
 hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,
                                         int64_t N, const int32_t* lens, const int32_t* offs, const int32_t* soffs,
                                         int64_t nsplits, int64_t max_split_len, int64_t out_capacity,
@@ -1136,34 +1231,22 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
   const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
   const int64_t tiles_m = (max_split_len + kTile - 1) / kTile;
   const int64_t bands = wide ? (N + kWideCols - 1) / kWideCols : (N + kTile - 1) / kTile;
-  // Unused dynamic LDS caps the wide kernel's residency at 4 workgroups per
-  // CU (6 by its own LDS and registers): fewer tiles' partial output lines
-  // wait in L2 at once. Ragged cfg5 splits: 49.6 us against 51.0, and 59.8
-  // against 62.8 right after a 512 MB fill (dirty caches, as in a layer step).
-  const int per_wg = current_device_caps().lds_per_workgroup / 4 - 2560;
-  const size_t reserve = per_wg > (int)sizeof(WideSmem) ? (size_t)(per_wg - (int)sizeof(WideSmem)) : 0;
+  const size_t reserve = split_lds_reserve();
   const bool out_line = (reinterpret_cast<uintptr_t>(out) & 127) == 0;
+  const DeviceSplits splits{lens, offs, soffs};
   // A launch holds at most 2^32 - 1 work-items along x (gridDim.x times the
   // workgroup size), so the flat grid's limit depends on the kernel's width.
   const int64_t flat_threads = wide ? 256 : kRcThreads;
   if (nsplits <= kFlatMaxSplits && tiles_m * bands + 7 <= (int64_t)UINT32_MAX / flat_threads / nsplits) {
     const dim3 grid((unsigned)flat_grid_blocks(nsplits, tiles_m, bands));
     if (wide) {
-      // band walk up to 64 splits on rows of more than 16 bands, else contiguous ranges
-      const bool walk = nsplits <= 64 && bands > 16;
-      auto kernel = narrow_n ? (nsplits > 64 ? row_to_fp8_col_msplit_flat_kernel<2, false, true>
-                                : walk     ? row_to_fp8_col_msplit_flat_kernel<1, true, true>
-                                           : row_to_fp8_col_msplit_flat_kernel<1, false, true>)
-                             : (nsplits > 64 ? row_to_fp8_col_msplit_flat_kernel<2, false, false>
-                                : walk     ? row_to_fp8_col_msplit_flat_kernel<1, true, false>
-                                           : row_to_fp8_col_msplit_flat_kernel<1, false, false>);
-      return launch(kernel, grid, dim3(256), reserve, stream, static_cast<const uint8_t*>(q),
-                    static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, lens, offs, soffs, total_rows, N,
-                    out_s_rows, eps, out_line, (int)nsplits, (int)tiles_m, (int)bands);
+      return launch(split_flat_kernel<DeviceSplits>(nsplits, bands, narrow_n), grid, dim3(256), reserve, stream,
+                    static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s,
+                    splits, total_rows, N, out_s_rows, eps, out_line, (int)nsplits, (int)tiles_m, (int)bands);
     }
     auto kernel = nsplits <= 64 ? row_to_fp8_col_msplit_narrow_flat_kernel<1> : row_to_fp8_col_msplit_narrow_flat_kernel<2>;
     return launch(kernel, grid, dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),
-                  static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, lens, offs, soffs, total_rows, N,
+                  static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, splits, total_rows, N,
                   out_s_rows, eps, vin, vs, (int)nsplits, (int)tiles_m, (int)bands);
   }
   // Grid y (row tiles) and z (column bands) hold at most 65536 each: longer

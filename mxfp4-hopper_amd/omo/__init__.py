@@ -22,6 +22,8 @@ nothing:
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from ._abi import check as _check
@@ -36,6 +38,7 @@ __all__ = [
     "omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit",
     "omo_per_token_Mxfp4ToFp8_col",
     "omo_per_token_Mxfp4ToFp8",
+    "omo_Mxfp4RowToBf16ToFp8Col_splits",
     "omo_quant_mxfp4_dual",
     "omo_quant_mxfp4_dual_grouped",
     "omo_quant_mxfp4_packed",
@@ -249,6 +252,29 @@ def omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit(input, input_s, output_q, output
             input.data_ptr(), input.size(0), input.size(1), input_s.data_ptr(), input_s.numel(), output_q.data_ptr(),
             output_q.numel(), output_s.data_ptr(), output_s.numel(), m_splits.data_ptr(), split_offsets.data_ptr(),
             scale_offsets.data_ptr(), m_splits.numel(), int(max_split_len), float(eps), stream))
+
+
+def omo_Mxfp4RowToBf16ToFp8Col_splits(input, input_s, output_q, output_s, m_splits, eps):
+    """omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit for splits back to back
+    whose lengths the host knows: ``m_splits`` is a sequence of ints summing to
+    the rows, passed by value with the launch. Up to 128 splits, N % 32 == 0
+    and 16 B aligned codes (NotImplementedError otherwise)."""
+    for t, n in ((input, "input"), (output_q, "output_q")):
+        _check_input(t, n)
+    _same_device(input, input_s, output_q, output_s)
+    _check_input(input_s, "input_s")
+    _check_input(output_s, "output_s")
+    if input.dim() != 2:
+        raise RuntimeError("input must be 2-D [total_M, N/2]")
+    _check_dtype(input, torch.uint8, "input")
+    _check_dtype(input_s, torch.uint8, "input_s")
+    _check_dtype(output_q, _FP8, "output_q")
+    _check_dtype(output_s, torch.float32, "output_s")
+    lens = (ctypes.c_int64 * len(m_splits))(*m_splits)
+    with _on_device(input) as stream:
+        _check(_lib.omo_hip_Mxfp4RowToBf16ToFp8Col_splits(
+            input.data_ptr(), input.size(0), input.size(1), input_s.data_ptr(), input_s.numel(), output_q.data_ptr(),
+            output_q.numel(), output_s.data_ptr(), output_s.numel(), lens, len(m_splits), float(eps), stream))
 
 
 def omo_per_token_group_quant_fp4_fused_ToFp8(input, output_q, output_s, output_bf16_q, output_bf16_s, group_size,

@@ -35,6 +35,8 @@ SIGNATURES = {
                                                  _P],
     "omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _P,
                                                         _I64, _I64, _F, _P],
+    "omo_hip_Mxfp4RowToBf16ToFp8Col_splits": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64,
+                                              ctypes.POINTER(_I64), _I64, _F, _P],
     "omo_hip_quant_mxfp4_dual": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _F, _P],
     "omo_hip_quant_mxfp4_dual_grouped": [ctypes.POINTER(DualItem), _I64, _F, _P],
     "omo_hip_quant_mxfp4_packed": [_P, _I64, _I64, _P, _I64, _F, _P],

@@ -14,6 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from omo import (
+    omo_Mxfp4RowToBf16ToFp8Col_splits,
     omo_per_token_Mxfp4RowToBf16ToFp8Col,
     omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit,
     omo_per_token_Mxfp4ToBf16_dequant,
@@ -159,27 +160,47 @@ def split_metadata(m_splits: List[int], device) -> tuple:
     return meta[0], meta[1], meta[2], (max(lens) if lens else 0), o, so
 
 
+# Most splits that travel with the launch itself.
+MAX_VALUE_SPLITS = 128
+
+
 def omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper(data: torch.Tensor, scale: torch.Tensor,
                                                         m_splits: List[int], eps: float = 1e-10):
     """Reconstructed wrapper of omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit for
     TE's grouped wgrad (code/transformer_engine-2.8.diff:159-176): codes
     [sum(m), N/2] + scales -> (list of fp8 [N, m_i], list of fp32
-    [ceil(m_i/128), N]), one per expert split, each a view of one buffer."""
+    [ceil(m_i/128), N]), one per expert split, each a view of one buffer.
+
+    Up to 128 splits of 16 B aligned code rows travel by value with the
+    launch. More splits, and rows the 256-column tiles do not take, go through
+    a device copy of the metadata, for which the host waits."""
     assert data.dim() == 2 and data.is_contiguous(), "`data` must be a contiguous 2-D tensor"
     total_m, half = data.shape
     N = half * 2
-    lens, offs, soffs, max_len, rows, srows = split_metadata(m_splits, data.device)
+    by_value = len(m_splits) <= MAX_VALUE_SPLITS and N % 32 == 0 and data.data_ptr() % 16 == 0 and total_m < 2**31
+    if by_value:
+        lens = [int(m) for m in m_splits]
+        if any(m < 0 for m in lens):
+            raise ValueError(f"m_splits must be non-negative, got {lens}")
+        rows, tiles = sum(lens), [(m + 127) // 128 for m in lens]
+        srows = sum(tiles)
+    else:
+        lens, offs, soffs, max_len, rows, srows = split_metadata(m_splits, data.device)
+        tiles = [(int(m) + 127) // 128 for m in m_splits]
     if rows != total_m:
         raise ValueError(f"sum(m_splits)={rows} does not match data rows {total_m}")
     out_q = torch.empty(total_m * N, device=data.device, dtype=fp8_type_)
     out_s = torch.empty((srows, N), device=data.device, dtype=torch.float)
     if len(m_splits) > 0 and N > 0 and total_m > 0:
-        omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit(data, scale.contiguous(), out_q, out_s, lens, offs, soffs, max_len,
-                                                    eps)
+        if by_value:
+            omo_Mxfp4RowToBf16ToFp8Col_splits(data, scale.contiguous(), out_q, out_s, lens, eps)
+        else:
+            omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit(data, scale.contiguous(), out_q, out_s, lens, offs, soffs,
+                                                        max_len, eps)
     y_data, y_scale, o = [], [], 0
     for m in m_splits:
         m = int(m)
         y_data.append(out_q[o * N:(o + m) * N].view(N, m))
         o += m
-    y_scale = list(torch.split(out_s, [(int(m) + 127) // 128 for m in m_splits], dim=0))
+    y_scale = list(torch.split(out_s, tiles, dim=0))
     return y_data, y_scale
