@@ -234,6 +234,24 @@ OMO_API int omo_hip_permute_Mxfp4ToFp8(const void* codes, int64_t codes_bytes, i
                                        void* output_q, int64_t output_q_bytes, void* output_s,
                                        int64_t output_s_elems, void* stream);
 
+/* Expert-major row order of a MoE routing map (the row map of TE's
+ * moe_permute, code/transformer_engine-2.8.diff:220-356). map [tokens,
+ * experts], one byte per pair, non-zero where routed; fewer than 2^31 pairs.
+ * Two calls in stream order:
+ *   omo_hip_route_counts: counts [experts, omo_hip_route_chunks(tokens, experts)]
+ *     (int32), the routed tokens of each expert per chunk of tokens; an
+ *     expert's row sums to its load.
+ *   omo_hip_route_rows: src_rows[r] = token of the r-th routed pair by
+ *     expert, then token (pairs past src_elems are dropped; with pad, the
+ *     entries after the last pair are set to -1), and, where dest is not
+ *     NULL, dest[t * experts + e] = r, or -1 where the pair is not routed. */
+OMO_API int64_t omo_hip_route_chunks(int64_t tokens, int64_t experts);
+OMO_API int omo_hip_route_counts(const void* map, int64_t tokens, int64_t experts, int32_t* counts,
+                                 int64_t counts_elems, void* stream);
+OMO_API int omo_hip_route_rows(const void* map, int64_t tokens, int64_t experts, const int32_t* counts,
+                               int64_t counts_elems, int32_t* src_rows, int64_t src_elems, int pad, int32_t* dest,
+                               int64_t dest_elems, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

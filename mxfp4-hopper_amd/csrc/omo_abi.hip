@@ -123,6 +123,18 @@ int check_permute(const char* fn, const void* codes, int64_t codes_bytes, int64_
   return OMO_OK;
 }
 
+// Shared checks of the routing entry points.
+int check_route(const char* fn, const void* map, int64_t tokens, int64_t experts, const void* counts,
+                int64_t counts_elems) {
+  REQUIRE(tokens >= 0 && experts >= 0, "%s: negative shape", fn);
+  const int64_t pairs = size_mul(tokens, experts);
+  REQUIRE(pairs >= 0 && pairs < ((int64_t)1 << 31) && experts <= 4 * 65534, "%s: routing map too large", fn);
+  REQUIRE_BUF("routing map", map, pairs, pairs);
+  REQUIRE_BUF("counts", counts, counts_elems, pairs == 0 ? 0 : experts * omo_hip::route_chunks(tokens, experts));
+  REQUIRE(aligned(counts, 4), "%s: counts must be 4-byte aligned", fn);
+  return OMO_OK;
+}
+
 // Checks of one dual-layout quantize (single or grouped).
 int check_dual(const char* fn, const void* input, int64_t rows, int64_t cols, const void* row_q, int64_t row_q_bytes,
                const void* row_s, int64_t row_s_bytes, const void* col_q, int64_t col_q_bytes, const void* col_s,
@@ -441,6 +453,37 @@ int omo_hip_mxfp4_permute_rows(const void* codes, int64_t codes_bytes, int64_t c
   return from_hip(omo_hip::launch_gather_rows(codes, code_stride, cols / 2, scales, scale_stride, cols / 32,
                                               src_rows, num_tokens, num_out, out_codes, out_scales,
                                               as_stream(stream)),
+                  fn);
+}
+
+int64_t omo_hip_route_chunks(int64_t tokens, int64_t experts) {
+  return tokens > 0 && experts > 0 ? omo_hip::route_chunks(tokens, experts) : 0;
+}
+
+int omo_hip_route_counts(const void* map, int64_t tokens, int64_t experts, int32_t* counts, int64_t counts_elems,
+                         void* stream) {
+  const char* fn = "omo_route_counts";
+  int rc = check_route(fn, map, tokens, experts, counts, counts_elems);
+  if (rc != OMO_OK) return rc;
+  if (tokens == 0 || experts == 0) return ok();
+  return from_hip(omo_hip::launch_route_counts(map, tokens, experts, counts, as_stream(stream)), fn);
+}
+
+int omo_hip_route_rows(const void* map, int64_t tokens, int64_t experts, const int32_t* counts, int64_t counts_elems,
+                       int32_t* src_rows, int64_t src_elems, int pad, int32_t* dest, int64_t dest_elems,
+                       void* stream) {
+  const char* fn = "omo_route_rows";
+  int rc = check_route(fn, map, tokens, experts, counts, counts_elems);
+  if (rc != OMO_OK) return rc;
+  REQUIRE(src_elems >= 0 && src_elems < ((int64_t)1 << 31), "%s: bad src_rows size", fn);
+  REQUIRE(src_elems == 0 || src_rows != nullptr, "%s: src_rows: null pointer", fn);
+  if (dest) REQUIRE_BUF("dest", dest, dest_elems, tokens * experts);
+  REQUIRE(aligned(src_rows, 4) && aligned(dest, 4), "%s: misaligned buffer", fn);
+  REQUIRE(!pad || tokens > 0 || src_elems == 0, "%s: no tokens to pad after", fn);
+  REQUIRE(!pad || experts > 0 || src_elems == 0, "%s: no experts to pad after", fn);
+  if (tokens == 0 || experts == 0) return ok();
+  return from_hip(omo_hip::launch_route_rows(map, tokens, experts, counts, src_rows, src_elems, pad != 0, dest,
+                                             as_stream(stream)),
                   fn);
 }
 

@@ -1,0 +1,51 @@
+"""The row map of a routing map by the HIP kernels against the torch
+composition of the same map on the CPU: whole numbers, so every value."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _map(T, E, p, seed):
+    return torch.rand((T, E), generator=torch.Generator().manual_seed(seed)) < p
+
+
+# One token, one expert; experts that are not a multiple of the four of a
+# workgroup; token counts around a wave (64), a workgroup step (256) and
+# several steps per chunk (more than 64 or, with many experts, 8 chunks);
+# nothing routed and everything routed.
+@pytest.mark.parametrize("T,E,p", [(1, 1, 1.0), (1, 1, 0.0), (63, 3, 0.5), (64, 4, 0.3), (65, 5, 1.0), (256, 64, 0.125),
+                                   (257, 6, 0.4), (4096, 64, 0.125), (16640, 8, 0.2), (40000, 2, 0.5),
+                                   (5000, 520, 0.02)])
+@pytest.mark.parametrize("pad", [None, 0, 7, 3000])
+def test_row_map(dev, T, E, p, pad):
+    from omo_python_api.permutation import make_row_id_map
+    print("row map", T, E, p, pad, flush=True)
+    rm = _map(T, E, p, T + E)
+    num_out = None if pad is None else int(rm.sum()) + pad
+    src, m_splits, dest = make_row_id_map(rm.to(dev), num_out)
+    es, em, ed = make_row_id_map(rm, num_out)
+    assert m_splits == em and all(isinstance(m, int) for m in m_splits)
+    assert src.dtype == es.dtype and dest.dtype == ed.dtype and src.is_contiguous()
+    assert torch.equal(src.cpu(), es) and torch.equal(dest.cpu(), ed)
+    assert src.untyped_storage().nbytes() == 4 * src.numel()
+
+
+def test_row_map_forms(dev):
+    """Strided and misaligned maps, 0/1 maps of other types, too few rows."""
+    from omo_python_api.permutation import make_row_id_map
+    rm = _map(300, 12, 0.3, 1)
+    es, em, ed = make_row_id_map(rm)
+    wide = torch.zeros((300, 20), dtype=torch.bool, device=dev)
+    wide[:, 3:15] = rm.to(dev)
+    flat = torch.zeros(300 * 12 + 1, dtype=torch.bool, device=dev)
+    flat[1:] = rm.to(dev).view(-1)
+    forms = [wide[:, 3:15], flat[1:].view(300, 12), rm.to(dev).t().contiguous().t(), rm.to(dev).int(), rm.to(dev).float()]
+    for f in forms:
+        src, m_splits, dest = make_row_id_map(f)
+        assert m_splits == em and torch.equal(src.cpu(), es) and torch.equal(dest.cpu(), ed)
+    with pytest.raises(ValueError, match="smaller"):
+        make_row_id_map(rm.to(dev), int(rm.sum()) - 1)
+    for T, E in ((0, 4), (4, 0)):
+        src, m_splits, dest = make_row_id_map(torch.zeros((T, E), dtype=torch.bool, device=dev), 3)
+        assert src.tolist() == [-1] * 3 and m_splits == [0] * E and dest.shape == (T, E)
