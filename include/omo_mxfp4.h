@@ -91,6 +91,17 @@ OMO_API int omo_hip_per_token_Mxfp4ToBf16ToFp8(const void* input, int64_t rows, 
                                        int64_t output_s_elems, int group_size, float eps, float fp4_min,
                                        float fp4_max, int scale_ue8m0, void* stream);
 
+/* omo_hip_per_token_Mxfp4ToFp8 of rows that may end inside a 128-element
+ * group (row_bytes % 16 == 0): the outputs, padding included, are those of
+ * codes padded with zeros to P = row_bytes rounded up to 64 bytes and scales
+ * to P/16, as the reference's wrapper pads them (code/kernel/api/mxfp4_dequant.py:122-187),
+ * without the padded copies. input: [rows, row_bytes] (8-byte aligned);
+ * input_s: rows*row_bytes/16 bytes; output_q: [rows, 2*P] fp8 (16-byte
+ * aligned); output_s: rows*P/64 floats; rows*P % 128 == 0. */
+OMO_API int omo_hip_Mxfp4ToFp8_padded(const void* input, int64_t rows, int64_t row_bytes, const void* input_s,
+                              int64_t input_s_bytes, void* output_q, int64_t output_q_bytes, void* output_s,
+                              int64_t output_s_elems, void* stream);
+
 /* MXFP4 rowwise -> FP8 transposed [2*row_bytes, rows] with 128-row
  * power-of-two scales [rows/128, 2*row_bytes] (sign dropped, as the reference).
  * Replaces omo::omo_per_token_Mxfp4ToFp8_col

@@ -72,20 +72,25 @@ int check_requant_common(const char* fn, const void* input, int64_t rows, int64_
   return OMO_OK;
 }
 
-int requant_rowwise(const char* fn, const void* input, int64_t rows, int64_t row_bytes, const void* input_s,
-                    int64_t input_s_bytes, void* output_q, int64_t output_q_bytes, void* output_s,
+// multiple: what row_bytes has to divide by (64, or 16 where rows that end
+// inside a group count as zero-padded to 64 bytes).
+int requant_rowwise(const char* fn, int64_t multiple, const void* input, int64_t rows, int64_t row_bytes,
+                    const void* input_s, int64_t input_s_bytes, void* output_q, int64_t output_q_bytes, void* output_s,
                     int64_t output_s_elems, int scale_ue8m0, void* stream) {
-  int rc = check_requant_common(fn, input, rows, row_bytes, scale_ue8m0);
+  REQUIRE(row_bytes <= kMaxSize, "%s: shape too large", fn);
+  const int64_t padded = row_bytes > 0 && multiple < 64 ? (row_bytes + 63) / 64 * 64 : row_bytes;
+  int rc = check_requant_common(fn, input, rows, padded, scale_ue8m0);
   if (rc != OMO_OK) return rc;
-  REQUIRE(row_bytes % 64 == 0, "%s: row bytes must be a multiple of 64 (got %lld); pad as the wrapper does", fn,
-          (long long)row_bytes);
-  const int64_t n = rows * row_bytes;
+  REQUIRE(row_bytes % multiple == 0, "%s: row bytes must be a multiple of %lld (got %lld); pad as the wrapper does", fn,
+          (long long)multiple, (long long)row_bytes);
+  const int64_t n = rows * row_bytes, np = rows * padded;
   REQUIRE_BUF("input", input, n, n);
   REQUIRE_BUF("input_s", input_s, input_s_bytes, n / 16);
-  REQUIRE_BUF("output_q", output_q, output_q_bytes, 2 * n);
-  REQUIRE_BUF("output_s", output_s, output_s_elems, n / 64);
-  REQUIRE(n / 64 < (int64_t)1 << 31, "%s: too many 128-element groups", fn);
-  REQUIRE(aligned(input, 8) && aligned(input_s, 4) && aligned(output_q, 16) && aligned(output_s, 4),
+  REQUIRE_BUF("output_q", output_q, output_q_bytes, 2 * np);
+  REQUIRE_BUF("output_s", output_s, output_s_elems, np / 64);
+  REQUIRE(np / 64 < (int64_t)1 << 31, "%s: too many 128-element groups", fn);
+  REQUIRE(aligned(input, 8) && (aligned(input_s, 4) || padded != row_bytes) && aligned(output_q, 16) &&
+              aligned(output_s, 4),
           "%s: misaligned buffer (input needs 8 B, input_s 4 B, output_q 16 B)", fn);
   if (n == 0) return ok();
   return from_hip(omo_hip::launch_mxfp4_to_fp8(input, input_s, output_q, static_cast<float*>(output_s), rows,
@@ -216,7 +221,7 @@ int omo_hip_per_token_Mxfp4ToFp8(const void* input, int64_t rows, int64_t row_by
                                  int64_t output_s_elems, int group_size, float eps, float fp4_min, float fp4_max,
                                  int scale_ue8m0, void* stream) {
   (void)group_size; (void)eps; (void)fp4_min; (void)fp4_max;
-  return requant_rowwise("omo_per_token_Mxfp4ToFp8", input, rows, row_bytes, input_s, input_s_bytes, output_q,
+  return requant_rowwise("omo_per_token_Mxfp4ToFp8", 64, input, rows, row_bytes, input_s, input_s_bytes, output_q,
                          output_q_bytes, output_s, output_s_elems, scale_ue8m0, stream);
 }
 
@@ -225,8 +230,15 @@ int omo_hip_per_token_Mxfp4ToBf16ToFp8(const void* input, int64_t rows, int64_t 
                                        int64_t output_s_elems, int group_size, float eps, float fp4_min,
                                        float fp4_max, int scale_ue8m0, void* stream) {
   (void)group_size; (void)eps; (void)fp4_min; (void)fp4_max;
-  return requant_rowwise("omo_per_token_Mxfp4ToBf16ToFp8", input, rows, row_bytes, input_s, input_s_bytes, output_q,
+  return requant_rowwise("omo_per_token_Mxfp4ToBf16ToFp8", 64, input, rows, row_bytes, input_s, input_s_bytes, output_q,
                          output_q_bytes, output_s, output_s_elems, scale_ue8m0, stream);
+}
+
+int omo_hip_Mxfp4ToFp8_padded(const void* input, int64_t rows, int64_t row_bytes, const void* input_s,
+                              int64_t input_s_bytes, void* output_q, int64_t output_q_bytes, void* output_s,
+                              int64_t output_s_elems, void* stream) {
+  return requant_rowwise("omo_Mxfp4ToFp8_padded", 16, input, rows, row_bytes, input_s, input_s_bytes, output_q,
+                         output_q_bytes, output_s, output_s_elems, 0, stream);
 }
 
 int omo_hip_per_token_Mxfp4ToFp8_col(const void* input, int64_t rows, int64_t row_bytes, const void* input_s,

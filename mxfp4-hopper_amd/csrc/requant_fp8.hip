@@ -122,12 +122,20 @@ constexpr int kRqRowsSmall = 8;
 // ROWS64: rows addressed with 64-bit products (a gather, or strides or
 // output rows of 2^24 bytes and more); otherwise addresses are a
 // workgroup-uniform tile base plus 32-bit lane offsets (24-bit products).
-template <int ROWS, bool ALIGN8, bool ROWS64>
+// TAIL: the input rows end inside the last group: kb code bytes (a multiple
+// of 16) and ks = kb / 16 scale bytes a row. The output is that of rows
+// padded with zero codes and zero scale bytes to whole groups: pairs past the
+// row read its last pair and are zeroed, and a group's four scale bytes, at
+// any byte alignment, are read as one dword that ends at the row's end at the
+// latest, shifted down. Padding by torch first (two fills, two copies, then
+// this kernel) took 23 us of kernels at 4096 x 2880, this form 6.
+template <int ROWS, bool ALIGN8, bool ROWS64, bool TAIL>
 __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __restrict__ q, int64_t q_stride,
                                                            const uint8_t* __restrict__ s, int64_t s_stride,
                                                            const int32_t* __restrict__ src, int64_t n_src,
                                                            u32x4* __restrict__ out, float* __restrict__ out_s,
-                                                           uint32_t M, uint32_t gpr, uint32_t gx) {
+                                                           uint32_t M, uint32_t gpr, uint32_t gx, uint32_t kb,
+                                                           uint32_t ks) {
   constexpr int PPR = 8 * kRqGroups;  // pairs per tile row
   constexpr int UNROLL = ROWS * PPR / 256;
   constexpr int RSTEP = 256 / PPR;    // rows between one lane's pairs
@@ -136,7 +144,10 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
   const uint32_t t = threadIdx.x;
   const uint32_t row0 = by * ROWS;                 // first row of the tile
   const uint32_t cp = bx * PPR + t % PPR;          // the lane's pair column, the same in each of its rows
-  const uint32_t cpc = min(cp, 8 * gpr - 1);
+  const uint32_t cpc = min(cp, (TAIL ? kb / 8 : 8 * gpr) - 1);
+  // the lane's scale dword: byte offset in the row, and how far down its bytes move
+  const uint32_t so = TAIL ? min(4 * (cpc >> 3), max(ks, 4u) - 4) : 4 * (cpc >> 3);
+  const uint32_t sdown = TAIL ? 8 * (4 * (cpc >> 3) - so) : 0;
   const uint32_t lr0 = t / PPR;                    // the lane's first row within the tile
   // Every load is issued at clamped in-bounds indices (and zeroed afterwards
   // for a padding row): loads under a per-lane branch made the compiler wait
@@ -159,7 +170,7 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
       pad[u] = sr[u] < 0 || sr[u] >= n_src;
       const int64_t row = pad[u] ? 0 : sr[u];
       qp[u] = q + row * q_stride + 8 * cpc;
-      sp[u] = s + row * s_stride + 4 * (cpc >> 3);
+      sp[u] = s + row * s_stride + so;
     }
   } else {
     const uint8_t* qt = q + (int64_t)row0 * q_stride;
@@ -168,7 +179,7 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
     for (int u = 0; u < UNROLL; u++) {
       const uint32_t lr = min(row0 + lr0 + u * RSTEP, M - 1) - row0;
       qp[u] = qt + (__umul24(lr, (uint32_t)q_stride) + 8 * cpc);
-      sp[u] = st + (__umul24(lr, (uint32_t)s_stride) + 4 * (cpc >> 3));
+      sp[u] = st + (__umul24(lr, (uint32_t)s_stride) + so);
       pad[u] = false;
     }
   }
@@ -183,7 +194,15 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
         c[u][0] = *reinterpret_cast<const uint32_t*>(qp[u]);
         c[u][1] = *reinterpret_cast<const uint32_t*>(qp[u] + 4);
       }
-      sd[u] = *reinterpret_cast<const uint32_t*>(sp[u]);
+      if (!TAIL) {
+        sd[u] = *reinterpret_cast<const uint32_t*>(sp[u]);
+      } else if (ks >= 4) {
+        __builtin_memcpy(&sd[u], sp[u], 4);
+      } else {  // rows of one to three blocks
+        sd[u] = sp[u][0];
+        if (ks > 1) sd[u] |= (uint32_t)sp[u][1] << 8;
+        if (ks > 2) sd[u] |= (uint32_t)sp[u][2] << 16;
+      }
     }
   } else {
 #pragma unroll
@@ -192,6 +211,10 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
 #pragma unroll
   for (int u = 0; u < UNROLL; u++) {
     if (pad[u]) c[u][0] = c[u][1] = sd[u] = 0u;
+    if (TAIL) {
+      sd[u] >>= sdown;
+      if (8 * cp >= kb) c[u][0] = c[u][1] = 0u;
+    }
   }
   const uint32_t sh = 8 * ((t & 7u) >> 1);  // byte of s_i in the group's scale dword (cp & 7 == t & 7)
   u32x4* ot = out + (int64_t)row0 * (8 * (int64_t)gpr) + bx * PPR;
@@ -242,7 +265,8 @@ hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void*
                                     const int32_t* src, int64_t n_src, void* out, float* out_s, int64_t M, int64_t Kb,
                                     hipStream_t stream) {
   if (M == 0 || Kb == 0) return hipSuccess;
-  const int64_t gpr = Kb / 64;
+  const int64_t gpr = (Kb + 63) / 64;
+  const bool tail = Kb % 64 != 0;
   const int64_t gx = (gpr + kRqGroups - 1) / kRqGroups;
   const bool small = gx * ((M + kRqRows - 1) / kRqRows) < 2 * (int64_t)current_device_caps().cus;
   // Without a gather, 16-row tiles (two pairs per lane, twice the workgroups)
@@ -253,21 +277,27 @@ hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void*
   const int rows = small ? kRqRowsSmall : (src ? kRqRows : kRqRowsPlain);
   const int64_t gy = (M + rows - 1) / rows;
   const bool a8 = (q_stride % 8 == 0) && ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
-  const bool r64 = src || q_stride >= (1 << 24) || s_stride >= (1 << 24) || 2 * Kb >= (1 << 24);
+  const bool r64 = src || q_stride >= (1 << 24) || s_stride >= (1 << 24) || 128 * gpr >= (1 << 24);
   using Kernel = void (*)(const uint8_t*, int64_t, const uint8_t*, int64_t, const int32_t*, int64_t, u32x4*, float*,
-                          uint32_t, uint32_t, uint32_t);
+                          uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
   // [rows: 8, 16, 32][a8][r64]
   static const Kernel table[3][2][2] = {
-      {{mxfp4_to_fp8_kernel<kRqRowsSmall, false, false>, mxfp4_to_fp8_kernel<kRqRowsSmall, false, true>},
-       {mxfp4_to_fp8_kernel<kRqRowsSmall, true, false>, mxfp4_to_fp8_kernel<kRqRowsSmall, true, true>}},
-      {{mxfp4_to_fp8_kernel<kRqRowsPlain, false, false>, mxfp4_to_fp8_kernel<kRqRowsPlain, false, true>},
-       {mxfp4_to_fp8_kernel<kRqRowsPlain, true, false>, mxfp4_to_fp8_kernel<kRqRowsPlain, true, true>}},
-      {{mxfp4_to_fp8_kernel<kRqRows, false, false>, mxfp4_to_fp8_kernel<kRqRows, false, true>},
-       {mxfp4_to_fp8_kernel<kRqRows, true, false>, mxfp4_to_fp8_kernel<kRqRows, true, true>}}};
+      {{mxfp4_to_fp8_kernel<kRqRowsSmall, false, false, false>, mxfp4_to_fp8_kernel<kRqRowsSmall, false, true, false>},
+       {mxfp4_to_fp8_kernel<kRqRowsSmall, true, false, false>, mxfp4_to_fp8_kernel<kRqRowsSmall, true, true, false>}},
+      {{mxfp4_to_fp8_kernel<kRqRowsPlain, false, false, false>, mxfp4_to_fp8_kernel<kRqRowsPlain, false, true, false>},
+       {mxfp4_to_fp8_kernel<kRqRowsPlain, true, false, false>, mxfp4_to_fp8_kernel<kRqRowsPlain, true, true, false>}},
+      {{mxfp4_to_fp8_kernel<kRqRows, false, false, false>, mxfp4_to_fp8_kernel<kRqRows, false, true, false>},
+       {mxfp4_to_fp8_kernel<kRqRows, true, false, false>, mxfp4_to_fp8_kernel<kRqRows, true, true, false>}}};
+  // rows ending inside a group (no gather, 8 B aligned rows): [rows: 8, 16][r64]
+  static const Kernel tails[2][2] = {
+      {mxfp4_to_fp8_kernel<kRqRowsSmall, true, false, true>, mxfp4_to_fp8_kernel<kRqRowsSmall, true, true, true>},
+      {mxfp4_to_fp8_kernel<kRqRowsPlain, true, false, true>, mxfp4_to_fp8_kernel<kRqRowsPlain, true, true, true>}};
+  if (tail && (src || !a8)) return hipErrorInvalidValue;
   const int ri = rows == kRqRowsSmall ? 0 : rows == kRqRowsPlain ? 1 : 2;
-  return launch(table[ri][a8][r64], dim3((unsigned)(gx * gy)), dim3(256), 0, stream,
+  return launch(tail ? tails[ri][r64] : table[ri][a8][r64], dim3((unsigned)(gx * gy)), dim3(256), 0, stream,
                 static_cast<const uint8_t*>(q), q_stride, static_cast<const uint8_t*>(s), s_stride, src, n_src,
-                static_cast<u32x4*>(out), out_s, (uint32_t)M, (uint32_t)gpr, (uint32_t)gx);
+                static_cast<u32x4*>(out), out_s, (uint32_t)M, (uint32_t)gpr, (uint32_t)gx, (uint32_t)Kb,
+                (uint32_t)(Kb / 16));
 }
 
 hipError_t launch_mxfp4_to_fp8(const void* q, const void* s, void* out, float* out_s, int64_t M, int64_t Kb,

@@ -39,6 +39,7 @@ __all__ = [
     "omo_per_token_Mxfp4ToFp8_col",
     "omo_per_token_Mxfp4ToFp8",
     "omo_Mxfp4RowToBf16ToFp8Col_splits",
+    "omo_Mxfp4ToFp8_padded",
     "omo_quant_mxfp4_dual",
     "omo_quant_mxfp4_dual_grouped",
     "omo_quant_mxfp4_packed",
@@ -191,6 +192,27 @@ def omo_per_token_Mxfp4ToBf16ToFp8(input, input_s, output_q, output_s, group_siz
     same signature and call site shape as omo_per_token_Mxfp4ToFp8, computed by it."""
     _requant_rowwise(_lib.omo_hip_per_token_Mxfp4ToBf16ToFp8, "omo_per_token_Mxfp4ToBf16ToFp8", input, input_s,
                      output_q, output_s, group_size, eps, fp4_min, fp4_max, scale_ue8m0)
+
+
+def omo_Mxfp4ToFp8_padded(input, input_s, output_q, output_s):
+    """omo_per_token_Mxfp4ToFp8 of rows [M, K/2] whose width K % 32 == 0 may
+    end inside a 128-element group: writes the outputs of the zero-padded rows
+    (output_q [M, Kp], output_s [Kp/128, M], Kp = K rounded up to 128)."""
+    _check_input(input, "input")
+    _check_input(output_q, "output_q")
+    if input.dim() != 2:
+        raise RuntimeError("omo_Mxfp4ToFp8_padded: input must be 2-D [M, K/2]")
+    _same_device(input, input_s, output_q, output_s)
+    _check_input(input_s, "input_s")
+    _check_input(output_s, "output_s")
+    _check_dtype(input, torch.uint8, "input")
+    _check_dtype(input_s, torch.uint8, "input_s")
+    _check_dtype(output_q, _FP8, "output_q")
+    _check_dtype(output_s, torch.float32, "output_s")
+    with _on_device(input) as stream:
+        _check(_lib.omo_hip_Mxfp4ToFp8_padded(
+            input.data_ptr(), input.size(0), input.size(1), input_s.data_ptr(), input_s.numel(), output_q.data_ptr(),
+            output_q.numel(), output_s.data_ptr(), output_s.numel(), stream))
 
 
 def omo_per_token_Mxfp4ToFp8_col(input, input_s, output_q, output_s, group_size, eps, fp4_min, fp4_max, scale_ue8m0):

@@ -30,6 +30,7 @@ SIGNATURES = {
     "omo_hip_per_token_Mxfp4ToBf16_dequant": [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_per_token_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_per_token_Mxfp4ToBf16ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
+    "omo_hip_Mxfp4ToFp8_padded": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],
     "omo_hip_per_token_Mxfp4ToFp8_col": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_per_token_Mxfp4RowToBf16ToFp8Col": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _F,
                                                  _P],

@@ -15,6 +15,7 @@ import torch.nn.functional as F
 
 from omo import (
     omo_Mxfp4RowToBf16ToFp8Col_splits,
+    omo_Mxfp4ToFp8_padded,
     omo_per_token_Mxfp4RowToBf16ToFp8Col,
     omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit,
     omo_per_token_Mxfp4ToBf16_dequant,
@@ -83,23 +84,42 @@ def omo_per_token_mxfp4ToBf16ToFp8_wrapper(x: torch.Tensor, x_in_s: torch.Tensor
     return x_q, x_s
 
 
+def _pads_in_kernel(x: torch.Tensor, x_in_s: torch.Tensor) -> bool:
+    """Whether the FP8 requant can read these rows unpadded: they end inside a
+    128-element group, on a whole 32-element block, with one contiguous scale
+    row of their own width each. Anything else is padded by torch first."""
+    if x.dim() != 2 or x.shape[1] % 16 != 0:
+        return False
+    rows, half = x.shape
+    return (tuple(x_in_s.shape) == (rows, half // 16) and x_in_s.is_contiguous() and x.dtype == x_in_s.dtype == uint8_type
+            and x.is_cuda and x.device == x_in_s.device and x.data_ptr() % 8 == 0
+            and rows * ((half + 63) // 64) % 2 == 0)  # what the kernel refuses is refused by the padded route
+
+
 def omo_per_token_mxfp4ToFp8_wrapper(x: torch.Tensor, x_in_s: torch.Tensor, m_splits: List[int] = None):
     """mxfp4_dequant.py:122-187 (called at code/transformer_engine-2.8.diff:163):
     codes padded to 64 bytes and scales to 4 columns, fp8 [M, 2Kp] + fp32
     [2Kp/128, M], sliced, then split by m_splits along rows (fp8, dim 0) and
-    columns (scales, dim 1)."""
+    columns (scales, dim 1). Widths K % 32 == 0 are padded inside the kernel."""
     group_size = 128
     eps = 1e-10
     scale_ue8m0 = False
     assert x.is_contiguous(), "`x` is not contiguous"
-    x_padded, original_w = pad_to_multiple(x, multiple=64)
-    x_in_s_pad, original_w_scale = pad_to_multiple(x_in_s, multiple=4)
-    out_shape = (*x_padded.shape[:-1], x_padded.shape[-1] * 2)
-    scale_shape = ((x_padded.shape[-1] * 2 // 128), *x_padded.shape[:-1])
+    original_w, original_w_scale = x.shape[-1], x_in_s.shape[-1]
+    in_kernel = original_w % 64 != 0 and _pads_in_kernel(x, x_in_s)
+    padded_w = (original_w + 63) // 64 * 64
+    out_shape = (*x.shape[:-1], padded_w * 2)
+    scale_shape = ((padded_w * 2 // 128), *x.shape[:-1])
     x_q = torch.empty(out_shape, device=x.device, dtype=fp8_type_)
     x_s = torch.empty(scale_shape, device=x.device, dtype=torch.float)
     if x.shape[0] > 0:
-        omo_per_token_Mxfp4ToFp8(x_padded, x_in_s_pad, x_q, x_s, group_size, eps, mxfp4_min, mxfp4_max, scale_ue8m0)
+        if in_kernel:
+            omo_Mxfp4ToFp8_padded(x, x_in_s, x_q, x_s)
+        else:
+            x_padded, _ = pad_to_multiple(x, multiple=64)
+            x_in_s_pad, _ = pad_to_multiple(x_in_s, multiple=4)
+            omo_per_token_Mxfp4ToFp8(x_padded, x_in_s_pad, x_q, x_s, group_size, eps, mxfp4_min, mxfp4_max,
+                                     scale_ue8m0)
     x_q = x_q[:, :original_w * 2]
     # the reference slices the scale rows with the MX scale width
     # (mxfp4_dequant.py:172), which keeps every row
