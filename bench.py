@@ -391,7 +391,7 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
                                                   n // 32, 32, 1e-10, -6.0, 6.0, 0, cur()), "quantize")
     del x6
     y6 = [torch.empty(n, dtype=torch.bfloat16, device=dev) for _ in range(ns)]
-    pair("dequant", "dequant 8192x7168 (dequant_bf16_kernel)", bq, ns,
+    pair("dequant", "dequant 8192x7168 (dequant_kernel)", bq, ns,
          lambda i: chk(lib.omo_hip_per_token_Mxfp4ToBf16_dequant(q6[i].data_ptr(), n // 2, s6[i].data_ptr(), n // 32,
                                                                 y6[i].data_ptr(), n, None, 0, 32, 1e-10, -6.0, 6.0,
                                                                 0, cur()), "dequant"),

@@ -69,6 +69,19 @@ OMO_API int omo_hip_per_token_Mxfp4ToBf16_dequant(const void* input, int64_t inp
                                           void* output_s, int64_t output_s_bytes, int group_size, float eps,
                                           float fp4_min, float fp4_max, int scale_ue8m0, void* stream);
 
+/* Output types of the dequants below. */
+#define OMO_BF16 0
+#define OMO_F16 1
+#define OMO_F32 2
+
+/* omo_hip_per_token_Mxfp4ToBf16_dequant into any of those types: the value of
+ * every element is the bf16 result converted (fp16: RNE; fp32: exact), what
+ * the reference's wrapper does in a second pass over the bf16 tensor
+ * (code/kernel/api/mxfp4_dequant.py:39-74, x_q.to(dtype)). Sizes and alignment
+ * as above; output: 2*input_bytes elements. */
+OMO_API int omo_hip_Mxfp4_dequant(const void* input, int64_t input_bytes, const void* input_s, int64_t input_s_bytes,
+                          void* output, int64_t output_elems, int output_type, void* stream);
+
 /* MXFP4 -> FP8 E4M3 rowwise requant with 1x128 power-of-two fp32 scales
  * stored transposed [row_bytes/64, rows].
  * Replaces omo::omo_per_token_Mxfp4ToFp8 (code/kernel/per_token_Mxfp4ToFp8.cu:238-309,
@@ -210,6 +223,10 @@ OMO_API int omo_hip_quant_mxfp4_packed(const void* input, int64_t rows, int64_t 
  * input 4-byte aligned. */
 OMO_API int omo_hip_packed_Mxfp4ToBf16_dequant(const void* input, int64_t rows, int64_t cols, void* output,
                                                int64_t output_elems, void* stream);
+
+/* The same into any output type, as omo_hip_Mxfp4_dequant. */
+OMO_API int omo_hip_packed_Mxfp4_dequant(const void* input, int64_t rows, int64_t cols, void* output,
+                                         int64_t output_elems, int output_type, void* stream);
 
 /* MXFP4 -> FP8 E4M3 rowwise requant of payload rows: output_q [rows, cols]
  * fp8 (16-byte aligned) and output_s [cols/128, rows] fp32, the outputs of

@@ -533,7 +533,7 @@ __global__ __launch_bounds__(256) void requant_floor(const uint8_t* __restrict__
   }
 }
 
-// ---- dequant to bf16, U code dwords per lane (dequant_bf16_kernel<U, U == 4>, the product's choice of U)
+// ---- dequant to bf16, U code dwords per lane (dequant_kernel<OutBf16, U, U == 4>, the product's choice of U)
 template <int U>
 __global__ __launch_bounds__(256) void dequant_floor(const uint32_t* __restrict__ q, const uint8_t* __restrict__ s,
                                                      fu32x4* __restrict__ out, int64_t ndw) {

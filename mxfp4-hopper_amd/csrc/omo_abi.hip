@@ -106,6 +106,25 @@ int check_packed(const char* fn, int64_t rows, int64_t cols) {
   return OMO_OK;
 }
 
+int packed_dequant(const char* fn, const void* input, int64_t rows, int64_t cols, void* output, int64_t output_elems,
+                   int output_type, void* stream) {
+  REQUIRE(output_type >= OMO_BF16 && output_type <= OMO_F32, "%s: unknown output type %d", fn, output_type);
+  int rc = check_packed(fn, rows, cols);
+  if (rc != OMO_OK) return rc;
+  // an fp32 row takes twice the workgroups of check_packed's bound
+  REQUIRE(rows < ((int64_t)1 << 30) / (cols / 8 / 256 + 1) || output_type != OMO_F32, "%s: too many rows", fn);
+  const int64_t stride = cols / 32 * 17;
+  REQUIRE_BUF("input", input, rows * stride, rows * stride);
+  REQUIRE_BUF("output", output, output_elems, rows * cols);
+  REQUIRE(aligned(input, 4) && aligned(output, 16), "%s: input must be 4-byte and output 16-byte aligned", fn);
+  if (rows == 0 || cols == 0) return ok();
+  const uint8_t* in = static_cast<const uint8_t*>(input);
+  return from_hip(omo_hip::launch_dequant_rows(in, stride, in + cols / 2, stride, output,
+                                               static_cast<omo_hip::FloatType>(output_type), rows, cols,
+                                               as_stream(stream)),
+                  fn);
+}
+
 // Shared checks of the permutation entry points: strided input rows of codes
 // and scales, num_out int32 source indices.
 int check_permute(const char* fn, const void* codes, int64_t codes_bytes, int64_t code_stride, const void* scales,
@@ -213,7 +232,25 @@ int omo_hip_per_token_Mxfp4ToBf16_dequant(const void* input, int64_t input_bytes
   REQUIRE_BUF("output_q", output_q, output_q_elems, 2 * input_bytes);
   REQUIRE(aligned(input, 4) && aligned(output_q, 16), "%s: input must be 4-byte and output_q 16-byte aligned", fn);
   if (input_bytes == 0) return ok();
-  return from_hip(omo_hip::launch_dequant_bf16(input, input_s, output_q, input_bytes, as_stream(stream)), fn);
+  return from_hip(omo_hip::launch_dequant(input, input_s, output_q, omo_hip::FloatType::kBf16, input_bytes,
+                                          as_stream(stream)),
+                  fn);
+}
+
+int omo_hip_Mxfp4_dequant(const void* input, int64_t input_bytes, const void* input_s, int64_t input_s_bytes,
+                          void* output, int64_t output_elems, int output_type, void* stream) {
+  const char* fn = "omo_Mxfp4_dequant";
+  REQUIRE(output_type >= OMO_BF16 && output_type <= OMO_F32, "%s: unknown output type %d", fn, output_type);
+  REQUIRE(input_bytes >= 0 && input_bytes % 128 == 0, "%s: input.numel() %% 128 != 0", fn);
+  REQUIRE(input_bytes <= kMaxSize, "%s: shape too large", fn);
+  REQUIRE_BUF("input", input, input_bytes, input_bytes);
+  REQUIRE_BUF("input_s", input_s, input_s_bytes, input_bytes / 16);
+  REQUIRE_BUF("output", output, output_elems, 2 * input_bytes);
+  REQUIRE(aligned(input, 4) && aligned(output, 16), "%s: input must be 4-byte and output 16-byte aligned", fn);
+  if (input_bytes == 0) return ok();
+  return from_hip(omo_hip::launch_dequant(input, input_s, output, static_cast<omo_hip::FloatType>(output_type),
+                                          input_bytes, as_stream(stream)),
+                  fn);
 }
 
 int omo_hip_per_token_Mxfp4ToFp8(const void* input, int64_t rows, int64_t row_bytes, const void* input_s,
@@ -417,18 +454,12 @@ int omo_hip_quant_mxfp4_packed(const void* input, int64_t rows, int64_t cols, vo
 
 int omo_hip_packed_Mxfp4ToBf16_dequant(const void* input, int64_t rows, int64_t cols, void* output,
                                        int64_t output_elems, void* stream) {
-  const char* fn = "omo_packed_Mxfp4ToBf16_dequant";
-  int rc = check_packed(fn, rows, cols);
-  if (rc != OMO_OK) return rc;
-  const int64_t stride = cols / 32 * 17;
-  REQUIRE_BUF("input", input, rows * stride, rows * stride);
-  REQUIRE_BUF("output", output, output_elems, rows * cols);
-  REQUIRE(aligned(input, 4) && aligned(output, 16), "%s: input must be 4-byte and output 16-byte aligned", fn);
-  if (rows == 0 || cols == 0) return ok();
-  const uint8_t* in = static_cast<const uint8_t*>(input);
-  return from_hip(omo_hip::launch_dequant_rows(in, stride, in + cols / 2, stride, output, rows, cols,
-                                               as_stream(stream)),
-                  fn);
+  return packed_dequant("omo_packed_Mxfp4ToBf16_dequant", input, rows, cols, output, output_elems, OMO_BF16, stream);
+}
+
+int omo_hip_packed_Mxfp4_dequant(const void* input, int64_t rows, int64_t cols, void* output, int64_t output_elems,
+                                 int output_type, void* stream) {
+  return packed_dequant("omo_packed_Mxfp4_dequant", input, rows, cols, output, output_elems, output_type, stream);
 }
 
 int omo_hip_packed_Mxfp4ToFp8(const void* input, int64_t rows, int64_t cols, void* output_q, int64_t output_q_bytes,

@@ -30,7 +30,11 @@ hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipSt
 hipError_t launch_quant_rowwise(const void* x, void* q, void* s, int64_t numel, float eps, float fp4_min,
                                 float fp4_max, hipStream_t stream);
 
-hipError_t launch_dequant_bf16(const void* q, const void* s, void* out, int64_t nbytes, hipStream_t stream);
+// Output type of a dequant (the OMO_BF16 / OMO_F16 / OMO_F32 of the C ABI).
+enum class FloatType { kBf16 = 0, kF16 = 1, kF32 = 2 };
+
+hipError_t launch_dequant(const void* q, const void* s, void* out, FloatType type, int64_t nbytes,
+                          hipStream_t stream);
 
 hipError_t launch_mxfp4_to_fp8(const void* q, const void* s, void* out, float* out_s, int64_t M, int64_t Kb,
                                hipStream_t stream);
@@ -59,7 +63,7 @@ hipError_t launch_quant_rows(const void* x, void* q, int64_t q_stride, void* s, 
                              int64_t K, float eps, hipStream_t stream);
 
 hipError_t launch_dequant_rows(const void* q, int64_t q_stride, const void* s, int64_t s_stride, void* out,
-                               int64_t rows, int64_t K, hipStream_t stream);
+                               FloatType type, int64_t rows, int64_t K, hipStream_t stream);
 
 // src: optional int32 source row per output row (indices outside [0, n_src)
 // read zeros); M output rows. Kb code bytes per row: a multiple of 64, or,

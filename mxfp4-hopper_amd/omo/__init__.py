@@ -27,6 +27,9 @@ import ctypes
 import torch
 
 from ._abi import check as _check
+from ._abi import OMO_BF16 as _BF16
+from ._abi import OMO_F16 as _F16
+from ._abi import OMO_F32 as _F32
 from ._abi import lib as _lib
 
 __all__ = [
@@ -40,11 +43,13 @@ __all__ = [
     "omo_per_token_Mxfp4ToFp8",
     "omo_Mxfp4RowToBf16ToFp8Col_splits",
     "omo_Mxfp4ToFp8_padded",
+    "omo_Mxfp4_dequant",
     "omo_quant_mxfp4_dual",
     "omo_quant_mxfp4_dual_grouped",
     "omo_quant_mxfp4_packed",
     "omo_packed_Mxfp4ToBf16_dequant",
     "omo_packed_Mxfp4ToFp8",
+    "omo_packed_Mxfp4_dequant",
     "omo_mxfp4_permute_rows",
     "omo_permute_Mxfp4ToFp8",
     "omo_route_counts",
@@ -52,6 +57,9 @@ __all__ = [
 ]
 
 _FP8 = torch.float8_e4m3fn
+
+# dtypes a dequant writes directly
+DEQUANT_TYPES = {torch.bfloat16: _BF16, torch.float16: _F16, torch.float32: _F32}
 
 
 def _check_input(t: torch.Tensor, name: str) -> None:
@@ -153,6 +161,29 @@ def omo_per_token_Mxfp4ToBf16_dequant(input, input_s, output_q, output_s, group_
             input.data_ptr(), input.numel(), input_s.data_ptr(), input_s.numel(), output_q.data_ptr(),
             output_q.numel(), output_s.data_ptr(), _nbytes(output_s), int(group_size), float(eps), float(fp4_min),
             float(fp4_max), int(bool(scale_ue8m0)), stream))
+
+
+def _dequant_type(t: torch.Tensor) -> int:
+    if t.dtype not in DEQUANT_TYPES:
+        raise RuntimeError(f"output must be one of {list(DEQUANT_TYPES)}, got {t.dtype}")
+    return DEQUANT_TYPES[t.dtype]
+
+
+def omo_Mxfp4_dequant(input, input_s, output):
+    """MXFP4 -> bf16, fp16 or fp32 (output's dtype) over the flat code tensor:
+    omo_per_token_Mxfp4ToBf16_dequant's values converted to that dtype, in one
+    pass."""
+    _check_input(input, "input")
+    _check_input(output, "output")
+    _check_eq(input.numel() % 128, 0, "input.numel() % group_size == 0")
+    _same_device(input, input_s, output)
+    _check_input(input_s, "input_s")
+    _check_dtype(input, torch.uint8, "input")
+    _check_dtype(input_s, torch.uint8, "input_s")
+    kind = _dequant_type(output)
+    with _on_device(input) as stream:
+        _check(_lib.omo_hip_Mxfp4_dequant(input.data_ptr(), input.numel(), input_s.data_ptr(), input_s.numel(),
+                                          output.data_ptr(), output.numel(), kind, stream))
 
 
 def _requant_args(name, input, input_s, output_q, output_s):
@@ -391,6 +422,21 @@ def omo_packed_Mxfp4ToBf16_dequant(input, output):
     with _on_device(input) as stream:
         _check(_lib.omo_hip_packed_Mxfp4ToBf16_dequant(input.data_ptr(), input.size(0), cols, output.data_ptr(),
                                                        output.numel(), stream))
+
+
+def omo_packed_Mxfp4_dequant(input, output):
+    """Payload rows [T, 17H/32] -> [T, H] in output's dtype (bf16, fp16 or fp32)."""
+    _check_input(input, "input")
+    _check_input(output, "output")
+    _same_device(input, output)
+    if input.dim() != 2:
+        raise RuntimeError("input must be 2-D")
+    _check_dtype(input, torch.uint8, "input")
+    kind = _dequant_type(output)
+    cols = _payload_cols(input)
+    with _on_device(input) as stream:
+        _check(_lib.omo_hip_packed_Mxfp4_dequant(input.data_ptr(), input.size(0), cols, output.data_ptr(),
+                                                 output.numel(), kind, stream))
 
 
 def omo_packed_Mxfp4ToFp8(input, output_q, output_s):

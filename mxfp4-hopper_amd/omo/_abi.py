@@ -14,6 +14,7 @@ OMO_OK = 0
 OMO_ERR_INVALID_ARGUMENT = -1
 OMO_ERR_UNSUPPORTED = -2
 OMO_ERR_HIP = -3
+OMO_BF16, OMO_F16, OMO_F32 = 0, 1, 2
 
 _P, _I64, _I, _F = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
 
@@ -28,6 +29,8 @@ class DualItem(ctypes.Structure):
 SIGNATURES = {
     "omo_hip_per_token_group_quant_fp4": [_P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_per_token_Mxfp4ToBf16_dequant": [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
+    "omo_hip_Mxfp4_dequant": [_P, _I64, _P, _I64, _P, _I64, _I, _P],
+    "omo_hip_packed_Mxfp4_dequant": [_P, _I64, _I64, _P, _I64, _I, _P],
     "omo_hip_per_token_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_per_token_Mxfp4ToBf16ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _F, _F, _F, _I, _P],
     "omo_hip_Mxfp4ToFp8_padded": [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],

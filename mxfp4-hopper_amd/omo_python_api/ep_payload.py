@@ -17,7 +17,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from omo import omo_packed_Mxfp4ToBf16_dequant, omo_packed_Mxfp4ToFp8, omo_quant_mxfp4_packed
+from omo import DEQUANT_TYPES, omo_packed_Mxfp4_dequant, omo_packed_Mxfp4ToFp8, omo_quant_mxfp4_packed
 
 
 def payload_width(hidden: int) -> int:
@@ -73,9 +73,9 @@ def packed_mxfp4ToBf16(packed: torch.Tensor, dtype: torch.dtype = torch.bfloat16
     omo_per_token_mxfp4ToBf16_dequant_wrapper(*split_payload(packed), dtype)."""
     assert packed.is_contiguous(), "payload is not contiguous"
     T, H = packed.size(0), hidden_of(packed)
-    out = torch.empty((T, H), device=packed.device, dtype=torch.bfloat16)
+    out = torch.empty((T, H), device=packed.device, dtype=dtype if dtype in DEQUANT_TYPES else torch.bfloat16)
     if T > 0:
-        omo_packed_Mxfp4ToBf16_dequant(packed, out)
+        omo_packed_Mxfp4_dequant(packed, out)
     return out.to(dtype)
 
 

@@ -14,11 +14,12 @@ import torch
 import torch.nn.functional as F
 
 from omo import (
+    DEQUANT_TYPES,
     omo_Mxfp4RowToBf16ToFp8Col_splits,
     omo_Mxfp4ToFp8_padded,
+    omo_Mxfp4_dequant,
     omo_per_token_Mxfp4RowToBf16ToFp8Col,
     omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit,
-    omo_per_token_Mxfp4ToBf16_dequant,
     omo_per_token_Mxfp4ToBf16ToFp8,
     omo_per_token_Mxfp4ToFp8,
     omo_per_token_Mxfp4ToFp8_col,
@@ -51,18 +52,18 @@ def unpad_from_multiple(x_padded, original_size):
 
 def omo_per_token_mxfp4ToBf16_dequant_wrapper(x: torch.Tensor, x_in_s: torch.Tensor, dtype):
     """codes [M, K/2] + scales [M, K/32] -> x_q.to(dtype) of shape [M, K]
-    (mxfp4_dequant.py:39-74; called at code/transformer_engine-2.8.diff:392)."""
+    (mxfp4_dequant.py:39-74; called at code/transformer_engine-2.8.diff:392).
+    fp16 and fp32 are written by the dequant itself; any other dtype is
+    converted from bf16 in a second pass."""
     group_size = 32
-    eps = 1e-10
-    scale_ue8m0 = False
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
     out_shape = (*x.shape[:-1], x.shape[-1] * 2)
-    scale_shape = (*x.shape[:-1], x.shape[-1] * 2 // 128)
-    x_q = torch.empty(out_shape, device=x.device, dtype=torch.bfloat16)
-    x_s = torch.empty(scale_shape, device=x.device, dtype=torch.float)
+    x_q = torch.empty(out_shape, device=x.device, dtype=dtype if dtype in DEQUANT_TYPES else torch.bfloat16)
     if x.shape[0] > 0:
-        omo_per_token_Mxfp4ToBf16_dequant(x, x_in_s, x_q, x_s, group_size, eps, mxfp4_min, mxfp4_max, scale_ue8m0)
+        if x.dim() != 2:  # the reference's check of its scale output, shaped like x
+            raise RuntimeError(f"Expected output_s.dim() == 2 ({x.dim()} vs. 2)")
+        omo_Mxfp4_dequant(x, x_in_s, x_q)
     return x_q.to(dtype)
 
 
