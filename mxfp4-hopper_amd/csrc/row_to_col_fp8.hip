@@ -698,7 +698,8 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
 // 0; cols_valid a multiple of 32): the missing 16 B code chunks of a row read
 // its last chunk and are zeroed, their scale bytes read as 127, and the lanes
 // of the missing columns store nothing.
-template <bool MSPLIT, bool RAGGED, bool PARTIAL = false, bool SBYTE = false>
+// NT_CODES: the code loads are non-temporal.
+template <bool MSPLIT, bool RAGGED, bool PARTIAL, bool SBYTE, bool NT_CODES>
 __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restrict__ q, const uint8_t* __restrict__ s,
                                           int64_t N, int64_t row0, int rows_valid, int64_t col0, float eps,
                                           float* __restrict__ out_s_row, uint8_t* __restrict__ obase, int64_t cstride,
@@ -712,10 +713,10 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
   // waited for completion before the next was issued (dense 4000 x 7168:
   // 10.6 against 11.4 us).
   // Lane t loads chunk t & 7 of rows (t >> 3) + 32k: one 64-bit row product
-  // per lane, the rest workgroup-uniform steps of 32 rows. Per split the code
-  // loads are non-temporal (cfg5's 8 splits 50.3 against 49.0 us); the
-  // dense kernel, one round of resident workgroups, keeps ordinary ones
-  // (4096 x 7168 8.9 against 9.5 us non-temporal).
+  // per lane, the rest workgroup-uniform steps of 32 rows. Code loads are
+  // non-temporal per split (cfg5's 8 splits 50.3 against 49.0 us) and in the
+  // dense rows-fastest order (4001 x 7168 12.6 against 11.8), ordinary in the
+  // other dense orders (4096 x 7168 8.9 against 9.5 us non-temporal).
   u32x4 cv[4];
   const uint8_t* qt = q + row0 * (N / 2) + col0 / 2 + 16 * (PARTIAL ? min(t & 7, nch - 1) : (t & 7));
 #pragma unroll
@@ -723,7 +724,7 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
     const int r = (t >> 3) + 32 * k;
     const int64_t rr = RAGGED ? min(r, rows_valid - 1) : (t >> 3);
     const u32x4* src = reinterpret_cast<const u32x4*>(qt + rr * (N / 2) + (RAGGED ? 0 : 32 * k * (N / 2)));
-    cv[k] = MSPLIT ? __builtin_nontemporal_load(src) : *src;
+    cv[k] = NT_CODES ? __builtin_nontemporal_load(src) : *src;
   }
   u32x2 sv = {0x7F7F7F7Fu, 0x7F7F7F7Fu};
   if (t < kTile) {
@@ -778,41 +779,88 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
 
 // A tile of band col0 / 256: the whole band, or (NARROWN, N % 256 != 0)
 // the last band's N - col0 columns.
-template <bool MSPLIT, bool RAGGED, bool NARROWN>
+template <bool MSPLIT, bool RAGGED, bool NARROWN, bool NT_CODES>
 __device__ __forceinline__ void wide_tile_any(WideSmem& sm, const uint8_t* __restrict__ q,
                                               const uint8_t* __restrict__ s, int64_t N, int64_t row0, int rows_valid,
                                               int64_t col0, float eps, float* __restrict__ out_s_row,
                                               uint8_t* __restrict__ obase, int64_t cstride, bool line_nt) {
   if (!NARROWN || col0 + kWideCols <= N) {
-    wide_tile<MSPLIT, RAGGED, false, NARROWN>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
+    wide_tile<MSPLIT, RAGGED, false, NARROWN, NT_CODES>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
                                               line_nt);
   } else {
-    wide_tile<MSPLIT, RAGGED, true, NARROWN>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
+    wide_tile<MSPLIT, RAGGED, true, NARROWN, NT_CODES>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
                                              line_nt, (int)(N - col0));
   }
 }
 
-// Dense, tile (bm, bn) = blockIdx renumbered per XCD, bn fastest. Not
-// RAGGED: whole aligned tiles (M % 128 == 0, 16 B aligned output). RAGGED:
-// any M, any output alignment (the last row tile partial). NARROWN: N % 32
-// == 0 but not a multiple of 256, or scale rows not 8 B aligned (the last
-// band partial, scale bytes read one by one).
-template <bool RAGGED, bool NARROWN>
+// Band walk: tile (S row tiles x B bands, T = S * B, numbered band by band
+// with the row tile fastest) of position j in XCD xcd's walk over its
+// contiguous range of per_xcd tiles, row tile by row tile. False past the
+// range.
+__device__ __forceinline__ bool band_walk_tile(int xcd, int j, int S, int T, int per_xcd, int* bm, int* bn) {
+  const int lo = xcd * per_xcd, hi = min(T, lo + per_xcd);
+  if (j >= hi - lo) return false;
+  const int bn0 = lo / S, m0 = lo - bn0 * S;  // first tile of the range
+  const int bn1 = hi / S, m1 = hi - bn1 * S;  // one past the last
+  // tiles of the range in row tiles below m: band bn0 holds [m0, S) (or
+  // [m0, m1) when bn0 == bn1), bands bn0 + 1 .. bn1 - 1 all, band bn1 [0, m1)
+  auto below = [&](int m) {
+    if (bn0 == bn1) return max(0, min(m, m1) - m0);
+    return m * (bn1 - bn0 - 1) + max(0, m - m0) + min(m, m1);
+  };
+  int a = 0, b = S;  // below(a) <= j < below(b) = hi - lo
+  while (b - a > 1) {
+    const int mid = (a + b) >> 1;
+    if (below(mid) <= j) a = mid;
+    else b = mid;
+  }
+  *bm = a;
+  *bn = bn0 + (a >= m0 ? 0 : 1) + (j - below(a));
+  return true;
+}
+
+// Dense. Not RAGGED: whole aligned tiles (M % 128 == 0, 16 B aligned
+// output). RAGGED: any M, any output alignment (the last row tile partial).
+// NARROWN: N % 32 == 0 but not a multiple of 256, or scale rows not 8 B
+// aligned (the last band partial, scale bytes read one by one).
+//
+// ORDER: which tiles share an XCD at a time.
+//  * Bands fastest within each XCD's contiguous range (each XCD a run of row
+//    tiles, every band): 4096 x 7168 8.9 us against 9.3 with row tiles fastest
+//    and 9.2-9.4 with each XCD a 2-D block of tiles.
+//  * Where M is no multiple of 128 the row tiles m and m + 1 of a band share
+//    every one of its output lines, and the lines are whole in L2 only while
+//    both tiles are at work on one XCD. Rows fastest (each XCD a run of bands,
+//    code loads non-temporal) keeps them next to each other: 4001 x 7168 11.8
+//    us against 15.4 bands fastest, 4700 x 7168 13.5 against 19.4, 8190 x 5120
+//    18.2 against 22.4, 16383 x 2048 12.9 against 15.7.
+//  * Past one round of workgroups the band walk of the per-split kernels with
+//    ordinary code loads and four workgroups per CU: 16383 x 7168 51.1 us
+//    against 64.0 bands fastest and 52.2 rows fastest, 10001 x 7168 32.5
+//    against 42.7 and 33.6, 16383 x 2880 24.0 against 23.8 and 25.5.
+enum DenseOrder { kBandsFastest, kRowsFastest, kBandWalk };
+
+template <bool RAGGED, bool NARROWN, DenseOrder ORDER>
 __global__ __launch_bounds__(256, 4) void row_to_fp8_col_wide_kernel(const uint8_t* __restrict__ q,
                                                                      const uint8_t* __restrict__ s,
                                                                      uint8_t* __restrict__ out,
                                                                      float* __restrict__ out_s, int64_t M, int64_t N,
-                                                                     float eps) {
+                                                                     float eps, int row_tiles, int bands) {
   __shared__ WideSmem sm;
-  // bands fastest within each XCD's contiguous range (each XCD a run of row
-  // tiles, every band): 4096 x 7168 8.9 us against 9.3 with row tiles
-  // fastest and 9.2-9.4 with each XCD a 2-D block of tiles
-  const uint32_t L = xcd_contiguous(blockIdx.x, gridDim.x), gx = (uint32_t)((N + kWideCols - 1) / kWideCols);
-  const int64_t bn = L % gx, bm = L / gx;
-  const int64_t row0 = bm * kTile, col0 = bn * kWideCols;
+  int bm, bn;
+  if (ORDER == kBandWalk) {
+    const int tiles = row_tiles * bands;
+    if (!band_walk_tile((int)(blockIdx.x & 7u), (int)(blockIdx.x >> 3), row_tiles, tiles, (tiles + 7) / 8, &bm, &bn))
+      return;
+  } else {
+    const int L = (int)xcd_contiguous(blockIdx.x, gridDim.x), fast = ORDER == kRowsFastest ? row_tiles : bands;
+    bm = ORDER == kRowsFastest ? L % fast : L / fast;
+    bn = ORDER == kRowsFastest ? L / fast : L % fast;
+  }
+  const int64_t row0 = (int64_t)bm * kTile, col0 = (int64_t)bn * kWideCols;
   const int rows_valid = RAGGED ? (int)(M - row0 < kTile ? M - row0 : kTile) : kTile;
-  wide_tile_any<false, RAGGED, NARROWN>(sm, q, s, N, row0, rows_valid, col0, eps, out_s + bm * N + col0,
-                                        out + col0 * M + row0, M, false);
+  wide_tile_any<false, RAGGED, NARROWN, ORDER == kRowsFastest>(sm, q, s, N, row0, rows_valid, col0, eps,
+                                                               out_s + bm * N + col0, out + col0 * M + row0, M, false);
 }
 
 // Per split on the 256-column tiles: workgroup (split, bm, bn) as in
@@ -837,7 +885,7 @@ __device__ __forceinline__ void msplit_wide_tile(WideSmem& sm, const uint8_t* __
   if (start < 0 || start + len > total_rows || sstart < 0 || sstart + bm >= out_s_rows) return;
   const int64_t row0 = start + bm * kTile, col0 = bn * kWideCols;
   const int rows_valid = (int)(len - bm * kTile < kTile ? len - bm * kTile : kTile);
-  wide_tile_any<true, true, NARROWN>(sm, q, s, N, row0, rows_valid, col0, eps, out_s + (sstart + bm) * N + col0,
+  wide_tile_any<true, true, NARROWN, true>(sm, q, s, N, row0, rows_valid, col0, eps, out_s + (sstart + bm) * N + col0,
                                      out + start * N + col0 * len + bm * kTile, len,
                                      out_line && len % kTile == 0 && (start * N) % kTile == 0);
 }
@@ -916,32 +964,6 @@ constexpr int kFlatMaxSplits = 128;  // lane l of each wave holds splits l and l
 // most ceil(tm * bands / 8) tiles of each split.
 __host__ __device__ constexpr int64_t flat_grid_blocks(int64_t nsplits, int64_t tm, int64_t bands) {
   return 8 * nsplits * ((tm * bands + 7) / 8);
-}
-
-// Band walk: tile (S row tiles x B bands, T = S * B, numbered band by band
-// with the row tile fastest) of position j in XCD xcd's walk over its
-// contiguous range of per_xcd tiles, row tile by row tile. False past the
-// range.
-__device__ __forceinline__ bool band_walk_tile(int xcd, int j, int S, int T, int per_xcd, int* bm, int* bn) {
-  const int lo = xcd * per_xcd, hi = min(T, lo + per_xcd);
-  if (j >= hi - lo) return false;
-  const int bn0 = lo / S, m0 = lo - bn0 * S;  // first tile of the range
-  const int bn1 = hi / S, m1 = hi - bn1 * S;  // one past the last
-  // tiles of the range in row tiles below m: band bn0 holds [m0, S) (or
-  // [m0, m1) when bn0 == bn1), bands bn0 + 1 .. bn1 - 1 all, band bn1 [0, m1)
-  auto below = [&](int m) {
-    if (bn0 == bn1) return max(0, min(m, m1) - m0);
-    return m * (bn1 - bn0 - 1) + max(0, m - m0) + min(m, m1);
-  };
-  int a = 0, b = S;  // below(a) <= j < below(b) = hi - lo
-  while (b - a > 1) {
-    const int mid = (a + b) >> 1;
-    if (below(mid) <= j) a = mid;
-    else b = mid;
-  }
-  *bm = a;
-  *bn = bn0 + (a >= m0 ? 0 : 1) + (j - below(a));
-  return true;
 }
 
 // Where a wave of the flat grid reads the splits from. load() gives lane l
@@ -1131,6 +1153,16 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_narrow_flat_
   msplit_narrow_tile(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, vin, vs);
 }
 
+// Dynamic LDS, unused, that caps the wide per-split kernel's residency at 4
+// workgroups per CU (6 by its own LDS and registers): fewer tiles' partial
+// output lines wait in L2 at once. Ragged cfg5 splits: 49.6 us against 51.0,
+// and 59.8 against 62.8 right after a 512 MB fill (dirty caches, as in a
+// layer step).
+static size_t split_lds_reserve() {
+  const int per_wg = current_device_caps().lds_per_workgroup / 4 - 2560;
+  return per_wg > (int)sizeof(WideSmem) ? (size_t)(per_wg - (int)sizeof(WideSmem)) : 0;
+}
+
 hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float* out_s, int64_t M, int64_t N, float eps,
                                  hipStream_t stream) {
   if (M == 0 || N == 0) return hipSuccess;
@@ -1145,11 +1177,26 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
     // 16384 x 7040: 29.2 against 56.0; 4096 x 2880: 5.6 against 8.4.
     const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
     const bool whole = vout && M % kTile == 0;
-    const dim3 grid((unsigned)(((M + kTile - 1) / kTile) * ((N + kWideCols - 1) / kWideCols)));
-    auto kernel = narrow_n ? (whole ? row_to_fp8_col_wide_kernel<false, true> : row_to_fp8_col_wide_kernel<true, true>)
-                           : (whole ? row_to_fp8_col_wide_kernel<false, false> : row_to_fp8_col_wide_kernel<true, false>);
-    return launch(kernel, grid, dim3(256), 0, stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
-                  static_cast<uint8_t*>(out), out_s, M, N, eps);
+    const int64_t row_tiles = (M + kTile - 1) / kTile, bands = (N + kWideCols - 1) / kWideCols;
+    const int64_t tiles = row_tiles * bands, cus = current_device_caps().cus;
+    // Ragged: rows fastest while the tiles are fewer than one round of
+    // resident workgroups (six per CU), the band walk beyond. Bands fastest
+    // where many CUs stay idle all the same (five tiles per eight CUs: 1000 x
+    // 2880, 96 tiles, 5.2 us against 5.6 rows fastest, 1500 x 2880, 144, 5.9
+    // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1).
+    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : tiles < 6 * cus ? kRowsFastest : kBandWalk;
+    auto kernel = narrow_n ? (whole                    ? row_to_fp8_col_wide_kernel<false, true, kBandsFastest>
+                              : order == kBandsFastest ? row_to_fp8_col_wide_kernel<true, true, kBandsFastest>
+                              : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, true, kRowsFastest>
+                                                       : row_to_fp8_col_wide_kernel<true, true, kBandWalk>)
+                           : (whole                    ? row_to_fp8_col_wide_kernel<false, false, kBandsFastest>
+                              : order == kBandsFastest ? row_to_fp8_col_wide_kernel<true, false, kBandsFastest>
+                              : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, false, kRowsFastest>
+                                                       : row_to_fp8_col_wide_kernel<true, false, kBandWalk>);
+    const int64_t grid = order == kBandWalk ? (tiles + 7) / 8 * 8 : tiles;
+    return launch(kernel, dim3((unsigned)grid), dim3(256), order == kBandWalk ? split_lds_reserve() : 0, stream,
+                  static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M,
+                  N, eps, (int)row_tiles, (int)bands);
   }
   const int64_t tiles_m = (M + kTile - 1) / kTile, tiles = tiles_m * ((N + kTile - 1) / kTile);
   // one wave of resident blocks: two 512-thread blocks per CU at this
@@ -1160,16 +1207,6 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
   return launch(kernel, dim3((unsigned)grid), dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),
                      static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M, N, (int)tiles_m, (int)tiles,
                      eps, vin, vs);
-}
-
-// Dynamic LDS, unused, that caps the wide per-split kernel's residency at 4
-// workgroups per CU (6 by its own LDS and registers): fewer tiles' partial
-// output lines wait in L2 at once. Ragged cfg5 splits: 49.6 us against 51.0,
-// and 59.8 against 62.8 right after a 512 MB fill (dirty caches, as in a
-// layer step).
-static size_t split_lds_reserve() {
-  const int per_wg = current_device_caps().lds_per_workgroup / 4 - 2560;
-  return per_wg > (int)sizeof(WideSmem) ? (size_t)(per_wg - (int)sizeof(WideSmem)) : 0;
 }
 
 // The wide flat kernel's form for a split count and width: band walk up to
