@@ -1,0 +1,43 @@
+"""Dual-layout quantize on tensors of whole 64 x 256 tiles, and the same with
+scale buffers that cannot take the wide stores: every byte against the
+rowwise oracle of x and of its transpose, alone and grouped."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import bits_u16, bits_u8
+
+pytestmark = pytest.mark.gpu
+
+
+def _outs(dev, M, K, row_shift, col_shift):
+    def buf(rows, cols, shift):
+        flat = torch.full((rows * cols + 16,), 0xAB, dtype=torch.uint8, device=dev)
+        return flat[shift:shift + rows * cols].view(rows, cols)
+    return (buf(M, K // 2, 0), buf(M, K // 32, row_shift), buf(K, M // 2, 0), buf(K, M // 32, col_shift))
+
+
+def _check(oracle, x, outs):
+    M, K = x.shape
+    for bits, q, s in ((bits_u16(x), outs[0], outs[1]), (bits_u16(x.t()), outs[2], outs[3])):
+        eq, es = oracle.quant_mxfp4(np.ascontiguousarray(bits).reshape(-1))
+        np.testing.assert_array_equal(bits_u8(q).reshape(-1), np.asarray(eq).reshape(-1))
+        np.testing.assert_array_equal(bits_u8(s).reshape(-1), np.asarray(es).reshape(-1))
+
+
+# one tile; two of each; an inf block (the restated path); one tile short of whole
+@pytest.mark.parametrize("M,K", [(64, 256), (128, 512), (96, 256), (64, 288)])
+@pytest.mark.parametrize("row_shift,col_shift", [(0, 0), (4, 0), (0, 1)])
+def test_whole_tiles(oracle, dev, M, K, row_shift, col_shift):
+    import omo
+    print("dual whole tiles", M, K, row_shift, col_shift, flush=True)
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(M + K)).to(torch.bfloat16)
+    x[3, 40], x[33, 7] = float("inf"), 0.0
+    outs = _outs(dev, M, K, row_shift, col_shift)
+    grouped = [_outs(dev, M, K, row_shift, col_shift), _outs(dev, M, K, 0, 0)]
+    xd = x.to(dev)
+    omo.omo_quant_mxfp4_dual(xd, *outs)
+    omo.omo_quant_mxfp4_dual_grouped([xd, xd], grouped)
+    torch.cuda.synchronize()
+    for o in [outs] + grouped:
+        _check(oracle, x, o)
