@@ -1153,13 +1153,14 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_narrow_flat_
   msplit_narrow_tile(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, vin, vs);
 }
 
-// Dynamic LDS, unused, that caps the wide per-split kernel's residency at 4
-// workgroups per CU (6 by its own LDS and registers): fewer tiles' partial
-// output lines wait in L2 at once. Ragged cfg5 splits: 49.6 us against 51.0,
-// and 59.8 against 62.8 right after a 512 MB fill (dirty caches, as in a
-// layer step).
-static size_t split_lds_reserve() {
-  const int per_wg = current_device_caps().lds_per_workgroup / 4 - 2560;
+// Dynamic LDS, unused, that caps the residency of wide tiles with ragged
+// output lines at 4 workgroups per CU (6 by their own LDS): fewer tiles'
+// partial output lines wait in L2 at once. Ragged cfg5 splits: 49.6 us
+// against 51.0, and 59.8 against 62.8 right after a 512 MB fill (dirty
+// caches, as in a layer step).
+static size_t ragged_lds_reserve() {
+  const DeviceCaps dc = current_device_caps();
+  const int per_wg = dc.lds_per_workgroup / 4 - 2560;
   return per_wg > (int)sizeof(WideSmem) ? (size_t)(per_wg - (int)sizeof(WideSmem)) : 0;
 }
 
@@ -1179,12 +1180,14 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
     const bool whole = vout && M % kTile == 0;
     const int64_t row_tiles = (M + kTile - 1) / kTile, bands = (N + kWideCols - 1) / kWideCols;
     const int64_t tiles = row_tiles * bands, cus = current_device_caps().cus;
-    // Ragged: rows fastest while the tiles are fewer than one round of
-    // resident workgroups (six per CU), the band walk beyond. Bands fastest
+    // Ragged: rows fastest while the tiles are one round of resident
+    // workgroups (five per CU, by registers), the band walk beyond (10500 x
+    // 4096, 1328 tiles, 20.5 us against 21.1 rows fastest; 16383 x 2816, 1408,
+    // 21.9 against 23.5; 8190 x 5120, 1280, 20.7 against 18.2). Bands fastest
     // where many CUs stay idle all the same (five tiles per eight CUs: 1000 x
     // 2880, 96 tiles, 5.2 us against 5.6 rows fastest, 1500 x 2880, 144, 5.9
     // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1).
-    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : tiles < 6 * cus ? kRowsFastest : kBandWalk;
+    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : tiles <= 5 * cus ? kRowsFastest : kBandWalk;
     auto kernel = narrow_n ? (whole                    ? row_to_fp8_col_wide_kernel<false, true, kBandsFastest>
                               : order == kBandsFastest ? row_to_fp8_col_wide_kernel<true, true, kBandsFastest>
                               : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, true, kRowsFastest>
@@ -1194,7 +1197,7 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
                               : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, false, kRowsFastest>
                                                        : row_to_fp8_col_wide_kernel<true, false, kBandWalk>);
     const int64_t grid = order == kBandWalk ? (tiles + 7) / 8 * 8 : tiles;
-    return launch(kernel, dim3((unsigned)grid), dim3(256), order == kBandWalk ? split_lds_reserve() : 0, stream,
+    return launch(kernel, dim3((unsigned)grid), dim3(256), order == kBandWalk ? ragged_lds_reserve() : 0, stream,
                   static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M,
                   N, eps, (int)row_tiles, (int)bands);
   }
@@ -1209,13 +1212,24 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
                      eps, vin, vs);
 }
 
-// The wide flat kernel's form for a split count and width: band walk up to
-// 64 splits on rows of more than 16 bands, else contiguous ranges.
-static bool split_walk(int64_t nsplits, int64_t bands) { return nsplits <= 64 && bands > 16; }
+// The same for splits, but none where there are at most about the tiles of
+// one round of workgroups, which the cap would make two (8 splits, cold
+// buffers: 8000 x 4096 and 16431 x 2048, 1060 tiles, 17.5 -> 14.4 us; 10500 x
+// 4096, 1410 tiles, 22.3 -> 21.0; at 32 splits 23.5 -> 24.2).
+static size_t split_lds_reserve(int64_t tiles) {
+  return tiles < 6 * (int64_t)current_device_caps().cus ? 0 : ragged_lds_reserve();
+}
+
+// The wide flat kernel's form for a split count and width: band walk on rows
+// of more than 16 bands up to `most` splits, else contiguous ranges. With
+// device lengths up to 64 splits. With lengths by value, whose grid has no
+// empty workgroups, up to 16: at 32 splits the ranges are ahead (16431 x 7168,
+// cold buffers, 52.7 us against 55.4; 8000 x 7168 28.6 against 30.4), at 16
+// the walk (52.6 against 51.8; 20000 x 7168 67.4 against 62.5).
+static bool split_walk(int64_t nsplits, int64_t bands, int64_t most) { return nsplits <= most && bands > 16; }
 
 template <typename Splits>
-static auto split_flat_kernel(int64_t nsplits, int64_t bands, bool narrow_n) {
-  const bool walk = split_walk(nsplits, bands);
+static auto split_flat_kernel(int64_t nsplits, bool walk, bool narrow_n) {
   return narrow_n ? (nsplits > 64 ? row_to_fp8_col_msplit_flat_kernel<2, false, true, Splits>
                      : walk      ? row_to_fp8_col_msplit_flat_kernel<1, true, true, Splits>
                                  : row_to_fp8_col_msplit_flat_kernel<1, false, true, Splits>)
@@ -1238,7 +1252,7 @@ hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out,
   ValueSplits v;
   memset(&v, 0, sizeof(v));
   const int64_t bands = (N + kWideCols - 1) / kWideCols;
-  const bool walk = split_walk(nsplits, bands);
+  const bool walk = split_walk(nsplits, bands, 16);
   int64_t row_tiles = 0, per_xcd = 0;
   for (int64_t i = 0; i < nsplits; i++) {
     const int64_t tiles = (lens[i] + kTile - 1) / kTile;
@@ -1250,8 +1264,8 @@ hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out,
   if (grid == 0) return hipSuccess;
   const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
   const bool out_line = (reinterpret_cast<uintptr_t>(out) & 127) == 0;
-  return launch(split_flat_kernel<ValueSplits>(nsplits, bands, narrow_n), dim3((unsigned)grid), dim3(256),
-                split_lds_reserve(), stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
+  return launch(split_flat_kernel<ValueSplits>(nsplits, walk, narrow_n), dim3((unsigned)grid), dim3(256),
+                split_lds_reserve(row_tiles * bands), stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
                 static_cast<uint8_t*>(out), out_s, v, total_rows, N, out_s_rows, eps, out_line, (int)nsplits,
                 (int)row_tiles, (int)bands);
 }
@@ -1268,7 +1282,7 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
   const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
   const int64_t tiles_m = (max_split_len + kTile - 1) / kTile;
   const int64_t bands = wide ? (N + kWideCols - 1) / kWideCols : (N + kTile - 1) / kTile;
-  const size_t reserve = split_lds_reserve();
+  const size_t reserve = split_lds_reserve((total_rows / kTile + nsplits) * bands);  // at most so many tiles
   const bool out_line = (reinterpret_cast<uintptr_t>(out) & 127) == 0;
   const DeviceSplits splits{lens, offs, soffs};
   // A launch holds at most 2^32 - 1 work-items along x (gridDim.x times the
@@ -1277,7 +1291,7 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
   if (nsplits <= kFlatMaxSplits && tiles_m * bands + 7 <= (int64_t)UINT32_MAX / flat_threads / nsplits) {
     const dim3 grid((unsigned)flat_grid_blocks(nsplits, tiles_m, bands));
     if (wide) {
-      return launch(split_flat_kernel<DeviceSplits>(nsplits, bands, narrow_n), grid, dim3(256), reserve, stream,
+      return launch(split_flat_kernel<DeviceSplits>(nsplits, split_walk(nsplits, bands, 64), narrow_n), grid, dim3(256), reserve, stream,
                     static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s,
                     splits, total_rows, N, out_s_rows, eps, out_line, (int)nsplits, (int)tiles_m, (int)bands);
     }
