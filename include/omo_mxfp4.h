@@ -268,14 +268,16 @@ OMO_API int omo_hip_permute_Mxfp4ToFp8(const void* codes, int64_t codes_bytes, i
  * Two calls in stream order:
  *   omo_hip_route_counts: counts [experts, omo_hip_route_chunks(tokens, experts)]
  *     (int32), the routed tokens of each expert per chunk of tokens; an
- *     expert's row sums to its load.
+ *     expert's row sums to its load. host_counts: NULL, or pinned host memory
+ *     of the same size for a second copy, valid once the stream has been
+ *     waited for.
  *   omo_hip_route_rows: src_rows[r] = token of the r-th routed pair by
  *     expert, then token (pairs past src_elems are dropped; with pad, the
  *     entries after the last pair are set to -1), and, where dest is not
  *     NULL, dest[t * experts + e] = r, or -1 where the pair is not routed. */
 OMO_API int64_t omo_hip_route_chunks(int64_t tokens, int64_t experts);
 OMO_API int omo_hip_route_counts(const void* map, int64_t tokens, int64_t experts, int32_t* counts,
-                                 int64_t counts_elems, void* stream);
+                                 int64_t counts_elems, int32_t* host_counts, void* stream);
 OMO_API int omo_hip_route_rows(const void* map, int64_t tokens, int64_t experts, const int32_t* counts,
                                int64_t counts_elems, int32_t* src_rows, int64_t src_elems, int pad, int32_t* dest,
                                int64_t dest_elems, void* stream);

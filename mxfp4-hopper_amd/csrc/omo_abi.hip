@@ -504,12 +504,13 @@ int64_t omo_hip_route_chunks(int64_t tokens, int64_t experts) {
 }
 
 int omo_hip_route_counts(const void* map, int64_t tokens, int64_t experts, int32_t* counts, int64_t counts_elems,
-                         void* stream) {
+                         int32_t* host_counts, void* stream) {
   const char* fn = "omo_route_counts";
   int rc = check_route(fn, map, tokens, experts, counts, counts_elems);
   if (rc != OMO_OK) return rc;
+  REQUIRE(aligned(host_counts, 4), "%s: host_counts must be 4-byte aligned", fn);
   if (tokens == 0 || experts == 0) return ok();
-  return from_hip(omo_hip::launch_route_counts(map, tokens, experts, counts, as_stream(stream)), fn);
+  return from_hip(omo_hip::launch_route_counts(map, tokens, experts, counts, host_counts, as_stream(stream)), fn);
 }
 
 int omo_hip_route_rows(const void* map, int64_t tokens, int64_t experts, const int32_t* counts, int64_t counts_elems,

@@ -81,11 +81,13 @@ hipError_t launch_gather_rows(const void* a, int64_t a_stride, int64_t a_bytes, 
                               void* out_b, hipStream_t stream);
 
 // Expert-major row order of a routing map [T, E] (T, E >= 1, at most 2^31 - 1
-// pairs, E at most 4 * 65534): counts [E, route_chunks(T, E)], then src (rows at
+// pairs, E at most 4 * 65534): counts [E, route_chunks(T, E)] (also to
+// host_counts, pinned host memory, where not null), then src (rows at
 // or past src_len not written; pad: the rest of src set to -1) and, where not
 // null, dest [T, E].
 int64_t route_chunks(int64_t T, int64_t E);
-hipError_t launch_route_counts(const void* map, int64_t T, int64_t E, int32_t* counts, hipStream_t stream);
+hipError_t launch_route_counts(const void* map, int64_t T, int64_t E, int32_t* counts, int32_t* host_counts,
+                               hipStream_t stream);
 hipError_t launch_route_rows(const void* map, int64_t T, int64_t E, const int32_t* counts, int32_t* src,
                              int64_t src_len, bool pad, int32_t* dest, hipStream_t stream);
 

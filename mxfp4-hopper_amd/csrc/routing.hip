@@ -17,7 +17,7 @@
 // fills: 18 launches, 65 us of kernels, three waits of the host) made a
 // permute + FP8 requant of 4096 tokens x 7168, 8 of 64 experts, 193.9 us a
 // call, of which the requant is 51.8; these two launches take 3.5 + 4.7 us
-// (kernel trace) and the call 84.1.
+// (kernel trace) and the call 70.3. The host reads the counts between them.
 #include <algorithm>
 
 #include "omo_internal.h"
@@ -62,7 +62,8 @@ __device__ __forceinline__ bool route_flag(uint32_t w, int k) { return ((w >> (8
 template <bool VEC>
 __global__ __launch_bounds__(kRouteThreads) void route_counts_kernel(const uint8_t* __restrict__ map, int64_t T, int E,
                                                                      int64_t span, int chunks,
-                                                                     int32_t* __restrict__ counts) {
+                                                                     int32_t* __restrict__ counts,
+                                                                     int32_t* __restrict__ host_counts) {
   __shared__ int part[kRouteThreads / 64][kRouteExperts];
   const int chunk = blockIdx.x, e0 = blockIdx.y * kRouteExperts;
   const int t = threadIdx.x, wave = t >> 6;
@@ -77,8 +78,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_counts_kernel(const uint8
     for (int k = 0; k < kRouteExperts; k++) part[wave][k] = n[k];
   }
   __syncthreads();
-  if (t < kRouteExperts && e0 + t < E)
-    counts[(int64_t)(e0 + t) * chunks + chunk] = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+  if (t < kRouteExperts && e0 + t < E) {
+    const int sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+    const int64_t at = (int64_t)(e0 + t) * chunks + chunk;
+    counts[at] = sum;
+    if (host_counts) host_counts[at] = sum;
+  }
 }
 
 __device__ __forceinline__ int wave_sum(int v) {
@@ -163,12 +168,13 @@ __global__ __launch_bounds__(kRouteThreads) void route_rows_kernel(const uint8_t
 
 static bool route_vec(const void* map, int64_t E) { return E % 4 == 0 && (reinterpret_cast<uintptr_t>(map) & 3) == 0; }
 
-hipError_t launch_route_counts(const void* map, int64_t T, int64_t E, int32_t* counts, hipStream_t stream) {
+hipError_t launch_route_counts(const void* map, int64_t T, int64_t E, int32_t* counts, int32_t* host_counts,
+                               hipStream_t stream) {
   const int64_t chunks = route_chunks(T, E);
   const dim3 grid((unsigned)chunks, (unsigned)((E + kRouteExperts - 1) / kRouteExperts));
   auto kernel = route_vec(map, E) ? route_counts_kernel<true> : route_counts_kernel<false>;
   return launch(kernel, grid, dim3(kRouteThreads), 0, stream, static_cast<const uint8_t*>(map), T, (int)E,
-                route_span(T, E), (int)chunks, counts);
+                route_span(T, E), (int)chunks, counts, host_counts);
 }
 
 hipError_t launch_route_rows(const void* map, int64_t T, int64_t E, const int32_t* counts, int32_t* src,

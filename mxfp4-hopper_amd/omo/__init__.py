@@ -52,8 +52,6 @@ __all__ = [
     "omo_packed_Mxfp4_dequant",
     "omo_mxfp4_permute_rows",
     "omo_permute_Mxfp4ToFp8",
-    "omo_route_counts",
-    "omo_route_rows",
 ]
 
 _FP8 = torch.float8_e4m3fn
@@ -512,34 +510,3 @@ def omo_permute_Mxfp4ToFp8(codes, scales, src_rows, output_q, output_s):
     with _on_device(codes) as stream:
         _check(_lib.omo_hip_permute_Mxfp4ToFp8(*args, output_q.data_ptr(), output_q.numel(), output_s.data_ptr(),
                                                output_s.numel(), stream))
-
-
-def omo_route_counts(routing_map):
-    """Routed tokens of each expert per chunk of tokens, int32 [E, chunks], of
-    a contiguous bool routing map [T, E]."""
-    _check_input(routing_map, "routing_map")
-    if routing_map.dim() != 2:
-        raise RuntimeError("routing_map must be 2-D [tokens, experts]")
-    _check_dtype(routing_map, torch.bool, "routing_map")
-    T, E = routing_map.shape
-    counts = torch.empty((E, _lib.omo_hip_route_chunks(T, E)), dtype=torch.int32, device=routing_map.device)
-    with _on_device(routing_map) as stream:
-        _check(_lib.omo_hip_route_counts(routing_map.data_ptr(), T, E, counts.data_ptr(), counts.numel(), stream))
-    return counts
-
-
-def omo_route_rows(routing_map, counts, src_rows, pad, dest=None):
-    """Expert-major rows of a counted routing map: src_rows[r] = token of the
-    r-th routed (token, expert) pair by expert, then token (``pad``: -1 after
-    the last; pairs past its end are dropped), dest[t, e] = r or -1."""
-    _check_input(routing_map, "routing_map")
-    _check_dtype(routing_map, torch.bool, "routing_map")
-    for t, n in ((counts, "counts"), (src_rows, "src_rows")) + (() if dest is None else ((dest, "dest"),)):
-        _check_input(t, n)
-        _check_dtype(t, torch.int32, n)
-        _same_device(routing_map, t)
-    T, E = routing_map.shape
-    with _on_device(routing_map) as stream:
-        _check(_lib.omo_hip_route_rows(
-            routing_map.data_ptr(), T, E, counts.data_ptr(), counts.numel(), src_rows.data_ptr(), src_rows.numel(),
-            int(bool(pad)), 0 if dest is None else dest.data_ptr(), 0 if dest is None else dest.numel(), stream))

@@ -48,7 +48,7 @@ SIGNATURES = {
     "omo_hip_packed_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P],
     "omo_hip_mxfp4_permute_rows": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],
     "omo_hip_permute_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],
-    "omo_hip_route_counts": [_P, _I64, _I64, _P, _I64, _P],
+    "omo_hip_route_counts": [_P, _I64, _I64, _P, _I64, _P, _P],
     "omo_hip_route_rows": [_P, _I64, _I64, _P, _I64, _P, _I64, _I, _P, _I64, _P],
 }
 
@@ -63,8 +63,6 @@ def _load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = ctypes.c_int
-    lib.omo_hip_route_chunks.restype = ctypes.c_int64
-    lib.omo_hip_route_chunks.argtypes = [_I64, _I64]
     lib.omo_hip_abi_version.restype = ctypes.c_int
     lib.omo_hip_abi_version.argtypes = []
     lib.omo_hip_last_error.restype = ctypes.c_char_p

@@ -18,6 +18,7 @@ from typing import List, Optional, Tuple
 import torch
 
 from omo import DEQUANT_TYPES, omo_packed_Mxfp4_dequant, omo_packed_Mxfp4ToFp8, omo_quant_mxfp4_packed
+from omo._native import native
 
 
 def payload_width(hidden: int) -> int:
@@ -59,6 +60,9 @@ def fp4_quantize_packed(x: torch.Tensor, eps: float = 1e-10) -> torch.Tensor:
     """Fused ``fp4_quantize`` (megatron-0.15.0rc7.diff:163-170): bf16 [T, H]
     (H % 128 == 0) -> payload [T, 17H/32] uint8, equal to
     join_payload(*omo_per_token_group_quant_mxfp4(x))."""
+    done = native.quantize_packed(x, eps)
+    if done is not None:
+        return done
     assert x.dim() == 2, "`x` must be 2-D [tokens, hidden]"
     assert x.is_contiguous(), "`x` is not contiguous"
     T, H = x.shape
@@ -84,6 +88,9 @@ def packed_mxfp4ToFp8(packed: torch.Tensor, m_splits: Optional[List[int]] = None
     by ``m_splits`` along tokens as omo_per_token_mxfp4ToFp8_wrapper does
     (code/kernel/api/mxfp4_dequant.py:172-181); without m_splits the whole
     tensors are returned."""
+    done = native.requant_packed(packed, m_splits)
+    if done is not None:
+        return done
     assert packed.is_contiguous(), "payload is not contiguous"
     T, H = packed.size(0), hidden_of(packed)
     x_q = torch.empty((T, H), device=packed.device, dtype=torch.float8_e4m3fn)

@@ -2,13 +2,17 @@
 
 Mirrors code/kernel/api/mxfp4.py: same function names, defaults, output
 allocation and return values. The wrappers allocate the outputs with
-``torch.empty`` and call ``omo`` on the current stream.
+``torch.empty`` and call ``omo`` on the current stream. The entries that
+training calls try the native form of the same steps first
+(csrc/binding/omo_native.cpp); it answers None where a call is not the
+ordinary one, and the Python code here takes it.
 """
 from typing import Optional
 
 import torch
 
 from omo import omo_per_token_group_quant_fp4, omo_quant_mxfp4_dual, omo_quant_mxfp4_dual_grouped
+from omo._native import native
 
 fp8_type_ = torch.float8_e4m3fn
 uint8_type = torch.uint8
@@ -110,6 +114,9 @@ def omo_per_token_group_quant_mxfp4(x: torch.Tensor):
     """The quantize entry used by TE (mxfp4.py:118-156; called at
     code/transformer_engine-2.8.diff:672-673). x [M, K] bf16, K % 32 == 0 ->
     (codes uint8 [M, K/2], scales uint8 E8M0 [M, K/32])."""
+    done = native.quantize(x)
+    if done is not None:
+        return done
     group_size = 32
     eps = 1e-10
     scale_ue8m0 = False
@@ -137,6 +144,9 @@ def omo_per_token_group_quant_mxfp4_dual(x: torch.Tensor, eps: float = 1e-10):
     col scales [K, M/32]); the column pair equals
     omo_per_token_group_quant_mxfp4(x.T.contiguous()), which is how TE builds
     the columnwise usage (code/transformer_engine-2.8.diff:1463-1466)."""
+    done = native.quantize_dual(x, eps)
+    if done is not None:
+        return done
     assert x.dim() == 2, "`x` must be 2-D"
     M, K = x.shape
     assert M % 32 == 0 and K % 32 == 0, "both dimensions of `x` must be multiples of 32"
@@ -154,6 +164,9 @@ def omo_per_token_group_quant_mxfp4_dual_grouped(xs, eps: float = 1e-10):
     """omo_per_token_group_quant_mxfp4_dual over a list of 2-D bf16 tensors
     (e.g. the gate/up/down weights of all local experts) in one launch; returns
     one (row codes, row scales, col codes, col scales) tuple per tensor."""
+    done = native.quantize_dual_grouped(xs, eps)
+    if done is not None:
+        return done
     outs = []
     for x in xs:
         assert x.dim() == 2, "every tensor must be 2-D"

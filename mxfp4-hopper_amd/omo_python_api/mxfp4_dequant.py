@@ -7,6 +7,10 @@ reference does not ship:
   * omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper (code/transformer_engine-2.8.diff:70, 159-176)
 Their contracts are reconstructed from those call sites and from the host
 checks of the bound functions; eps = 1e-10 as in every shipped wrapper.
+
+The wrappers that training calls try the native form of the same steps first
+(csrc/binding/omo_native.cpp), which answers None where a call is not the
+ordinary one.
 """
 from typing import List
 
@@ -24,6 +28,7 @@ from omo import (
     omo_per_token_Mxfp4ToFp8,
     omo_per_token_Mxfp4ToFp8_col,
 )
+from omo._native import native
 
 fp8_type_ = torch.float8_e4m3fn
 uint8_type = torch.uint8
@@ -55,6 +60,9 @@ def omo_per_token_mxfp4ToBf16_dequant_wrapper(x: torch.Tensor, x_in_s: torch.Ten
     (mxfp4_dequant.py:39-74; called at code/transformer_engine-2.8.diff:392).
     fp16 and fp32 are written by the dequant itself; any other dtype is
     converted from bf16 in a second pass."""
+    done = native.dequantize(x, x_in_s, dtype)
+    if done is not None:
+        return done
     group_size = 32
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
@@ -102,6 +110,9 @@ def omo_per_token_mxfp4ToFp8_wrapper(x: torch.Tensor, x_in_s: torch.Tensor, m_sp
     codes padded to 64 bytes and scales to 4 columns, fp8 [M, 2Kp] + fp32
     [2Kp/128, M], sliced, then split by m_splits along rows (fp8, dim 0) and
     columns (scales, dim 1). Widths K % 32 == 0 are padded inside the kernel."""
+    done = native.requant(x, x_in_s, m_splits)
+    if done is not None:
+        return done
     group_size = 128
     eps = 1e-10
     scale_ue8m0 = False
@@ -154,6 +165,9 @@ def omo_per_token_mxfp4RowToBf16ToFp8Col_wrapper(data: torch.Tensor, scale: torc
     dense wgrad (code/transformer_engine-2.8.diff:259-272): codes [M, N/2] +
     scales [M, N/32] -> (fp8 columnwise data [N, M], fp32 columnwise
     scale_inv [ceil(M/128), N]) in TE's GEMM_READY layout."""
+    done = native.row_to_col(data, scale, eps)
+    if done is not None:
+        return done
     assert data.dim() == 2 and data.is_contiguous(), "`data` must be a contiguous 2-D tensor"
     M, half = data.shape
     N = half * 2
@@ -195,6 +209,9 @@ def omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper(data: torch.Tensor, scal
     Up to 128 splits of 16 B aligned code rows travel by value with the
     launch. More splits, and rows the 256-column tiles do not take, go through
     a device copy of the metadata, for which the host waits."""
+    done = native.row_to_col_splits(data, scale, m_splits, eps)
+    if done is not None:
+        return done
     assert data.dim() == 2 and data.is_contiguous(), "`data` must be a contiguous 2-D tensor"
     total_m, half = data.shape
     N = half * 2

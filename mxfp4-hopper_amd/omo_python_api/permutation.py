@@ -21,7 +21,8 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from omo import omo_mxfp4_permute_rows, omo_permute_Mxfp4ToFp8, omo_route_counts, omo_route_rows
+from omo import omo_mxfp4_permute_rows, omo_permute_Mxfp4ToFp8
+from omo._native import native
 
 
 def make_row_id_map(routing_map: torch.Tensor, num_out_tokens: Optional[int] = None
@@ -30,46 +31,18 @@ def make_row_id_map(routing_map: torch.Tensor, num_out_tokens: Optional[int] = N
     m_splits (routed tokens per expert), dest int32 [T, E]: the output row of
     each routed (token, expert) pair, -1 where not routed). Output rows are
     ordered by expert, then token; rows past the routed count are padding
-    (src_rows = -1)."""
-    rows, m_splits, dest = _row_map(routing_map, num_out_tokens, True)
-    return _own_rows(rows), m_splits, dest
+    (src_rows = -1).
 
-
-def _row_map(routing_map: torch.Tensor, num_out_tokens: Optional[int], want_dest: bool):
-    """make_row_id_map without its copy of the row order: src_rows may be the
-    head of a larger buffer (``_own_rows`` cuts it out). dest is None unless
-    asked for."""
-    rm = routing_map.bool()
-    T, E = rm.shape
-    if not (type(rm) is torch.Tensor and rm.is_cuda and 0 < T * E < 2**31 and E <= 4 * 65534
-            and (num_out_tokens is None or 0 <= num_out_tokens < 2**31)):
-        return _row_map_generic(rm, num_out_tokens)
-    # Both launches are enqueued before the host reads the loads: the row
-    # order then waits for nothing, and only the conversion that needs the
-    # number of rows follows the read. Without num_out_tokens that number is
-    # not known yet, so the order goes to a buffer for every pair.
-    rm = rm.contiguous()
-    counts = omo_route_counts(rm)
-    src = torch.empty((T * E if num_out_tokens is None else num_out_tokens,), dtype=torch.int32, device=rm.device)
-    dest = torch.empty((T, E), dtype=torch.int32, device=rm.device) if want_dest else None
-    omo_route_rows(rm, counts, src, num_out_tokens is not None, dest)
-    m_splits = counts.cpu().sum(1).tolist()
-    n = sum(m_splits)
-    if num_out_tokens is None:
-        return src[:n], m_splits, dest
-    if num_out_tokens < n:
-        raise ValueError(f"num_out_tokens={num_out_tokens} is smaller than the {n} routed tokens")
-    return src, m_splits, dest
-
-
-def _own_rows(src: torch.Tensor) -> torch.Tensor:
-    """src on storage of its own size."""
-    return src if src.untyped_storage().nbytes() == src.numel() * 4 else src.clone()
+    On the GPU one launch counts, the host reads the loads and a second launch
+    orders; ``_row_map_generic`` takes the rest."""
+    rm = routing_map.bool().contiguous()
+    done = native.make_row_map(rm, num_out_tokens)
+    return _row_map_generic(rm, num_out_tokens) if done is None else done
 
 
 def _row_map_generic(rm: torch.Tensor, num_out_tokens: Optional[int]):
     """The row map by torch operations: routing maps on the CPU, empty ones,
-    ones past 2^31 pairs."""
+    ones past 2^31 pairs, tensor subclasses."""
     T, E = rm.shape
     e_idx, t_idx = torch.nonzero(rm.t(), as_tuple=True)  # expert-major, ascending tokens
     n = t_idx.numel()
@@ -115,15 +88,19 @@ def mxfp4_permute_to_fp8(codes: torch.Tensor, scales: torch.Tensor, routing_map:
     (fp8 [N, H], fp32 scales [H/128, N], src_rows, m_splits); with split=True
     the first two are split by m_splits (plus one trailing split of padding
     rows, if any) the way omo_per_token_mxfp4ToFp8_wrapper splits them."""
-    src, m_splits, _ = _row_map(routing_map, num_out_tokens, False)
-    N, H = src.numel(), codes.size(1) * 2
-    x_q = torch.empty((N, H), dtype=torch.float8_e4m3fn, device=codes.device)
-    x_s = torch.empty((H // 128, N), dtype=torch.float32, device=codes.device)
-    if N > 0:
-        omo_permute_Mxfp4ToFp8(codes, scales, src.to(codes.device), x_q, x_s)
-    src = _own_rows(src)  # after the requant is enqueued: nothing waits for the copy
+    rm = routing_map.bool().contiguous()
+    done = native.permute_to_fp8(codes, scales, rm, num_out_tokens)
+    if done is not None:
+        x_q, x_s, src, m_splits = done
+    else:
+        src, m_splits, _ = make_row_id_map(rm, num_out_tokens)
+        N, H = src.numel(), codes.size(1) * 2
+        x_q = torch.empty((N, H), dtype=torch.float8_e4m3fn, device=codes.device)
+        x_s = torch.empty((H // 128, N), dtype=torch.float32, device=codes.device)
+        if N > 0:
+            omo_permute_Mxfp4ToFp8(codes, scales, src.to(codes.device), x_q, x_s)
     if split:
-        sp = _splits_with_padding(m_splits, N)
+        sp = _splits_with_padding(m_splits, src.numel())
         return torch.split(x_q, sp, dim=0), torch.split(x_s, sp, dim=1), src, m_splits
     return x_q, x_s, src, m_splits
 
