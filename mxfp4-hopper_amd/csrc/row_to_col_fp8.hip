@@ -49,10 +49,13 @@ constexpr int kCodePitch = 64 + 16;  // LDS bytes per code row (16 B aligned row
 
 constexpr int kRcThreads = 512;
 
-// LDS row of tile row r: the 8 lanes of a column read rows 16q + j at the
-// same time; storing row 16q + j at 8j + q puts those rows at consecutive LDS
-// rows (distinct banks) instead of 16 rows apart (the same bank).
-__device__ __forceinline__ int lds_row(int r) { return ((r & 15) << 3) | (r >> 4); }
+// LDS row of tile row r: the 8 lanes of a column read rows R q + j at the
+// same time; storing row R q + j at 8j + q puts those rows at consecutive LDS
+// rows (distinct banks) instead of R rows apart (the same bank for 16).
+template <int R = 16>
+__device__ __forceinline__ int lds_row(int r) {
+  return ((r & (R - 1)) << 3) | (r >> (R == 16 ? 4 : R == 8 ? 3 : 2));
+}
 
 // Maximum over the 8 lanes 8k..8k+7 (all active).
 __device__ __forceinline__ float oct_fmax(float v) {
@@ -355,38 +358,48 @@ __device__ __forceinline__ void rc_tile(RowColSmem& sm, int rows_valid, int64_t 
   res.e1 = u32x4{w1[0], w1[1], w1[2], w1[3]};
 }
 
-// Write a lane's 16 bytes of one output column (rows 16q .. 16q+15 of the
-// tile) to dst[0 .. 16), stopping at rows_valid. dst may have any byte
-// alignment: the 16 B store is emitted as one global_store_dwordx4, which
-// the hardware splits when it is unaligned (checked at every offset 0..15).
-// A partial piece of n = 1..15 bytes is written as at most four stores of 8,
-// 4, 2 and 1 bytes (the bits of n, largest first), so each one's source
-// bytes start at a multiple of its size within the 16 (a loop of single
-// byte stores cost 4 us over cfg5's ragged splits).
-__device__ __forceinline__ void rc_store(uint8_t* __restrict__ dst, const u32x4& w, int r_base, int rows_valid) {
-  if (r_base + 16 <= rows_valid) {
-    __builtin_memcpy(dst, &w, 16);
+// R consecutive output bytes of one column, R = 16, 8 or 4.
+template <int R>
+using RowBytes = uint32_t __attribute__((ext_vector_type(R / 4)));
+
+// Write a lane's R bytes of one output column (rows r_base .. r_base + R - 1
+// of the tile) to dst[0 .. R), stopping at rows_valid. dst may have any byte
+// alignment: a whole piece is emitted as one store, which the hardware
+// splits when it is unaligned (checked at every offset 0..15). A partial
+// piece of n = 1 .. R - 1 bytes is written as stores of 8, 4, 2 and 1 bytes
+// (the bits of n, largest first), so each one's source bytes start at a
+// multiple of its size within the piece (a loop of single byte stores cost
+// 4 us over cfg5's ragged splits).
+template <int R>
+__device__ __forceinline__ void rc_store(uint8_t* __restrict__ dst, const RowBytes<R>& w, int r_base, int rows_valid) {
+  if (r_base + R <= rows_valid) {
+    __builtin_memcpy(dst, &w, R);
   } else if (r_base < rows_valid) {
     const int n = rows_valid - r_base;
     int pos = 0;
-    if (n & 8) {
-      const u32x2 h = {w[0], w[1]};
-      __builtin_memcpy(dst, &h, 8);
-      pos = 8;
+    uint32_t wd = w[0], wn = R > 4 ? w[R > 4 ? 1 : 0] : 0u;  // dwords holding byte pos, and the next
+    if constexpr (R > 8) {
+      if (n & 8) {
+        const u32x2 h = {wd, wn};
+        __builtin_memcpy(dst, &h, 8);
+        pos = 8;
+        wd = w[2];
+        wn = w[3];
+      }
     }
-    const uint32_t wd = pos ? w[2] : w[0];  // dword holding byte pos
-    const uint32_t wn = pos ? w[3] : w[1];  // the next one
-    if (n & 4) {
-      __builtin_memcpy(dst + pos, &wd, 4);
-      pos += 4;
+    if constexpr (R > 4) {
+      if (n & 4) {
+        __builtin_memcpy(dst + pos, &wd, 4);
+        pos += 4;
+        wd = wn;
+      }
     }
-    const uint32_t v = (n & 4) ? wn : wd;   // dword holding byte pos now
     if (n & 2) {
-      const uint16_t h = (uint16_t)v;
+      const uint16_t h = (uint16_t)wd;
       __builtin_memcpy(dst + pos, &h, 2);
       pos += 2;
     }
-    if (n & 1) dst[pos] = (uint8_t)((n & 2) ? v >> 16 : v);
+    if (n & 1) dst[pos] = (uint8_t)((n & 2) ? wd >> 16 : wd);
   }
 }
 
@@ -432,8 +445,8 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_kernel(const uint8_
       __builtin_nontemporal_store(res.e0, reinterpret_cast<u32x4*>(out + c * M + row0 + 16 * qq));
       __builtin_nontemporal_store(res.e1, reinterpret_cast<u32x4*>(out + (c + 1) * M + row0 + 16 * qq));
     } else if (c < N) {
-      rc_store(out + c * M + row0 + 16 * qq, res.e0, 16 * qq, rows_valid);
-      rc_store(out + (c + 1) * M + row0 + 16 * qq, res.e1, 16 * qq, rows_valid);
+      rc_store<16>(out + c * M + row0 + 16 * qq, res.e0, 16 * qq, rows_valid);
+      rc_store<16>(out + (c + 1) * M + row0 + 16 * qq, res.e1, 16 * qq, rows_valid);
     }
     if (nxt >= tiles) break;
     tile = nxt;
@@ -483,15 +496,15 @@ __device__ __forceinline__ void cvt_pk_f32_fp4_once(uint32_t src, float scale, f
   *hi = r[1];
 }
 
-// Column maxima of the lane's 16 rows in fp32, two values per conversion.
+// Column maxima of the lane's R rows in fp32, two values per conversion.
 // Measured and not kept: sign bits cleared and v_cvt_scalef32_pk_bf16_fp4
 // into packed 16-bit maxima (two columns per v_pk_max_u16, exact for scale
 // bytes 1..252, a quarter fewer instructions): 9.17 against 8.86 us at
 // 4096 x 7168.
-template <int B>
-__device__ __forceinline__ void wide_amax_fast(const uint32_t (&cw)[16], const float (&sc)[16], float (&a)[8]) {
+template <int B, int R>
+__device__ __forceinline__ void wide_amax_fast(const uint32_t (&cw)[R], const float (&sc)[R], float (&a)[8]) {
 #pragma unroll
-  for (int j = 0; j < 16; j++) {
+  for (int j = 0; j < R; j++) {
     float v0, v1;
     cvt_pk_f32_fp4<B>(cw[j], sc[j], &v0, &v1);
     a[2 * B] = fmaxf(a[2 * B], fabsf(v0));
@@ -499,12 +512,12 @@ __device__ __forceinline__ void wide_amax_fast(const uint32_t (&cw)[16], const f
   }
 }
 
-// Columns 2b, 2b+1 of the lane (the nibbles of code byte b) for its 16 rows.
-template <int B, bool CLAMP>
-__device__ __forceinline__ void wide_pair_fast(const uint32_t (&cw)[16], const float (&sc)[16], float m0, float m1,
-                                               u32x4& w0, u32x4& w1) {
+// Columns 2b, 2b+1 of the lane (the nibbles of code byte b) for its R rows.
+template <int B, bool CLAMP, int R>
+__device__ __forceinline__ void wide_pair_fast(const uint32_t (&cw)[R], const float (&sc)[R], float m0, float m1,
+                                               RowBytes<R>& w0, RowBytes<R>& w1) {
 #pragma unroll
-  for (int j4 = 0; j4 < 4; j4++) {
+  for (int j4 = 0; j4 < R / 4; j4++) {
     float x[4], y[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -524,12 +537,12 @@ __device__ __forceinline__ void wide_pair_fast(const uint32_t (&cw)[16], const f
 // (checked equal on the GPU for every finite 2^k, k = -126 .. 127, over all
 // E2M1 magnitudes times 2^e and random inputs), one instruction per two
 // values instead of three.
-template <int B>
-__device__ __forceinline__ void wide_pair_scaled(const uint32_t (&cw)[16], const float (&sc)[16], float inv0,
-                                                 float inv1, u32x4& w0, u32x4& w1) {
+template <int B, int R>
+__device__ __forceinline__ void wide_pair_scaled(const uint32_t (&cw)[R], const float (&sc)[R], float inv0,
+                                                 float inv1, RowBytes<R>& w0, RowBytes<R>& w1) {
   typedef short s16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-  for (int j4 = 0; j4 < 4; j4++) {
+  for (int j4 = 0; j4 < R / 4; j4++) {
     float x[4], y[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) cvt_pk_f32_fp4_once<B>(cw[4 * j4 + k], sc[4 * j4 + k], &x[k], &y[k]);
@@ -545,28 +558,29 @@ __device__ __forceinline__ void wide_pair_scaled(const uint32_t (&cw)[16], const
   }
 }
 
-// Conversion of one staged wide tile: lane (cg, qq) converts element columns
-// 8cg .. 8cg+7 of tile rows 16qq .. 16qq+15 and hands column e's 16 bytes
-// (rows in order) to put(e, w). codes: the tile's first LDS code row (rows
-// permuted by lds_row, pitch bytes apart); scl / fscl: the 128 scale bytes
-// and 2^(s-127) patterns of the lane's MX column; fast: every scale byte of
-// the tile is in [1, 252] (else the restatement). The scale-row entry of
-// column 8cg + qq goes to out_s_lane when store_s. The 8 lanes of a code
-// dword must be 8 adjacent lanes of a wave.
-template <bool MSPLIT, typename Put>
+// Conversion of one staged wide tile of at most 8 R rows: lane (cg, qq)
+// converts element columns 8cg .. 8cg+7 of tile rows R qq .. R qq + R - 1 and
+// hands column e's R bytes (rows in order) to put(e, w). codes: the tile's
+// first LDS code row (rows permuted by lds_row<R>, pitch bytes apart); scl /
+// fscl: the scale bytes and 2^(s-127) patterns of the lane's MX column; fast:
+// every scale byte of the tile is in [1, 252] (else the restatement). The
+// scale-row entry of column 8cg + qq goes to out_s_lane when store_s. The 8
+// lanes of a code dword must be 8 adjacent lanes of a wave.
+template <bool MSPLIT, int R, typename Put>
 __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, const uint8_t* scl, const uint32_t* fscl,
                                              int cg, int qq, float eps, bool fast, bool store_s,
                                              float* __restrict__ out_s_lane, Put&& put) {
-  uint32_t cw[16];
-  float sc[16];
+  uint32_t cw[R];
+  float sc[R];
 #pragma unroll
-  for (int j4 = 0; j4 < 4; j4++) {
-    const u32x4 f = *reinterpret_cast<const u32x4*>(fscl + 16 * qq + 4 * j4);
+  for (int j4 = 0; j4 < R / 4; j4++) {
+    const u32x4 f = *reinterpret_cast<const u32x4*>(fscl + R * qq + 4 * j4);
 #pragma unroll
     for (int k = 0; k < 4; k++) sc[4 * j4 + k] = __uint_as_float(f[k]);
   }
 #pragma unroll
-  for (int j = 0; j < 16; j++) cw[j] = *reinterpret_cast<const uint32_t*>(codes + lds_row(16 * qq + j) * pitch + 4 * cg);
+  for (int j = 0; j < R; j++)
+    cw[j] = *reinterpret_cast<const uint32_t*>(codes + lds_row<R>(R * qq + j) * pitch + 4 * cg);
   float a[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) a[e] = MSPLIT ? 0.0f : eps;
@@ -576,9 +590,9 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
     wide_amax_fast<2>(cw, sc, a);
     wide_amax_fast<3>(cw, sc, a);
   } else {
-    const u32x4 sw = *reinterpret_cast<const u32x4*>(scl + 16 * qq);
+    const RowBytes<R> sw = *reinterpret_cast<const RowBytes<R>*>(scl + R * qq);
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
+    for (int j = 0; j < R; j++) {
       const float s16 = bf16_to_f32(((sw[j >> 2] >> (8 * (j & 3))) & 0xFFu) << 7);
 #pragma unroll
       for (int e = 0; e < 8; e++) a[e] = fmaxf(a[e], fabsf(bf16_to_f32(e2m1_to_bf16_bits((cw[j] >> (4 * e)) & 0xFu)) * s16));
@@ -619,7 +633,7 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
     }
   }
   if (fast && finite_m) {
-    u32x4 w0, w1;
+    RowBytes<R> w0, w1;
     if (MSPLIT && no_clamp) {
       wide_pair_scaled<0>(cw, sc, iv[0], iv[1], w0, w1);
       put(0, w0);
@@ -661,12 +675,12 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
       put(7, w1);
     }
   } else {
-    const u32x4 sw = *reinterpret_cast<const u32x4*>(scl + 16 * qq);
+    const RowBytes<R> sw = *reinterpret_cast<const RowBytes<R>*>(scl + R * qq);
 #pragma unroll 1
     for (int e = 0; e < 8; e++) {
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
+      RowBytes<R> w = 0u;
 #pragma unroll
-      for (int j = 0; j < 16; j += 2) {
+      for (int j = 0; j < R; j += 2) {
         float x[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -676,7 +690,7 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
         }
         w[j >> 2] |= fp8x2_from_f32(x[0], x[1]) << (8 * (j & 3));
       }
-      put(e, u32x4{w[0], w[1], w[2], w[3]});
+      put(e, w);
     }
   }
 }
@@ -698,8 +712,9 @@ __device__ __forceinline__ void wide_convert(const uint8_t* codes, int pitch, co
 // 0; cols_valid a multiple of 32): the missing 16 B code chunks of a row read
 // its last chunk and are zeroed, their scale bytes read as 127, and the lanes
 // of the missing columns store nothing.
-// NT_CODES: the code loads are non-temporal.
-template <bool MSPLIT, bool RAGGED, bool PARTIAL, bool SBYTE, bool NT_CODES>
+// NT_CODES: the code loads are non-temporal. R: rows per lane; the tile has at
+// most 8 R rows (R < 16 only with RAGGED).
+template <bool MSPLIT, bool RAGGED, bool PARTIAL, bool SBYTE, bool NT_CODES, int R>
 __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restrict__ q, const uint8_t* __restrict__ s,
                                           int64_t N, int64_t row0, int rows_valid, int64_t col0, float eps,
                                           float* __restrict__ out_s_row, uint8_t* __restrict__ obase, int64_t cstride,
@@ -717,17 +732,18 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
   // non-temporal per split (cfg5's 8 splits 50.3 against 49.0 us) and in the
   // dense rows-fastest order (4001 x 7168 12.6 against 11.8), ordinary in the
   // other dense orders (4096 x 7168 8.9 against 9.5 us non-temporal).
-  u32x4 cv[4];
+  constexpr int kLoads = R / 4;  // rounds of 32 rows
+  u32x4 cv[kLoads];
   const uint8_t* qt = q + row0 * (N / 2) + col0 / 2 + 16 * (PARTIAL ? min(t & 7, nch - 1) : (t & 7));
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < kLoads; k++) {
     const int r = (t >> 3) + 32 * k;
     const int64_t rr = RAGGED ? min(r, rows_valid - 1) : (t >> 3);
     const u32x4* src = reinterpret_cast<const u32x4*>(qt + rr * (N / 2) + (RAGGED ? 0 : 32 * k * (N / 2)));
     cv[k] = NT_CODES ? __builtin_nontemporal_load(src) : *src;
   }
   u32x2 sv = {0x7F7F7F7Fu, 0x7F7F7F7Fu};
-  if (t < kTile) {
+  if (t < 8 * R) {
     const uint8_t* srow = s + (row0 + (RAGGED ? min(t, rows_valid - 1) : t)) * (N / 32) + col0 / 32;
     if (SBYTE) {
       uint32_t w[2] = {0u, 0u};
@@ -740,18 +756,18 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
   }
   if (RAGGED || PARTIAL) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < kLoads; k++) {
       const int r = (t + 256 * k) >> 3, c16 = (t + 256 * k) & 7;
       if ((RAGGED && r >= rows_valid) || (PARTIAL && c16 >= nch)) cv[k] = u32x4{0u, 0u, 0u, 0u};
     }
     if (RAGGED && t >= rows_valid) sv = u32x2{0x7F7F7F7Fu, 0x7F7F7F7Fu};
   }
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < kLoads; k++) {
     const int id = t + 256 * k, r = id >> 3, c16 = id & 7;
-    *reinterpret_cast<u32x4*>(sm.codes + lds_row(r) * kWidePitch + c16 * 16) = cv[k];
+    *reinterpret_cast<u32x4*>(sm.codes + lds_row<R>(r) * kWidePitch + c16 * 16) = cv[k];
   }
-  if (t < kTile) {
+  if (t < 8 * R) {
 #pragma unroll
     for (int c = 0; c < 8; c++) {
       const uint32_t b = (sv[c >> 2] >> (8 * (c & 3))) & 0xFFu;
@@ -765,32 +781,59 @@ __device__ __forceinline__ void wide_tile(WideSmem& sm, const uint8_t* __restric
     if ((t & 63) == 0) sm.odd_scales[t >> 6] = (uint32_t)odd;
   }
   __syncthreads();
-  const bool fast = (sm.odd_scales[0] | sm.odd_scales[1]) == 0u;
+  const bool fast = (sm.odd_scales[0] | (R > 8 ? sm.odd_scales[1] : 0u)) == 0u;
   const int qq = t & 7, cg = t >> 3, mx = cg >> 2;
   const bool col_ok = !PARTIAL || mx < nch;  // this lane's 8 element columns exist
-  uint8_t* o = obase + 8 * cg * cstride + 16 * qq;
-  wide_convert<MSPLIT>(sm.codes, kWidePitch, sm.scales[mx], sm.fscales[mx], cg, qq, eps, fast, col_ok,
-                       out_s_row + 8 * cg + qq, [&](int e, const u32x4& w) {
+  uint8_t* o = obase + 8 * cg * cstride + R * qq;
+  wide_convert<MSPLIT, R>(sm.codes, kWidePitch, sm.scales[mx], sm.fscales[mx], cg, qq, eps, fast, col_ok,
+                       out_s_row + 8 * cg + qq, [&](int e, const RowBytes<R>& w) {
                          if (PARTIAL && !col_ok) return;
-                         if (RAGGED && !line_nt) rc_store(o + e * cstride, w, 16 * qq, rows_valid);
-                         else __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(o + e * cstride));
+                         if (RAGGED && (R < 16 || !line_nt)) rc_store<R>(o + e * cstride, w, R * qq, rows_valid);
+                         else __builtin_nontemporal_store(w, reinterpret_cast<RowBytes<R>*>(o + e * cstride));
                        });
 }
 
 // A tile of band col0 / 256: the whole band, or (NARROWN, N % 256 != 0)
-// the last band's N - col0 columns.
-template <bool MSPLIT, bool RAGGED, bool NARROWN, bool NT_CODES>
+// the last band's N - col0 columns; R rows per lane.
+template <bool MSPLIT, bool RAGGED, bool NARROWN, bool NT_CODES, int R>
+__device__ __forceinline__ void wide_tile_rows(WideSmem& sm, const uint8_t* __restrict__ q,
+                                               const uint8_t* __restrict__ s, int64_t N, int64_t row0, int rows_valid,
+                                               int64_t col0, float eps, float* __restrict__ out_s_row,
+                                               uint8_t* __restrict__ obase, int64_t cstride, bool line_nt) {
+  if (!NARROWN || col0 + kWideCols <= N) {
+    wide_tile<MSPLIT, RAGGED, false, NARROWN, NT_CODES, R>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase,
+                                                           cstride, line_nt);
+  } else {
+    wide_tile<MSPLIT, RAGGED, true, NARROWN, NT_CODES, R>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase,
+                                                          cstride, line_nt, (int)(N - col0));
+  }
+}
+
+// FEW: a tile of at most 32 or 64 rows is staged, converted and stored with 4
+// or 8 rows per lane instead of 16: its time is that of its lanes' rows, not
+// of its data. 32 splits of 300 x 7168 9.4 -> 6.7 us, of 1000 x 7168 10.4 ->
+// 8.4, of 8000 x 7168 27.4 -> 26.3; 8 of 16431 x 7168 42.3 -> 41.6; dense 50 x
+// 7168 4.9 -> 4.3. Not in the dense orders for many tiles, which have at most
+// one such row tile and lost to the larger kernel (8190 x 5120 17.5 -> 18.6).
+template <bool MSPLIT, bool RAGGED, bool NARROWN, bool NT_CODES, bool FEW>
 __device__ __forceinline__ void wide_tile_any(WideSmem& sm, const uint8_t* __restrict__ q,
                                               const uint8_t* __restrict__ s, int64_t N, int64_t row0, int rows_valid,
                                               int64_t col0, float eps, float* __restrict__ out_s_row,
                                               uint8_t* __restrict__ obase, int64_t cstride, bool line_nt) {
-  if (!NARROWN || col0 + kWideCols <= N) {
-    wide_tile<MSPLIT, RAGGED, false, NARROWN, NT_CODES>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
-                                              line_nt);
-  } else {
-    wide_tile<MSPLIT, RAGGED, true, NARROWN, NT_CODES>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase, cstride,
-                                             line_nt, (int)(N - col0));
+  if constexpr (FEW) {
+    if (rows_valid <= 32) {
+      wide_tile_rows<MSPLIT, RAGGED, NARROWN, NT_CODES, 4>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase,
+                                                           cstride, line_nt);
+      return;
+    }
+    if (rows_valid <= 64) {
+      wide_tile_rows<MSPLIT, RAGGED, NARROWN, NT_CODES, 8>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase,
+                                                           cstride, line_nt);
+      return;
+    }
   }
+  wide_tile_rows<MSPLIT, RAGGED, NARROWN, NT_CODES, 16>(sm, q, s, N, row0, rows_valid, col0, eps, out_s_row, obase,
+                                                        cstride, line_nt);
 }
 
 // Band walk: tile (S row tiles x B bands, T = S * B, numbered band by band
@@ -859,8 +902,8 @@ __global__ __launch_bounds__(256, 4) void row_to_fp8_col_wide_kernel(const uint8
   }
   const int64_t row0 = (int64_t)bm * kTile, col0 = (int64_t)bn * kWideCols;
   const int rows_valid = RAGGED ? (int)(M - row0 < kTile ? M - row0 : kTile) : kTile;
-  wide_tile_any<false, RAGGED, NARROWN, ORDER == kRowsFastest>(sm, q, s, N, row0, rows_valid, col0, eps,
-                                                               out_s + bm * N + col0, out + col0 * M + row0, M, false);
+  wide_tile_any<false, RAGGED, NARROWN, ORDER == kRowsFastest, RAGGED && ORDER == kBandsFastest>(
+      sm, q, s, N, row0, rows_valid, col0, eps, out_s + bm * N + col0, out + col0 * M + row0, M, false);
 }
 
 // Per split on the 256-column tiles: workgroup (split, bm, bn) as in
@@ -885,7 +928,7 @@ __device__ __forceinline__ void msplit_wide_tile(WideSmem& sm, const uint8_t* __
   if (start < 0 || start + len > total_rows || sstart < 0 || sstart + bm >= out_s_rows) return;
   const int64_t row0 = start + bm * kTile, col0 = bn * kWideCols;
   const int rows_valid = (int)(len - bm * kTile < kTile ? len - bm * kTile : kTile);
-  wide_tile_any<true, true, NARROWN, true>(sm, q, s, N, row0, rows_valid, col0, eps, out_s + (sstart + bm) * N + col0,
+  wide_tile_any<true, true, NARROWN, true, true>(sm, q, s, N, row0, rows_valid, col0, eps, out_s + (sstart + bm) * N + col0,
                                      out + start * N + col0 * len + bm * kTile, len,
                                      out_line && len % kTile == 0 && (start * N) % kTile == 0);
 }
@@ -1118,8 +1161,8 @@ __device__ __forceinline__ void msplit_narrow_tile(RowColSmem& sm, const uint8_t
   const int64_t c = col0 + 2 * p;
   if (c < N) {  // N is even: both columns or neither
     const int64_t o0 = start * N + c * len + bm * kTile + 16 * qq;
-    rc_store(out + o0, res.e0, 16 * qq, rows_valid);
-    rc_store(out + o0 + len, res.e1, 16 * qq, rows_valid);
+    rc_store<16>(out + o0, res.e0, 16 * qq, rows_valid);
+    rc_store<16>(out + o0 + len, res.e1, 16 * qq, rows_valid);
   }
 }
 

@@ -109,3 +109,31 @@ def test_captured_replays(oracle, dev):
         eo, es = oracle.row_to_fp8_col_msplit(hq, hs, lens)
         np.testing.assert_array_equal(np.concatenate([bits_u8(y).reshape(-1) for y in ys]), eo)
         np.testing.assert_array_equal(torch.cat(ss).cpu().numpy().view(np.uint32), es.view(np.uint32))
+
+
+# Tiles of 1 .. 128 rows: both sides of the 32- and 64-row forms, every count
+# of bytes in a lane's last piece, outputs at every byte alignment; scale
+# bytes of the fast path and of the restatement.
+@pytest.mark.parametrize("lo,hi", [(118, 136), (0, 256)])
+@pytest.mark.parametrize("N", [256, 352])
+def test_rows_per_lane(oracle, dev, N, lo, hi):
+    import omo
+    for lens in (list(range(1, 40)) + [63, 64, 65, 66, 67], [128 + m for m in (1, 3, 31, 32, 33, 60, 64, 65, 97, 127)]):
+        M, srows = sum(lens), sum((m + 127) // 128 for m in lens)
+        r = np.random.default_rng(M + N)
+        q = r.integers(0, 256, (M, N // 2), dtype=np.uint8)
+        s = r.integers(lo, hi, (M, N // 32)).astype(np.uint8)
+        out_q = torch.full((M * N,), 0xAB, dtype=torch.uint8, device=dev).view(FP8)
+        out_s = torch.full((srows, N), float("nan"), dtype=torch.float32, device=dev)
+        omo.omo_Mxfp4RowToBf16ToFp8Col_splits(torch.from_numpy(q).to(dev), torch.from_numpy(s).to(dev), out_q, out_s,
+                                              lens, 1e-10)
+        eo, es = oracle.row_to_fp8_col_msplit(q, s, lens)
+        np.testing.assert_array_equal(bits_u8(out_q), eo)
+        np.testing.assert_array_equal(out_s.cpu().numpy().view(np.uint32), es.view(np.uint32))
+        for m in lens[::5]:  # the dense form of the same heights
+            out_q, out_s = torch.empty((N, m), dtype=FP8, device=dev), torch.empty((-(-m // 128), N), device=dev)
+            omo.omo_per_token_Mxfp4RowToBf16ToFp8Col(torch.from_numpy(q[:m]).to(dev), torch.from_numpy(s[:m]).to(dev),
+                                                     out_q, out_s, 1e-10)
+            eo, es = oracle.row_to_fp8_col(q[:m], s[:m])
+            np.testing.assert_array_equal(bits_u8(out_q), eo)
+            np.testing.assert_array_equal(out_s.cpu().numpy().view(np.uint32), es.view(np.uint32))
