@@ -89,10 +89,17 @@ __device__ __forceinline__ uint2 quant_half16_ref(const uint32_t (&p)[8], float 
 
 // One 64 x 256 tile (index `logical`, M-fastest) of the [M, K] tensor x,
 // 512 threads. FULL: every tile of the tensor is whole (M % 64 == 0, K % 256
-// == 0) and its row scales are 8 B, its column scales 2 B aligned: no
-// clamping, no store under a bounds test (512 x 7168 4.90 -> 4.72 us, 2048 x
-// 7168 11.6 -> 11.3, 8192 x 7168 35.0 -> 34.8).
-template <bool FULL>
+// == 0): no clamping, no store under a bounds test (512 x 7168 4.90 -> 4.72
+// us, 2048 x 7168 11.6 -> 11.3, 8192 x 7168 35.0 -> 34.8). LINES: K % 256 ==
+// 0, so that the 128 B of codes a tile gives a row are a whole line and are
+// stored non-temporally (1056 x 7168 7.0 us, 7.5 with ordinary stores).
+// Without, every such piece shares its lines with the next tile's, and
+// ordinary stores let L2 complete them (4096 x 2880 10.7 -> 10.4 us, 4064 x
+// 7136 22.2 -> 22.0, 8192 x 5344 31.2 -> 30.8). A row's 8 scale
+// bytes and a column's 2 leave as one store at any alignment (byte by byte
+// where rows of K / 32 bytes are not 8 B aligned, 4096 x 2880 took 10.9 us
+// against 10.7).
+template <bool FULL, bool LINES>
 __device__ __forceinline__ void dual_tile(const uint16_t* __restrict__ x, uint32_t* __restrict__ row_q,
                                           uint8_t* __restrict__ row_s, uint8_t* __restrict__ col_q,
                                           uint8_t* __restrict__ col_s, int64_t M, int64_t K, int tiles_m,
@@ -135,13 +142,17 @@ __device__ __forceinline__ void dual_tile(const uint16_t* __restrict__ x, uint32
   // for the store as well (loads and stores share one counter).
 #pragma unroll
   for (int k = 0; k < 4; k++)
-    if (FULL || (r0 + 16 * k < rows_valid && col < K)) __builtin_nontemporal_store(codes[k], rq + k * 2 * K);  // 16 rows down
+    if (FULL || (r0 + 16 * k < rows_valid && col < K)) {
+      if (LINES) __builtin_nontemporal_store(codes[k], rq + k * 2 * K);  // 16 rows down
+      else rq[k * 2 * K] = codes[k];
+    }
   __syncthreads();
   if (t < rows_valid) {
     uint8_t* rs = row_s + (m0 + t) * (K / 32) + k0 / 32;
     const int nsc = FULL ? 8 : (int)((K - k0) / 32 < 8 ? (K - k0) / 32 : 8);
-    if (FULL || (nsc == 8 && (reinterpret_cast<uintptr_t>(rs) & 7) == 0)) {
-      *reinterpret_cast<uint2*>(rs) = *reinterpret_cast<const uint2*>(rs_tile + t * 8);
+    if (FULL || nsc == 8) {
+      const uint2 v = *reinterpret_cast<const uint2*>(rs_tile + t * 8);
+      __builtin_memcpy(rs, &v, 8);
     } else {
       for (int j = 0; j < nsc; j++) rs[j] = rs_tile[t * 8 + j];
     }
@@ -190,10 +201,9 @@ __device__ __forceinline__ void dual_tile(const uint16_t* __restrict__ x, uint32
   if (h == 0 && (FULL || kc < K)) {
     const int64_t so = m0 / 32;  // even: m0 is a multiple of 64
     uint8_t* const cs = col_s + (kc + g) * (M / 32) + so;
-    if (FULL || (rows_valid == kDualRows && (M / 32) % 2 == 0 &&
-                 (reinterpret_cast<uintptr_t>(col_s) & 1) == 0)) {
-      const uint32_t pair = g == 0 ? (byte_a | (oa << 8)) : (ob | (byte_b << 8));
-      *reinterpret_cast<uint16_t*>(cs) = (uint16_t)pair;
+    if (FULL || rows_valid == kDualRows) {
+      const uint16_t pair = (uint16_t)(g == 0 ? (byte_a | (oa << 8)) : (ob | (byte_b << 8)));
+      __builtin_memcpy(cs, &pair, 2);
     } else if (active) {
       col_s[kc * (M / 32) + so + g] = (uint8_t)byte_a;
       col_s[(kc + 1) * (M / 32) + so + g] = (uint8_t)byte_b;
@@ -422,7 +432,7 @@ __global__ __launch_bounds__(kDualThreads) __attribute__((amdgpu_waves_per_eu(6)
 // range. Measured (graph replays): 8192 x 7168 37.1 us against 38.3, 4096 x
 // 7168 20.7 against 21.1; with fewer than six tiles per CU the ranges are
 // ahead (7168 x 2048 11.7 against 12.0, 2048 x 2048 5.5 against 5.9).
-template <bool FULL>
+template <bool FULL, bool LINES>
 __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(const uint16_t* __restrict__ x, uint32_t* __restrict__ row_q,
                                                          uint8_t* __restrict__ row_s, uint8_t* __restrict__ col_q,
                                                          uint8_t* __restrict__ col_s, int64_t M, int64_t K,
@@ -440,7 +450,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(const uint16_t
     logical = (b % kXcds) * per_xcd + b / kXcds;
     if (logical >= tiles) return;
   }
-  dual_tile<FULL>(x, row_q, row_s, col_q, col_s, M, K, tiles_m, logical, eps, c_eps, tile, rs_tile);
+  dual_tile<FULL, LINES>(x, row_q, row_s, col_q, col_s, M, K, tiles_m, logical, eps, c_eps, tile, rs_tile);
 }
 
 // Grouped form: one launch over up to kDualGroupMax tensors (e.g. the weights
@@ -476,7 +486,7 @@ struct DualGroup {
 // one XCD) took 215-218 us for those items and 224-226 us for all items,
 // against 206-211 us. The four-tile kernel in this per-item band-group order
 // (quant_dual_grouped_super_kernel) made the cfg5 layer step 3.5 us slower.
-template <bool FULL>
+template <bool FULL, bool LINES>
 __global__ __launch_bounds__(kDualThreads) void quant_dual_grouped_kernel(const DualGroup g) {
   __shared__ __attribute__((aligned(16))) uint8_t tile[kDualRows * kDualPitch];
   __shared__ __attribute__((aligned(8))) uint8_t rs_tile[kDualRows * 8];
@@ -491,7 +501,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_grouped_kernel(const 
   const DualItem& it = g.item[i];
   int ms, kb;
   if (!band_group_tile(xcd, j, it.tiles_m, it.tiles, it.per_xcd, &ms, &kb)) return;
-  dual_tile<FULL>(it.x, it.row_q, it.row_s, it.col_q, it.col_s, it.M, it.K, it.tiles_m, kb * it.tiles_m + ms, g.eps,
+  dual_tile<FULL, LINES>(it.x, it.row_q, it.row_s, it.col_q, it.col_s, it.M, it.K, it.tiles_m, kb * it.tiles_m + ms, g.eps,
                   g.c_eps, tile, rs_tile);
 }
 
@@ -522,11 +532,8 @@ static bool dual_super_ok(const void* x, const void* row_q, const void* col_q, i
          (reinterpret_cast<uintptr_t>(row_q) & 15) == 0 && (reinterpret_cast<uintptr_t>(col_q) & 15) == 0;
 }
 
-// Tensors of whole 64 x 256 tiles whose scales take the wide stores.
-static bool dual_full(const void* row_s, const void* col_s, int64_t M, int64_t K) {
-  return M % kDualRows == 0 && K % kDualCols == 0 && (reinterpret_cast<uintptr_t>(row_s) & 7) == 0 &&
-         (reinterpret_cast<uintptr_t>(col_s) & 1) == 0;
-}
+// Tensors of whole 64 x 256 tiles.
+static bool dual_full(int64_t M, int64_t K) { return M % kDualRows == 0 && K % kDualCols == 0; }
 
 hipError_t launch_quant_dual(const void* x, void* row_q, void* row_s, void* col_q, void* col_s, int64_t M, int64_t K,
                              float eps, hipStream_t stream) {
@@ -548,7 +555,9 @@ hipError_t launch_quant_dual(const void* x, void* row_q, void* row_s, void* col_
   }
   const int64_t per_xcd = (tiles + kXcds - 1) / kXcds;
   const bool band_group = tiles >= 6 * (int64_t)current_device_caps().cus;
-  auto kernel = dual_full(row_s, col_s, M, K) ? quant_dual_kernel<true> : quant_dual_kernel<false>;
+  auto kernel = dual_full(M, K)        ? quant_dual_kernel<true, true>
+                : K % kDualCols == 0 ? quant_dual_kernel<false, true>
+                                     : quant_dual_kernel<false, false>;
   return launch(kernel, dim3((unsigned)(per_xcd * kXcds)), dim3(kDualThreads), 0, stream,
                      static_cast<const uint16_t*>(x), static_cast<uint32_t*>(row_q), static_cast<uint8_t*>(row_s),
                      static_cast<uint8_t*>(col_q), static_cast<uint8_t*>(col_s), M, K, (int)tiles_m, (int)tiles,
@@ -561,11 +570,12 @@ hipError_t launch_quant_dual_grouped(const DualSpec* items, int count, float eps
     memset(&g, 0, sizeof(g));
     g.count = count - base < kDualGroupMax ? count - base : kDualGroupMax;
     // the four-tile kernel where every item would take it alone
-    bool super = true, full = true;
+    bool super = true, full = true, lines = true;
     for (int j = 0; j < g.count; j++) {
       const DualSpec& d = items[base + j];
       const int64_t st = ((d.M + kSuperRows - 1) / kSuperRows) * ((d.K + kDualCols - 1) / kDualCols);
-      full = full && dual_full(d.row_s, d.col_s, d.M, d.K);
+      full = full && dual_full(d.M, d.K);
+      lines = lines && d.K % kDualCols == 0;
       super = super && (d.M == 0 || d.K == 0 ||
                         (dual_super_ok(d.x, d.row_q, d.col_q, d.M, d.K) && st >= 4 * (int64_t)current_device_caps().cus));
     }
@@ -592,9 +602,10 @@ hipError_t launch_quant_dual_grouped(const DualSpec* items, int count, float eps
     g.per_xcd = super_slots;
     g.eps = eps;
     g.c_eps = host_c_eps(eps, 6.0f);
-    auto kernel = super  ? quant_dual_grouped_super_kernel
-                  : full ? quant_dual_grouped_kernel<true>
-                         : quant_dual_grouped_kernel<false>;
+    auto kernel = super   ? quant_dual_grouped_super_kernel
+                  : full  ? quant_dual_grouped_kernel<true, true>
+                  : lines ? quant_dual_grouped_kernel<false, true>
+                          : quant_dual_grouped_kernel<false, false>;
     const hipError_t e = launch(kernel, dim3((unsigned)(g.per_xcd * kXcds)), dim3(kDualThreads), 0, stream, g);
     if (e != hipSuccess) return e;
   }

@@ -1,6 +1,7 @@
-"""Dual-layout quantize on tensors of whole 64 x 256 tiles, and the same with
-scale buffers that cannot take the wide stores: every byte against the
-rowwise oracle of x and of its transpose, alone and grouped."""
+"""Dual-layout quantize on tensors of whole 64 x 256 tiles and just short of
+them, with scale buffers at odd addresses and rows of an odd number of scale
+bytes: every byte, and none around, against the rowwise oracle of x and of its
+transpose, alone and grouped."""
 import numpy as np
 import pytest
 import torch
@@ -25,9 +26,10 @@ def _check(oracle, x, outs):
         np.testing.assert_array_equal(bits_u8(s).reshape(-1), np.asarray(es).reshape(-1))
 
 
-# one tile; two of each; an inf block (the restated path); one tile short of whole
-@pytest.mark.parametrize("M,K", [(64, 256), (128, 512), (96, 256), (64, 288)])
-@pytest.mark.parametrize("row_shift,col_shift", [(0, 0), (4, 0), (0, 1)])
+# one tile; two of each; an inf block (the restated path); one tile short of
+# whole in each direction; 9 and 15 scale bytes per row, 3 and 5 per column
+@pytest.mark.parametrize("M,K", [(64, 256), (128, 512), (96, 256), (64, 288), (160, 480)])
+@pytest.mark.parametrize("row_shift,col_shift", [(0, 0), (4, 0), (0, 1), (3, 5)])
 def test_whole_tiles(oracle, dev, M, K, row_shift, col_shift):
     import omo
     print("dual whole tiles", M, K, row_shift, col_shift, flush=True)
@@ -41,3 +43,7 @@ def test_whole_tiles(oracle, dev, M, K, row_shift, col_shift):
     torch.cuda.synchronize()
     for o in [outs] + grouped:
         _check(oracle, x, o)
+        for buf in o:  # nothing before or after the buffer was written
+            whole = torch.as_strided(buf, (buf.untyped_storage().nbytes(),), (1,), 0)
+            at = buf.storage_offset()
+            assert (whole[:at] == 0xAB).all() and (whole[at + buf.numel():] == 0xAB).all()
