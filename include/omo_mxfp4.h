@@ -262,6 +262,15 @@ OMO_API int omo_hip_permute_Mxfp4ToFp8(const void* codes, int64_t codes_bytes, i
                                        void* output_q, int64_t output_q_bytes, void* output_s,
                                        int64_t output_s_elems, void* stream);
 
+/* The same, with src_rows also copied to src_copy (num_out int32, or NULL):
+ * a row order held in a larger scratch buffer needs no copy of its own. */
+OMO_API int omo_hip_permute_Mxfp4ToFp8_copy(const void* codes, int64_t codes_bytes, int64_t code_stride,
+                                            const void* scales, int64_t scales_bytes, int64_t scale_stride,
+                                            int64_t num_tokens, int64_t cols, const int32_t* src_rows,
+                                            int64_t num_out, int32_t* src_copy, void* output_q,
+                                            int64_t output_q_bytes, void* output_s, int64_t output_s_elems,
+                                            void* stream);
+
 /* Expert-major row order of a MoE routing map (the row map of TE's
  * moe_permute, code/transformer_engine-2.8.diff:220-356). map [tokens,
  * experts], one byte per pair, non-zero where routed; fewer than 2^31 pairs.

@@ -389,12 +389,16 @@ PyObject* requant_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // --------------------------------------------------------------- permutation
 struct RowMap {
-  Tensor src, dest;
+  Tensor src, dest;            // src: the row order, `rows` entries at its head
+  int64_t rows = 0;
   std::vector<int64_t> loads;
 };
 
-// num_out: rows asked for, or -1. False: a Python error is set.
-bool row_map(const Tensor& map, int64_t num_out, bool want_dest, RowMap* r) {
+// num_out: rows asked for, or -1. `ahead`: the order is enqueued before the
+// host waits for the loads, so that nothing is left to do after the wait; with
+// num_out < 0 its length is not known then and src is scratch for every pair.
+// False: a Python error is set.
+bool row_map(const Tensor& map, int64_t num_out, bool want_dest, bool ahead, RowMap* r) {
   const int64_t T = map.size(0), E = map.size(1), chunks = omo_hip_route_chunks(T, E);
   const hipStream_t stream = stream_of(map);
   const Tensor counts = empty_like_device(map, {E * chunks}, at::kInt);
@@ -404,10 +408,35 @@ bool row_map(const Tensor& map, int64_t num_out, bool want_dest, RowMap* r) {
   if (!ok(omo_hip_route_counts(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks, seen.data_ptr<int32_t>(),
                                stream)))
     return false;
+  auto order = [&](int64_t rows, bool pad) {
+    r->src = empty_like_device(map, {rows}, at::kInt);
+    if (want_dest) r->dest = empty_like_device(map, {T, E}, at::kInt);
+    return ok(omo_hip_route_rows(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
+                                 rows ? r->src.data_ptr<int32_t>() : nullptr, rows, pad,
+                                 want_dest ? r->dest.data_ptr<int32_t>() : nullptr, want_dest ? T * E : 0, stream));
+  };
   hipError_t e;
-  Py_BEGIN_ALLOW_THREADS
-  e = hipStreamSynchronize(stream);
-  Py_END_ALLOW_THREADS
+  if (ahead) {
+    hipEvent_t counted;
+    e = hipEventCreateWithFlags(&counted, hipEventDisableTiming);
+    if (e == hipSuccess) {
+      e = hipEventRecord(counted, stream);
+      if (e == hipSuccess && !order(num_out < 0 ? T * E : num_out, num_out >= 0)) {
+        (void)hipEventDestroy(counted);
+        return false;
+      }
+      if (e == hipSuccess) {
+        Py_BEGIN_ALLOW_THREADS
+        e = hipEventSynchronize(counted);
+        Py_END_ALLOW_THREADS
+      }
+      (void)hipEventDestroy(counted);
+    }
+  } else {
+    Py_BEGIN_ALLOW_THREADS
+    e = hipStreamSynchronize(stream);
+    Py_END_ALLOW_THREADS
+  }
   if (e != hipSuccess) {
     PyErr_Format(PyExc_RuntimeError, "omo_route_counts: %s", hipGetErrorString(e));
     return false;
@@ -424,12 +453,8 @@ bool row_map(const Tensor& map, int64_t num_out, bool want_dest, RowMap* r) {
                  (long long)routed);
     return false;
   }
-  r->src = empty_like_device(map, {num_out < 0 ? routed : num_out}, at::kInt);
-  if (want_dest) r->dest = empty_like_device(map, {T, E}, at::kInt);
-  return ok(omo_hip_route_rows(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
-                               r->src.numel() ? r->src.data_ptr<int32_t>() : nullptr, r->src.numel(),
-                               num_out > routed, want_dest ? r->dest.data_ptr<int32_t>() : nullptr,
-                               want_dest ? T * E : 0, stream));
+  r->rows = num_out < 0 ? routed : num_out;
+  return ahead || order(r->rows, num_out > routed);
 }
 
 const Tensor* plain_map(PyObject* o) {
@@ -470,7 +495,7 @@ PyObject* make_row_map(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!map || !num_out_of(a[1], &num_out) || !quiet()) return none();
   const c10::DeviceGuard guard(map->device());
   RowMap m;
-  if (!row_map(*map, num_out, true, &m)) return nullptr;
+  if (!row_map(*map, num_out, true, false, &m)) return nullptr;
   PyObject* loads = list_of_ints(m.loads);
   PyObject* rest = pair_of(loads, THPVariable_Wrap(std::move(m.dest)));
   PyObject* head = rest ? THPVariable_Wrap(std::move(m.src)) : nullptr;
@@ -505,15 +530,20 @@ PyObject* permute_to_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   const c10::DeviceGuard guard(map->device());
   RowMap m;
-  if (!row_map(*map, num_out, false, &m)) return nullptr;
-  const int64_t N = m.src.numel();
+  // The order goes ahead of the wait; the requant, which has to know the
+  // number of rows, copies it from the scratch to its own buffer.
+  if (!row_map(*map, num_out, false, true, &m)) return nullptr;
+  const int64_t N = m.rows;
+  const bool scratch = m.src.numel() != N;
+  const Tensor src = scratch ? empty_like_device(*codes, {N}, at::kInt) : m.src;
   const Tensor q = empty_like_device(*codes, {N, H}, kFp8), s = empty_like_device(*codes, {H / 128, N}, at::kFloat);
-  if (N > 0 && !ok(omo_hip_permute_Mxfp4ToFp8(codes->data_ptr(), cspan, cstride, scales->data_ptr(), sspan, sstride, T,
-                                              H, m.src.data_ptr<int32_t>(), N, q.data_ptr(), q.numel(), s.data_ptr(),
-                                              s.numel(), stream_of(*codes))))
+  if (N > 0 && !ok(omo_hip_permute_Mxfp4ToFp8_copy(
+                   codes->data_ptr(), cspan, cstride, scales->data_ptr(), sspan, sstride, T, H,
+                   m.src.data_ptr<int32_t>(), N, scratch ? src.data_ptr<int32_t>() : nullptr, q.data_ptr(), q.numel(),
+                   s.data_ptr(), s.numel(), stream_of(*codes))))
     return nullptr;
   PyObject* loads = list_of_ints(m.loads);
-  PyObject* ts = loads ? tuple_of({q, s, m.src}) : nullptr;
+  PyObject* ts = loads ? tuple_of({q, s, src}) : nullptr;
   PyObject* r = ts ? PyTuple_Pack(4, PyTuple_GET_ITEM(ts, 0), PyTuple_GET_ITEM(ts, 1), PyTuple_GET_ITEM(ts, 2), loads)
                    : nullptr;
   Py_XDECREF(ts);

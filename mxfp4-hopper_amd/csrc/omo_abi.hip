@@ -178,6 +178,29 @@ int check_dual(const char* fn, const void* input, int64_t rows, int64_t cols, co
   return OMO_OK;
 }
 
+int permute_to_fp8(const char* fn, const void* codes, int64_t codes_bytes, int64_t code_stride, const void* scales,
+                   int64_t scales_bytes, int64_t scale_stride, int64_t num_tokens, int64_t cols,
+                   const int32_t* src_rows, int64_t num_out, int32_t* src_copy, void* output_q,
+                   int64_t output_q_bytes, void* output_s, int64_t output_s_elems, void* stream) {
+  int rc = check_permute(fn, codes, codes_bytes, code_stride, scales, scales_bytes, scale_stride, num_tokens, cols,
+                         src_rows, num_out);
+  if (rc != OMO_OK) return rc;
+  REQUIRE(cols % 128 == 0, "%s: cols must be a multiple of 128 (got %lld)", fn, (long long)cols);
+  REQUIRE(code_stride % 4 == 0 && scale_stride % 4 == 0 && aligned(codes, 4) && aligned(scales, 4),
+          "%s: code and scale rows must be 4-byte aligned", fn);
+  REQUIRE(cols / 128 * num_out < ((int64_t)1 << 31), "%s: too many groups", fn);
+  REQUIRE_BUF("output_q", output_q, output_q_bytes, num_out * cols);
+  REQUIRE_BUF("output_s", output_s, output_s_elems, num_out * (cols / 128));
+  REQUIRE(aligned(output_q, 16) && aligned(output_s, 4), "%s: output_q needs 16-byte, output_s 4-byte alignment",
+          fn);
+  REQUIRE(aligned(src_copy, 4), "%s: src_copy must be 4-byte aligned", fn);
+  if (num_out == 0 || cols == 0) return ok();
+  return from_hip(omo_hip::launch_mxfp4_to_fp8_rows(codes, code_stride, scales, scale_stride, src_rows, num_tokens,
+                                                    src_copy, output_q, static_cast<float*>(output_s), num_out,
+                                                    cols / 2, as_stream(stream)),
+                  fn);
+}
+
 }  // namespace
 
 extern "C" {
@@ -476,7 +499,7 @@ int omo_hip_packed_Mxfp4ToFp8(const void* input, int64_t rows, int64_t cols, voi
           "%s: input needs 4-byte, output_q 16-byte, output_s 4-byte alignment", fn);
   if (rows == 0 || cols == 0) return ok();
   const uint8_t* in = static_cast<const uint8_t*>(input);
-  return from_hip(omo_hip::launch_mxfp4_to_fp8_rows(in, stride, in + cols / 2, stride, nullptr, rows, output_q,
+  return from_hip(omo_hip::launch_mxfp4_to_fp8_rows(in, stride, in + cols / 2, stride, nullptr, rows, nullptr, output_q,
                                                     static_cast<float*>(output_s), rows, cols / 2,
                                                     as_stream(stream)),
                   fn);
@@ -535,23 +558,18 @@ int omo_hip_permute_Mxfp4ToFp8(const void* codes, int64_t codes_bytes, int64_t c
                                int64_t scales_bytes, int64_t scale_stride, int64_t num_tokens, int64_t cols,
                                const int32_t* src_rows, int64_t num_out, void* output_q, int64_t output_q_bytes,
                                void* output_s, int64_t output_s_elems, void* stream) {
-  const char* fn = "omo_permute_Mxfp4ToFp8";
-  int rc = check_permute(fn, codes, codes_bytes, code_stride, scales, scales_bytes, scale_stride, num_tokens, cols,
-                         src_rows, num_out);
-  if (rc != OMO_OK) return rc;
-  REQUIRE(cols % 128 == 0, "%s: cols must be a multiple of 128 (got %lld)", fn, (long long)cols);
-  REQUIRE(code_stride % 4 == 0 && scale_stride % 4 == 0 && aligned(codes, 4) && aligned(scales, 4),
-          "%s: code and scale rows must be 4-byte aligned", fn);
-  REQUIRE(cols / 128 * num_out < ((int64_t)1 << 31), "%s: too many groups", fn);
-  REQUIRE_BUF("output_q", output_q, output_q_bytes, num_out * cols);
-  REQUIRE_BUF("output_s", output_s, output_s_elems, num_out * (cols / 128));
-  REQUIRE(aligned(output_q, 16) && aligned(output_s, 4), "%s: output_q needs 16-byte, output_s 4-byte alignment",
-          fn);
-  if (num_out == 0 || cols == 0) return ok();
-  return from_hip(omo_hip::launch_mxfp4_to_fp8_rows(codes, code_stride, scales, scale_stride, src_rows, num_tokens,
-                                                    output_q, static_cast<float*>(output_s), num_out, cols / 2,
-                                                    as_stream(stream)),
-                  fn);
+  return permute_to_fp8("omo_permute_Mxfp4ToFp8", codes, codes_bytes, code_stride, scales, scales_bytes, scale_stride,
+                        num_tokens, cols, src_rows, num_out, nullptr, output_q, output_q_bytes, output_s,
+                        output_s_elems, stream);
+}
+
+int omo_hip_permute_Mxfp4ToFp8_copy(const void* codes, int64_t codes_bytes, int64_t code_stride, const void* scales,
+                                    int64_t scales_bytes, int64_t scale_stride, int64_t num_tokens, int64_t cols,
+                                    const int32_t* src_rows, int64_t num_out, int32_t* src_copy, void* output_q,
+                                    int64_t output_q_bytes, void* output_s, int64_t output_s_elems, void* stream) {
+  return permute_to_fp8("omo_permute_Mxfp4ToFp8_copy", codes, codes_bytes, code_stride, scales, scales_bytes,
+                        scale_stride, num_tokens, cols, src_rows, num_out, src_copy, output_q, output_q_bytes,
+                        output_s, output_s_elems, stream);
 }
 
 }  // extern "C"

@@ -66,12 +66,12 @@ hipError_t launch_dequant_rows(const void* q, int64_t q_stride, const void* s, i
                                FloatType type, int64_t rows, int64_t K, hipStream_t stream);
 
 // src: optional int32 source row per output row (indices outside [0, n_src)
-// read zeros); M output rows. Kb code bytes per row: a multiple of 64, or,
+// read zeros), copied to src_out where not null; M output rows. Kb code bytes per row: a multiple of 64, or,
 // without src and with 8 B aligned rows, of 16 (the outputs then those of
 // rows padded with zeros to 64).
 hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void* s, int64_t s_stride,
-                                    const int32_t* src, int64_t n_src, void* out, float* out_s, int64_t M, int64_t Kb,
-                                    hipStream_t stream);
+                                    const int32_t* src, int64_t n_src, int32_t* src_out, void* out, float* out_s,
+                                    int64_t M, int64_t Kb, hipStream_t stream);
 
 // Gather rows of two byte tensors (codes and scales of MXFP4 rows) into
 // contiguous outputs: out row r = input row src[r]; zeros for indices

@@ -118,7 +118,8 @@ constexpr int kRqRowsSmall = 8;
 // src (optional): output row r reads input row src[r] (a gather, e.g. the
 // expert-major token order of a MoE permutation); an index outside
 // [0, n_src) reads zero codes and zero scale bytes, i.e. the row a permutation
-// pads with zeros, requantized.
+// pads with zeros, requantized. src_out (optional): a copy of src, so that a
+// row order built in a larger buffer needs no copy launch of its own.
 // ROWS64: rows addressed with 64-bit products (a gather, or strides or
 // output rows of 2^24 bytes and more); otherwise addresses are a
 // workgroup-uniform tile base plus 32-bit lane offsets (24-bit products).
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
                                                            const int32_t* __restrict__ src, int64_t n_src,
                                                            u32x4* __restrict__ out, float* __restrict__ out_s,
                                                            uint32_t M, uint32_t gpr, uint32_t gx, uint32_t kb,
-                                                           uint32_t ks) {
+                                                           uint32_t ks, int32_t* __restrict__ src_out) {
   constexpr int PPR = 8 * kRqGroups;  // pairs per tile row
   constexpr int UNROLL = ROWS * PPR / 256;
   constexpr int RSTEP = 256 / PPR;    // rows between one lane's pairs
@@ -161,6 +162,11 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
     if (src) {
 #pragma unroll
       for (int u = 0; u < UNROLL; u++) sr[u] = src[min(row0 + lr0 + u * RSTEP, M - 1)];
+      if (src_out && bx == 0 && t % PPR == 0) {
+#pragma unroll
+        for (int u = 0; u < UNROLL; u++)
+          if (row0 + lr0 + u * RSTEP < M) src_out[row0 + lr0 + u * RSTEP] = (int32_t)sr[u];
+      }
     } else {
 #pragma unroll
       for (int u = 0; u < UNROLL; u++) sr[u] = min(row0 + lr0 + u * RSTEP, M - 1);
@@ -262,8 +268,8 @@ __global__ __launch_bounds__(256) void mxfp4_to_fp8_kernel(const uint8_t* __rest
 }
 
 hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void* s, int64_t s_stride,
-                                    const int32_t* src, int64_t n_src, void* out, float* out_s, int64_t M, int64_t Kb,
-                                    hipStream_t stream) {
+                                    const int32_t* src, int64_t n_src, int32_t* src_out, void* out, float* out_s,
+                                    int64_t M, int64_t Kb, hipStream_t stream) {
   if (M == 0 || Kb == 0) return hipSuccess;
   const int64_t gpr = (Kb + 63) / 64;
   const bool tail = Kb % 64 != 0;
@@ -279,7 +285,7 @@ hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void*
   const bool a8 = (q_stride % 8 == 0) && ((reinterpret_cast<uintptr_t>(q) & 7) == 0);
   const bool r64 = src || q_stride >= (1 << 24) || s_stride >= (1 << 24) || 128 * gpr >= (1 << 24);
   using Kernel = void (*)(const uint8_t*, int64_t, const uint8_t*, int64_t, const int32_t*, int64_t, u32x4*, float*,
-                          uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
+                          uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, int32_t*);
   // [rows: 8, 16, 32][a8][r64]
   static const Kernel table[3][2][2] = {
       {{mxfp4_to_fp8_kernel<kRqRowsSmall, false, false, false>, mxfp4_to_fp8_kernel<kRqRowsSmall, false, true, false>},
@@ -297,12 +303,12 @@ hipError_t launch_mxfp4_to_fp8_rows(const void* q, int64_t q_stride, const void*
   return launch(tail ? tails[ri][r64] : table[ri][a8][r64], dim3((unsigned)(gx * gy)), dim3(256), 0, stream,
                 static_cast<const uint8_t*>(q), q_stride, static_cast<const uint8_t*>(s), s_stride, src, n_src,
                 static_cast<u32x4*>(out), out_s, (uint32_t)M, (uint32_t)gpr, (uint32_t)gx, (uint32_t)Kb,
-                (uint32_t)(Kb / 16));
+                (uint32_t)(Kb / 16), src_out);
 }
 
 hipError_t launch_mxfp4_to_fp8(const void* q, const void* s, void* out, float* out_s, int64_t M, int64_t Kb,
                                hipStream_t stream) {
-  return launch_mxfp4_to_fp8_rows(q, Kb, s, Kb / 16, nullptr, M, out, out_s, M, Kb, stream);
+  return launch_mxfp4_to_fp8_rows(q, Kb, s, Kb / 16, nullptr, M, nullptr, out, out_s, M, Kb, stream);
 }
 
 // ------------------------------------------------------------ transposed
