@@ -226,7 +226,6 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
     import ctypes
     fl = ctypes.CDLL(os.path.join(ROOT, "mxfp4-hopper_amd", "lib", "libomo_ceiling.so"))
     P, I64 = ctypes.c_void_p, ctypes.c_int64
-    fl.omo_floor_dual.argtypes = [P, P, P, P, P, I64, I64, P]
     fl.omo_floor_rowcol.argtypes = [P, P, P, P, I64, I64, P]
     fl.omo_floor_msplit.argtypes = [P, P, P, P, I64, I64, P, P, P, I64, I64, I64, P]
     fl.omo_floor_requant.argtypes = [P, P, P, P, I64, I64, P]
@@ -261,24 +260,27 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
     n = M * K
     xd = [wl.heavy_tail_weights(M, K, seed=33 + i, device=dev) for i in range(2)]
     od = [[torch.empty(b, dtype=torch.uint8, device=dev) for b in (n // 2, n // 32, n // 2, n // 32)] for _ in range(2)]
-    pair("dual", "dual-layout quantize 7168x18432 (quant_dual_super_kernel)", wl.dual_quant_bytes(n), 2,
+    PA1, I1 = ctypes.c_void_p * 1, ctypes.c_int64 * 1
+    d_ptrs = [[PA1(xd[i].data_ptr())] + [PA1(od[i][k].data_ptr()) for k in range(4)] for i in range(2)]
+    pair("dual", "dual-layout quantize 7168x18432 (quant_dual_kernel)", wl.dual_quant_bytes(n), 2,
          lambda i: chk(lib.omo_hip_quant_mxfp4_dual(xd[i].data_ptr(), M, K, od[i][0].data_ptr(), n // 2,
                                                     od[i][1].data_ptr(), n // 32, od[i][2].data_ptr(), n // 2,
                                                     od[i][3].data_ptr(), n // 32, 1e-10, cur()), "dual"),
-         lambda i: chk(fl.omo_floor_dual(xd[i].data_ptr(), od[i][0].data_ptr(), od[i][1].data_ptr(),
-                                         od[i][2].data_ptr(), od[i][3].data_ptr(), M, K, cur()), "dual floor"),
+         lambda i: chk(fl.omo_floor_dual_grouped(0, *d_ptrs[i], I1(M), I1(K), 1, cur()), "dual floor"),
          max(20, args.steps // 50))
-    for kind, name, what in ((1, "dual_no_scale_stores", "the product's schedule without its scale stores (the bound "
+    for kind, name, what in ((0, "dual_four_tiles", "a four-tile schedule (256-row workgroups, whole column lines) "
+                                                    "in band groups"),
+                             (1, "dual_no_scale_stores", "the four-tile schedule without its scale stores (the bound "
                                                          "of the code traffic; not a valid output)"),
-                             (2, "dual_scales_as_whole_lines", "the product's schedule with each workgroup's 4 KB of "
+                             (2, "dual_scales_as_whole_lines", "the four-tile schedule with each workgroup's 4 KB of "
                                                                "scale bytes stored as whole non-temporal lines "
                                                                "(layout-free bound; not a valid output)"),
-                             (3, "dual_k_fastest", "the product's stores in contiguous K-fastest super-tile "
+                             (3, "dual_k_fastest", "the four-tile schedule in contiguous K-fastest super-tile "
                                                    "ranges per XCD"),
-                             (4, "dual_m_fastest_ranges", "the product's stores in contiguous M-fastest super-tile "
+                             (4, "dual_m_fastest_ranges", "the four-tile schedule in contiguous M-fastest super-tile "
                                                           "ranges per XCD (each XCD finishing a band before the "
                                                           "next)"),
-                             (5, "dual_aligned_groups", "the product's stores with each XCD owning whole 8-band "
+                             (5, "dual_aligned_groups", "the four-tile schedule with each XCD owning whole 8-band "
                                                         "groups (64 B halves of the row-scale lines) and an eighth "
                                                         "of the leftover groups")):
         alt(name, f"dual-layout floor 7168x18432: {what}", wl.dual_quant_bytes(n), 2,
@@ -286,7 +288,7 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
                                                                od[i][1].data_ptr(), od[i][2].data_ptr(),
                                                                od[i][3].data_ptr(), M, K, cur()), "dual variant"),
             max(20, args.steps // 50), "dual")
-    del xd, od
+    del xd, od, d_ptrs
     # the grouped dual-layout quantize of cfg5's 24 expert weights (one-tile pattern)
     c5 = wl.CFG5
     w_shapes = [(c5["hidden"], c5["ffn"]), (c5["hidden"], c5["ffn"]), (c5["ffn"], c5["hidden"])] * c5["local_experts"]

@@ -47,3 +47,25 @@ def test_whole_tiles(oracle, dev, M, K, row_shift, col_shift):
             whole = torch.as_strided(buf, (buf.untyped_storage().nbytes(),), (1,), 0)
             at = buf.storage_offset()
             assert (whole[:at] == 0xAB).all() and (whole[at + buf.numel():] == 0xAB).all()
+
+
+# The orders of the tiles: ranges (few tiles), band groups in units of four
+# tiles with a last row of units of one to four (6 tiles per CU: 1536 tiles),
+# and grouped items of at most and of more than 64 bands side by side.
+@pytest.mark.parametrize("M,K", [(64 * 23, 256 * 67), (64 * 24, 256 * 64), (64 * 25 + 32, 256 * 62 + 32), (64 * 1538, 256)])
+def test_orders(oracle, dev, M, K):
+    import omo
+    print("dual order", M, K, flush=True)
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(K)).to(torch.bfloat16)
+    xd = x.to(dev)
+    outs = _outs(dev, M, K, 0, 0)
+    omo.omo_quant_mxfp4_dual(xd, *outs)
+    small = xd[:160, :].contiguous()
+    grouped = [_outs(dev, 160, K, 0, 0), _outs(dev, M, K, 0, 0), _outs(dev, 160, K, 0, 0)]
+    omo.omo_quant_mxfp4_dual_grouped([small, xd, small], grouped)
+    torch.cuda.synchronize()
+    _check(oracle, x, outs)
+    for a, b in zip(outs, grouped[1]):
+        assert torch.equal(a, b)
+    for o in (grouped[0], grouped[2]):
+        _check(oracle, x[:160], o)
