@@ -226,6 +226,7 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
     import ctypes
     fl = ctypes.CDLL(os.path.join(ROOT, "mxfp4-hopper_amd", "lib", "libomo_ceiling.so"))
     P, I64 = ctypes.c_void_p, ctypes.c_int64
+    fl.omo_floor_dual.argtypes = [P, P, P, P, P, I64, I64, P]
     fl.omo_floor_rowcol.argtypes = [P, P, P, P, I64, I64, P]
     fl.omo_floor_msplit.argtypes = [P, P, P, P, I64, I64, P, P, P, I64, I64, I64, P]
     fl.omo_floor_requant.argtypes = [P, P, P, P, I64, I64, P]
@@ -268,9 +269,12 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
                                                     od[i][3].data_ptr(), n // 32, 1e-10, cur()), "dual"),
          lambda i: chk(fl.omo_floor_dual_grouped(0, *d_ptrs[i], I1(M), I1(K), 1, cur()), "dual floor"),
          max(20, args.steps // 50))
-    for kind, name, what in ((0, "dual_four_tiles", "a four-tile schedule (256-row workgroups, whole column lines) "
-                                                    "in band groups"),
-                             (1, "dual_no_scale_stores", "the four-tile schedule without its scale stores (the bound "
+    alt("dual_four_tiles", "dual-layout floor 7168x18432: a four-tile schedule (256-row workgroups, whole column lines) "
+                           "in band groups", wl.dual_quant_bytes(n), 2,
+        lambda i: chk(fl.omo_floor_dual(xd[i].data_ptr(), od[i][0].data_ptr(), od[i][1].data_ptr(),
+                                        od[i][2].data_ptr(), od[i][3].data_ptr(), M, K, cur()), "dual four tiles"),
+        max(20, args.steps // 50), "dual")
+    for kind, name, what in ((1, "dual_no_scale_stores", "the four-tile schedule without its scale stores (the bound "
                                                          "of the code traffic; not a valid output)"),
                              (2, "dual_scales_as_whole_lines", "the four-tile schedule with each workgroup's 4 KB of "
                                                                "scale bytes stored as whole non-temporal lines "

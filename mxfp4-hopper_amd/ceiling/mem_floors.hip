@@ -574,19 +574,30 @@ int device_lds() {
 
 extern "C" {
 
-// The four-tile schedule of the dual-layout traffic for x [M, K] bf16 (M % 256
-// == 0, K % 256 == 0; outputs as the product's): kind 0 = in band groups, 1 =
+// Four-tile schedule of the dual-layout traffic for x [M, K] bf16 (M % 256 ==
+// 0, K % 256 == 0), in band groups: outputs as the product's (row codes M*K/2,
+// row scales M*K/32, column codes, column scales).
+__attribute__((visibility("default"))) int omo_floor_dual(const void* x, void* row_q, void* row_s, void* col_q,
+                                                          void* col_s, int64_t M, int64_t K, hipStream_t stream) {
+  if (M <= 0 || K <= 0 || M % 256 || K % 256) return -1;
+  const int tiles_ms = (int)(M / 256), tiles = (int)(tiles_ms * (K / 256)), per_xcd = (tiles + 7) / 8;
+  hipLaunchKernelGGL((dual_floor<0, 0>), dim3((unsigned)(per_xcd * 8)), dim3(512), 0, stream,
+                     static_cast<const uint16_t*>(x), static_cast<uint32_t*>(row_q), static_cast<uint8_t*>(row_s),
+                     static_cast<uint8_t*>(col_q), static_cast<uint8_t*>(col_s), M, K, tiles_ms, tiles, per_xcd);
+  return (int)hipGetLastError();
+}
+
+// Variants of the four-tile schedule on the same buffers: kind 1 =
 // no scale stores, 2 = scales as whole non-temporal lines (layout-free
 // bound), 3 = its stores in contiguous K-fastest ranges per XCD,
 // 4 = in contiguous M-fastest ranges per XCD, 5 = in aligned groups (K % 2048 == 0).
 __attribute__((visibility("default"))) int omo_floor_dual_variant(int kind, const void* x, void* row_q, void* row_s,
                                                                   void* col_q, void* col_s, int64_t M, int64_t K,
                                                                   hipStream_t stream) {
-  if (M <= 0 || K <= 0 || M % 256 || K % 256 || kind < 0 || kind > 5) return -1;
+  if (M <= 0 || K <= 0 || M % 256 || K % 256 || kind < 1 || kind > 5) return -1;
   if (kind == 5 && K % 2048) return -1;
   const int tiles_ms = (int)(M / 256), tiles = (int)(tiles_ms * (K / 256)), per_xcd = (tiles + 7) / 8;
-  auto kern = kind == 0   ? dual_floor<0, 0>
-              : kind == 1 ? dual_floor<1, 0>
+  auto kern = kind == 1 ? dual_floor<1, 0>
               : kind == 2 ? dual_floor<2, 0>
               : kind == 3 ? dual_floor<0, 2>
               : kind == 4 ? dual_floor<0, 1>
