@@ -394,53 +394,73 @@ struct RowMap {
   std::vector<int64_t> loads;
 };
 
+// A point of a stream that the host waits for. Pinned memory that a kernel
+// ahead of the point writes stays with its owner until the kernel is done:
+// destroyed with the wait outstanding (an exception, an early return), it waits.
+class HostWait {
+ public:
+  HostWait() { e_ = hipEventCreateWithFlags(&event_, hipEventDisableTiming); }
+  HostWait(const HostWait&) = delete;
+  HostWait& operator=(const HostWait&) = delete;
+  ~HostWait() {
+    if (pending_) (void)hipEventSynchronize(event_);
+    if (event_) (void)hipEventDestroy(event_);
+  }
+  hipError_t created() const { return e_; }
+  // Covers the work enqueued on the stream before the call.
+  hipError_t record(hipStream_t stream) {
+    const hipError_t e = hipEventRecord(event_, stream);
+    if (e == hipSuccess) pending_ = true;
+    else (void)hipStreamSynchronize(stream);
+    return e;
+  }
+  hipError_t wait() {
+    pending_ = false;
+    return hipEventSynchronize(event_);
+  }
+
+ private:
+  hipEvent_t event_ = nullptr;
+  hipError_t e_;
+  bool pending_ = false;
+};
+
 // num_out: rows asked for, or -1. `ahead`: the order is enqueued before the
 // host waits for the loads, so that nothing is left to do after the wait; with
 // num_out < 0 its length is not known then and src is scratch for every pair.
+// Everything whose size is known is allocated before the first launch.
 // False: a Python error is set.
 bool row_map(const Tensor& map, int64_t num_out, bool want_dest, bool ahead, RowMap* r) {
   const int64_t T = map.size(0), E = map.size(1), chunks = omo_hip_route_chunks(T, E);
   const hipStream_t stream = stream_of(map);
+  const auto hip_ok = [](hipError_t e) {
+    if (e != hipSuccess) PyErr_Format(PyExc_RuntimeError, "omo_route_counts: %s", hipGetErrorString(e));
+    return e == hipSuccess;
+  };
   const Tensor counts = empty_like_device(map, {E * chunks}, at::kInt);
   // The counts also go to pinned host memory, so that the host waits for the
   // counting launch alone and no copy follows it.
   const Tensor seen = at::empty({E * chunks}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  if (want_dest) r->dest = empty_like_device(map, {T, E}, at::kInt);
+  if (ahead) r->src = empty_like_device(map, {num_out < 0 ? T * E : num_out}, at::kInt);
+  HostWait counted;
+  if (!hip_ok(counted.created())) return false;
   if (!ok(omo_hip_route_counts(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks, seen.data_ptr<int32_t>(),
-                               stream)))
+                               stream)) ||
+      !hip_ok(counted.record(stream)))
     return false;
-  auto order = [&](int64_t rows, bool pad) {
-    r->src = empty_like_device(map, {rows}, at::kInt);
-    if (want_dest) r->dest = empty_like_device(map, {T, E}, at::kInt);
+  const auto order = [&](bool pad) {
+    const int64_t rows = r->src.numel();
     return ok(omo_hip_route_rows(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
                                  rows ? r->src.data_ptr<int32_t>() : nullptr, rows, pad,
                                  want_dest ? r->dest.data_ptr<int32_t>() : nullptr, want_dest ? T * E : 0, stream));
   };
+  if (ahead && !order(num_out >= 0)) return false;
   hipError_t e;
-  if (ahead) {
-    hipEvent_t counted;
-    e = hipEventCreateWithFlags(&counted, hipEventDisableTiming);
-    if (e == hipSuccess) {
-      e = hipEventRecord(counted, stream);
-      if (e == hipSuccess && !order(num_out < 0 ? T * E : num_out, num_out >= 0)) {
-        (void)hipEventDestroy(counted);
-        return false;
-      }
-      if (e == hipSuccess) {
-        Py_BEGIN_ALLOW_THREADS
-        e = hipEventSynchronize(counted);
-        Py_END_ALLOW_THREADS
-      }
-      (void)hipEventDestroy(counted);
-    }
-  } else {
-    Py_BEGIN_ALLOW_THREADS
-    e = hipStreamSynchronize(stream);
-    Py_END_ALLOW_THREADS
-  }
-  if (e != hipSuccess) {
-    PyErr_Format(PyExc_RuntimeError, "omo_route_counts: %s", hipGetErrorString(e));
-    return false;
-  }
+  Py_BEGIN_ALLOW_THREADS
+  e = counted.wait();
+  Py_END_ALLOW_THREADS
+  if (!hip_ok(e)) return false;
   const int32_t* c = seen.data_ptr<int32_t>();
   int64_t routed = 0;
   r->loads.assign((size_t)E, 0);
@@ -454,7 +474,9 @@ bool row_map(const Tensor& map, int64_t num_out, bool want_dest, bool ahead, Row
     return false;
   }
   r->rows = num_out < 0 ? routed : num_out;
-  return ahead || order(r->rows, num_out > routed);
+  if (ahead) return true;
+  r->src = empty_like_device(map, {r->rows}, at::kInt);
+  return order(num_out > routed);
 }
 
 const Tensor* plain_map(PyObject* o) {

@@ -208,3 +208,36 @@ def test_side_stream_and_threads(dev):
     for t in ts:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("num_out", [None, 1 << 24])
+def test_refused_row_order_leaves_pinned_memory_alone(dev, num_out):
+    """A permute whose row order (64 MB here) does not fit the device raises
+    out of memory; no launch of it writes host memory afterwards, which the
+    next pinned tensor of the counts' size would show, and the next call is
+    right."""
+    from omo_python_api.permutation import mxfp4_permute_to_fp8
+    T, E, chunks = 16384, 1024, 8
+    print("refused row order", num_out, flush=True)
+    q, s = _u8(dev, 0, 256, T, 64), _u8(dev, 120, 131, T, 4)
+    rm = torch.zeros((T, E), dtype=torch.bool, device=dev)
+    rm[::7, 5] = True
+    want = mxfp4_permute_to_fp8(q, s, rm, split=False)
+    want = [t.cpu() for t in want[:3]] + [want[3]]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (40 << 20)) / total)
+    try:
+        torch.cuda._sleep(50 * 2_400_000)  # what the call enqueues starts after the host is done below
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            mxfp4_permute_to_fp8(q, s, rm, num_out, split=False)
+        next_pinned = torch.empty((E * chunks,), dtype=torch.int32, pin_memory=True).fill_(-7)
+        torch.cuda.synchronize()
+        assert (next_pinned == -7).all()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    got = mxfp4_permute_to_fp8(q, s, rm, split=False)
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a.cpu().view(torch.uint8), b.view(torch.uint8))
+    assert got[3] == want[3]
