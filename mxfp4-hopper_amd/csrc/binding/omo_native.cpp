@@ -51,19 +51,22 @@ bool quiet() {
          !c10::impl::tls_local_dispatch_key_set().included_.has_any(kUnusual);
 }
 
-// The tensor behind o if it is a plain strided GPU tensor of this dtype, else null.
-const Tensor* plain(PyObject* o, at::ScalarType dtype) {
-  if (!THPVariable_CheckExact(o)) return nullptr;
+// The tensor behind o if it is a plain strided GPU tensor of this dtype, else
+// an undefined one. Held by value: what runs without the GIL keeps its inputs
+// whatever other threads do to o.
+Tensor plain(PyObject* o, at::ScalarType dtype) {
+  if (!THPVariable_CheckExact(o)) return {};
   const Tensor& t = THPVariable_Unpack(o);
   if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.scalar_type() != dtype ||
       t.key_set().has_any(kUnusual))
-    return nullptr;
-  return &t;
+    return {};
+  return t;
 }
 
-const Tensor* plain_matrix(PyObject* o, at::ScalarType dtype) {
-  const Tensor* t = plain(o, dtype);
-  return t && t->dim() == 2 && t->size(0) > 0 && t->size(1) > 0 && t->is_contiguous() ? t : nullptr;
+Tensor plain_matrix(PyObject* o, at::ScalarType dtype) {
+  Tensor t = plain(o, dtype);
+  if (t.defined() && (t.dim() != 2 || t.size(0) == 0 || t.size(1) == 0 || !t.is_contiguous())) t.reset();
+  return t;
 }
 
 bool aligned(const Tensor& t, uintptr_t a) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & (a - 1)) == 0; }
@@ -82,6 +85,20 @@ bool ok(int status) {
 }
 
 PyObject* none() { Py_RETURN_NONE; }
+
+// f() with the GIL released: allocation may free cached memory and wait for
+// the device, and a launch waits while its queue is full; other threads of the
+// program run meanwhile, as they do under torch.empty and ctypes. f calls no
+// Python. Releasing and taking it back adds at most 0.1 us to a call (quantize
+// of 16 x 7168, enqueued: 4.9 us before, 5.0 after).
+template <typename F>
+auto unlocked(F&& f) {
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f();
+}
 
 // A new tuple or list of tensors (steals nothing).
 PyObject* tuple_of(const std::vector<Tensor>& ts) {
@@ -165,24 +182,27 @@ bool arguments(const char* name, Py_ssize_t got, Py_ssize_t want) {
 PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("quantize", n, 1)) return nullptr;
-  const Tensor* x = plain_matrix(a[0], at::kBFloat16);
-  if (!x || x->size(1) % 32 != 0 || !aligned(*x, 16) || !quiet()) return none();
-  const int64_t M = x->size(0), K = x->size(1);
-  const c10::DeviceGuard guard(x->device());
-  Tensor q = empty_like_device(*x, {M, K / 2}, at::kByte), s = empty_like_device(*x, {M, K / 32}, at::kByte);
-  if (!ok(omo_hip_per_token_group_quant_fp4(x->data_ptr(), M * K, q.data_ptr(), M * K / 2, s.data_ptr(), M * K / 32, 32,
-                                            kEps, -6.0f, 6.0f, 0, stream_of(*x))))
+  const Tensor x = plain_matrix(a[0], at::kBFloat16);
+  if (!x.defined() || x.size(1) % 32 != 0 || !aligned(x, 16) || !quiet()) return none();
+  const int64_t M = x.size(0), K = x.size(1);
+  const c10::DeviceGuard guard(x.device());
+  Tensor q, s;
+  if (!ok(unlocked([&] {
+        q = empty_like_device(x, {M, K / 2}, at::kByte);
+        s = empty_like_device(x, {M, K / 32}, at::kByte);
+        return omo_hip_per_token_group_quant_fp4(x.data_ptr(), M * K, q.data_ptr(), M * K / 2, s.data_ptr(), M * K / 32,
+                                                 32, kEps, -6.0f, 6.0f, 0, stream_of(x));
+      })))
     return nullptr;
   return pair_of(THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(s)));
   END_HANDLE_TH_ERRORS
 }
 
-bool dual_takes(const Tensor* x) {
-  return x && x->size(0) % 32 == 0 && x->size(1) % 32 == 0 && aligned(*x, 16);
+bool dual_takes(const Tensor& x) {
+  return x.defined() && x.size(0) % 32 == 0 && x.size(1) % 32 == 0 && aligned(x, 16);
 }
 
-std::vector<Tensor> dual_outputs(const Tensor& x) {
-  const int64_t M = x.size(0), K = x.size(1);
+std::vector<Tensor> dual_outputs(const Tensor& x, int64_t M, int64_t K) {
   std::vector<Tensor> o;
   o.reserve(4);
   o.push_back(empty_like_device(x, {M, K / 2}, at::kByte));
@@ -197,13 +217,16 @@ PyObject* quantize_dual(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("quantize_dual", n, 2)) return nullptr;
   float eps;
-  const Tensor* x = plain_matrix(a[0], at::kBFloat16);
+  const Tensor x = plain_matrix(a[0], at::kBFloat16);
   if (!dual_takes(x) || !eps_of(a[1], &eps) || !quiet()) return none();
-  const int64_t N = x->numel();
-  const c10::DeviceGuard guard(x->device());
-  const std::vector<Tensor> o = dual_outputs(*x);
-  if (!ok(omo_hip_quant_mxfp4_dual(x->data_ptr(), x->size(0), x->size(1), o[0].data_ptr(), N / 2, o[1].data_ptr(),
-                                   N / 32, o[2].data_ptr(), N / 2, o[3].data_ptr(), N / 32, eps, stream_of(*x))))
+  const int64_t M = x.size(0), K = x.size(1), N = M * K;
+  const c10::DeviceGuard guard(x.device());
+  std::vector<Tensor> o;
+  if (!ok(unlocked([&] {
+        o = dual_outputs(x, M, K);
+        return omo_hip_quant_mxfp4_dual(x.data_ptr(), M, K, o[0].data_ptr(), N / 2, o[1].data_ptr(), N / 32,
+                                        o[2].data_ptr(), N / 2, o[3].data_ptr(), N / 32, eps, stream_of(x));
+      })))
     return nullptr;
   return tuple_of(o);
   END_HANDLE_TH_ERRORS
@@ -219,25 +242,27 @@ PyObject* quantize_dual_grouped(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Py_ssize_t count = list ? PyList_GET_SIZE(a[0]) : PyTuple_GET_SIZE(a[0]);
   if (count == 0) return none();
   std::vector<Tensor> xs;
+  std::vector<omo_dual_item> items;
   xs.reserve((size_t)count);
+  items.reserve((size_t)count);
   for (Py_ssize_t i = 0; i < count; i++) {
-    const Tensor* x = plain_matrix(list ? PyList_GET_ITEM(a[0], i) : PyTuple_GET_ITEM(a[0], i), at::kBFloat16);
-    if (!dual_takes(x) || (i > 0 && x->device() != xs[0].device())) return none();
-    xs.push_back(*x);
+    Tensor x = plain_matrix(list ? PyList_GET_ITEM(a[0], i) : PyTuple_GET_ITEM(a[0], i), at::kBFloat16);
+    if (!dual_takes(x) || (i > 0 && x.device() != xs[0].device())) return none();
+    items.push_back({nullptr, x.size(0), x.size(1), nullptr, 0, nullptr, 0, nullptr, 0, nullptr, 0});
+    xs.push_back(std::move(x));
   }
   const c10::DeviceGuard guard(xs[0].device());
-  std::vector<std::vector<Tensor>> outs;
-  std::vector<omo_dual_item> items;
-  outs.reserve(xs.size());
-  items.reserve(xs.size());
-  for (const Tensor& x : xs) {
-    outs.push_back(dual_outputs(x));
-    const std::vector<Tensor>& o = outs.back();
-    const int64_t N = x.numel();
-    items.push_back({x.data_ptr(), x.size(0), x.size(1), o[0].data_ptr(), N / 2, o[1].data_ptr(), N / 32,
-                     o[2].data_ptr(), N / 2, o[3].data_ptr(), N / 32});
-  }
-  if (!ok(omo_hip_quant_mxfp4_dual_grouped(items.data(), (int64_t)items.size(), eps, stream_of(xs[0])))) return nullptr;
+  std::vector<std::vector<Tensor>> outs(xs.size());
+  if (!ok(unlocked([&] {
+        for (size_t i = 0; i < xs.size(); i++) {
+          const int64_t M = items[i].rows, K = items[i].cols, N = M * K;
+          const std::vector<Tensor>& o = outs[i] = dual_outputs(xs[i], M, K);
+          items[i] = {xs[i].data_ptr(), M, K, o[0].data_ptr(), N / 2, o[1].data_ptr(), N / 32,
+                      o[2].data_ptr(), N / 2, o[3].data_ptr(), N / 32};
+        }
+        return omo_hip_quant_mxfp4_dual_grouped(items.data(), (int64_t)items.size(), eps, stream_of(xs[0]));
+      })))
+    return nullptr;
   PyObject* r = PyList_New(count);
   if (!r) return nullptr;
   for (Py_ssize_t i = 0; i < count; i++) {
@@ -257,19 +282,21 @@ PyObject* quantize_dual_grouped(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("dequantize", n, 3)) return nullptr;
-  const Tensor* x = plain_matrix(a[0], at::kByte);
-  const Tensor* s = plain(a[1], at::kByte);
-  if (!x || !s || !THPDtype_Check(a[2])) return none();
+  const Tensor x = plain_matrix(a[0], at::kByte), s = plain(a[1], at::kByte);
+  if (!x.defined() || !s.defined() || !THPDtype_Check(a[2])) return none();
   const at::ScalarType dtype = reinterpret_cast<THPDtype*>(a[2])->scalar_type;
   const int type = dtype == at::kBFloat16 ? OMO_BF16 : dtype == at::kHalf ? OMO_F16 : dtype == at::kFloat ? OMO_F32 : -1;
-  const int64_t M = x->size(0), half = x->size(1);
-  if (type < 0 || half % 32 != 0 || M * half % 128 != 0 || !s->is_contiguous() || s->numel() < M * half / 16 ||
-      s->device() != x->device() || !aligned(*x, 4) || !quiet())
+  const int64_t M = x.size(0), half = x.size(1), scales = s.numel();
+  if (type < 0 || half % 32 != 0 || M * half % 128 != 0 || !s.is_contiguous() || scales < M * half / 16 ||
+      s.device() != x.device() || !aligned(x, 4) || !quiet())
     return none();
-  const c10::DeviceGuard guard(x->device());
-  Tensor y = empty_like_device(*x, {M, 2 * half}, dtype);
-  if (!ok(omo_hip_Mxfp4_dequant(x->data_ptr(), M * half, s->data_ptr(), s->numel(), y.data_ptr(), y.numel(), type,
-                                stream_of(*x))))
+  const c10::DeviceGuard guard(x.device());
+  Tensor y;
+  if (!ok(unlocked([&] {
+        y = empty_like_device(x, {M, 2 * half}, dtype);
+        return omo_hip_Mxfp4_dequant(x.data_ptr(), M * half, s.data_ptr(), scales, y.data_ptr(), 2 * M * half, type,
+                                     stream_of(x));
+      })))
     return nullptr;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
@@ -284,17 +311,21 @@ PyObject* split_pair(const Tensor& q, const Tensor& s, const std::vector<int64_t
 PyObject* requant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("requant", n, 3)) return nullptr;
-  const Tensor *x = plain_matrix(a[0], at::kByte), *s = plain_matrix(a[1], at::kByte);
-  if (!x || !s || x->device() != s->device()) return none();
-  const int64_t M = x->size(0), half = x->size(1), groups = (half + 63) / 64;
+  const Tensor x = plain_matrix(a[0], at::kByte), s = plain_matrix(a[1], at::kByte);
+  if (!x.defined() || !s.defined() || x.device() != s.device()) return none();
+  const int64_t M = x.size(0), half = x.size(1), groups = (half + 63) / 64;
   std::vector<int64_t> lens;
-  if (half % 16 != 0 || s->size(0) != M || s->size(1) != half / 16 || M * groups % 2 != 0 || !aligned(*x, 8) ||
-      (half % 64 == 0 && !aligned(*s, 4)) || !splits_of(a[2], M, &lens) || !quiet())
+  if (half % 16 != 0 || s.size(0) != M || s.size(1) != half / 16 || M * groups % 2 != 0 || !aligned(x, 8) ||
+      (half % 64 == 0 && !aligned(s, 4)) || !splits_of(a[2], M, &lens) || !quiet())
     return none();
-  const c10::DeviceGuard guard(x->device());
-  Tensor q = empty_like_device(*x, {M, groups * 128}, kFp8), qs = empty_like_device(*x, {groups, M}, at::kFloat);
-  if (!ok(omo_hip_Mxfp4ToFp8_padded(x->data_ptr(), M, half, s->data_ptr(), s->numel(), q.data_ptr(), q.numel(),
-                                    qs.data_ptr(), qs.numel(), stream_of(*x))))
+  const c10::DeviceGuard guard(x.device());
+  Tensor q, qs;
+  if (!ok(unlocked([&] {
+        q = empty_like_device(x, {M, groups * 128}, kFp8);
+        qs = empty_like_device(x, {groups, M}, at::kFloat);
+        return omo_hip_Mxfp4ToFp8_padded(x.data_ptr(), M, half, s.data_ptr(), M * (half / 16), q.data_ptr(),
+                                         M * groups * 128, qs.data_ptr(), groups * M, stream_of(x));
+      })))
     return nullptr;
   return split_pair(half % 64 == 0 ? q : q.narrow(1, 0, 2 * half), qs, lens);
   END_HANDLE_TH_ERRORS
@@ -306,14 +337,18 @@ PyObject* row_to_col(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("row_to_col", n, 3)) return nullptr;
   float eps;
-  const Tensor *x = plain_matrix(a[0], at::kByte), *s = plain_matrix(a[1], at::kByte);
-  if (!x || !s || x->device() != s->device() || !eps_of(a[2], &eps)) return none();
-  const int64_t M = x->size(0), N = 2 * x->size(1), tiles = (M + 127) / 128;
-  if (s->size(0) != M || s->size(1) != (N + 31) / 32 || !quiet()) return none();
-  const c10::DeviceGuard guard(x->device());
-  Tensor q = empty_like_device(*x, {N, M}, kFp8), qs = empty_like_device(*x, {tiles, N}, at::kFloat);
-  if (!ok(omo_hip_per_token_Mxfp4RowToBf16ToFp8Col(x->data_ptr(), M, N / 2, s->data_ptr(), M, s->size(1), q.data_ptr(),
-                                                   N, M, qs.data_ptr(), tiles, N, eps, stream_of(*x))))
+  const Tensor x = plain_matrix(a[0], at::kByte), s = plain_matrix(a[1], at::kByte);
+  if (!x.defined() || !s.defined() || x.device() != s.device() || !eps_of(a[2], &eps)) return none();
+  const int64_t M = x.size(0), N = 2 * x.size(1), blocks = (N + 31) / 32, tiles = (M + 127) / 128;
+  if (s.size(0) != M || s.size(1) != blocks || !quiet()) return none();
+  const c10::DeviceGuard guard(x.device());
+  Tensor q, qs;
+  if (!ok(unlocked([&] {
+        q = empty_like_device(x, {N, M}, kFp8);
+        qs = empty_like_device(x, {tiles, N}, at::kFloat);
+        return omo_hip_per_token_Mxfp4RowToBf16ToFp8Col(x.data_ptr(), M, N / 2, s.data_ptr(), M, blocks, q.data_ptr(), N,
+                                                        M, qs.data_ptr(), tiles, N, eps, stream_of(x));
+      })))
     return nullptr;
   return pair_of(THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(qs)));
   END_HANDLE_TH_ERRORS
@@ -324,21 +359,26 @@ PyObject* row_to_col_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("row_to_col_splits", n, 4)) return nullptr;
   float eps;
-  const Tensor *x = plain_matrix(a[0], at::kByte), *s = plain(a[1], at::kByte);
-  if (!x || !s || x->device() != s->device() || !s->is_contiguous() || !eps_of(a[3], &eps)) return none();
-  const int64_t M = x->size(0), N = 2 * x->size(1);
+  const Tensor x = plain_matrix(a[0], at::kByte), s = plain(a[1], at::kByte);
+  if (!x.defined() || !s.defined() || x.device() != s.device() || !s.is_contiguous() || !eps_of(a[3], &eps))
+    return none();
+  const int64_t M = x.size(0), N = 2 * x.size(1), scales = s.numel();
   std::vector<int64_t> lens;
-  if (!splits_of(a[2], M, &lens) || lens.size() > 128 || N % 32 != 0 || M >= ((int64_t)1 << 31) || !aligned(*x, 16) ||
-      s->numel() < M * (N / 32) || !quiet())
+  if (!splits_of(a[2], M, &lens) || lens.size() > 128 || N % 32 != 0 || M >= ((int64_t)1 << 31) || !aligned(x, 16) ||
+      scales < M * (N / 32) || !quiet())
     return none();
   std::vector<int64_t> tiles(lens.size());
   int64_t rows = 0;
   for (size_t i = 0; i < lens.size(); i++) rows += tiles[i] = (lens[i] + 127) / 128;
-  const c10::DeviceGuard guard(x->device());
-  const Tensor q = empty_like_device(*x, {M * N}, kFp8), qs = empty_like_device(*x, {rows, N}, at::kFloat);
-  if (!ok(omo_hip_Mxfp4RowToBf16ToFp8Col_splits(x->data_ptr(), M, N / 2, s->data_ptr(), s->numel(), q.data_ptr(),
-                                                q.numel(), qs.data_ptr(), qs.numel(), lens.data(),
-                                                (int64_t)lens.size(), eps, stream_of(*x))))
+  const c10::DeviceGuard guard(x.device());
+  Tensor q, qs;
+  if (!ok(unlocked([&] {
+        q = empty_like_device(x, {M * N}, kFp8);
+        qs = empty_like_device(x, {rows, N}, at::kFloat);
+        return omo_hip_Mxfp4RowToBf16ToFp8Col_splits(x.data_ptr(), M, N / 2, s.data_ptr(), scales, q.data_ptr(), M * N,
+                                                     qs.data_ptr(), rows * N, lens.data(), (int64_t)lens.size(), eps,
+                                                     stream_of(x));
+      })))
     return nullptr;
   std::vector<Tensor> blocks;
   blocks.reserve(lens.size());
@@ -357,12 +397,15 @@ PyObject* quantize_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("quantize_packed", n, 2)) return nullptr;
   float eps;
-  const Tensor* x = plain_matrix(a[0], at::kBFloat16);
-  if (!x || x->size(1) % 128 != 0 || !aligned(*x, 16) || !eps_of(a[1], &eps) || !quiet()) return none();
-  const int64_t T = x->size(0), H = x->size(1);
-  const c10::DeviceGuard guard(x->device());
-  Tensor out = empty_like_device(*x, {T, H / 32 * 17}, at::kByte);
-  if (!ok(omo_hip_quant_mxfp4_packed(x->data_ptr(), T, H, out.data_ptr(), out.numel(), eps, stream_of(*x))))
+  const Tensor x = plain_matrix(a[0], at::kBFloat16);
+  if (!x.defined() || x.size(1) % 128 != 0 || !aligned(x, 16) || !eps_of(a[1], &eps) || !quiet()) return none();
+  const int64_t T = x.size(0), H = x.size(1);
+  const c10::DeviceGuard guard(x.device());
+  Tensor out;
+  if (!ok(unlocked([&] {
+        out = empty_like_device(x, {T, H / 32 * 17}, at::kByte);
+        return omo_hip_quant_mxfp4_packed(x.data_ptr(), T, H, out.data_ptr(), out.numel(), eps, stream_of(x));
+      })))
     return nullptr;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -372,15 +415,19 @@ PyObject* quantize_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* requant_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("requant_packed", n, 2)) return nullptr;
-  const Tensor* p = plain_matrix(a[0], at::kByte);
-  if (!p || p->size(1) % (17 * 4) != 0 || !aligned(*p, 4)) return none();
-  const int64_t T = p->size(0), H = p->size(1) / 17 * 32;
+  const Tensor p = plain_matrix(a[0], at::kByte);
+  if (!p.defined() || p.size(1) % (17 * 4) != 0 || !aligned(p, 4)) return none();
+  const int64_t T = p.size(0), H = p.size(1) / 17 * 32;
   std::vector<int64_t> lens;
   if ((a[1] != Py_None && !splits_of(a[1], T, &lens)) || !quiet()) return none();
-  const c10::DeviceGuard guard(p->device());
-  Tensor q = empty_like_device(*p, {T, H}, kFp8), s = empty_like_device(*p, {H / 128, T}, at::kFloat);
-  if (!ok(omo_hip_packed_Mxfp4ToFp8(p->data_ptr(), T, H, q.data_ptr(), q.numel(), s.data_ptr(), s.numel(),
-                                    stream_of(*p))))
+  const c10::DeviceGuard guard(p.device());
+  Tensor q, s;
+  if (!ok(unlocked([&] {
+        q = empty_like_device(p, {T, H}, kFp8);
+        s = empty_like_device(p, {H / 128, T}, at::kFloat);
+        return omo_hip_packed_Mxfp4ToFp8(p.data_ptr(), T, H, q.data_ptr(), q.numel(), s.data_ptr(), s.numel(),
+                                         stream_of(p));
+      })))
     return nullptr;
   if (a[1] != Py_None) return split_pair(q, s, lens);
   return pair_of(THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(s)));
@@ -392,7 +439,26 @@ struct RowMap {
   Tensor src, dest;            // src: the row order, `rows` entries at its head
   int64_t rows = 0;
   std::vector<int64_t> loads;
+  // what the call ended with: a status of the C ABI, a HIP error, or (wanted
+  // >= 0) fewer rows wanted than the `rows` routed
+  int status = OMO_OK;
+  hipError_t hip = hipSuccess;
+  int64_t wanted = -1;
 };
+
+// Raises the Python error of a row map that ended with one.
+bool ok(const RowMap& r) {
+  if (r.hip != hipSuccess) {
+    PyErr_Format(PyExc_RuntimeError, "omo_route_counts: %s", hipGetErrorString(r.hip));
+    return false;
+  }
+  if (r.wanted >= 0) {
+    PyErr_Format(PyExc_ValueError, "num_out_tokens=%lld is smaller than the %lld routed tokens", (long long)r.wanted,
+                 (long long)r.rows);
+    return false;
+  }
+  return ok(r.status);
+}
 
 // A point of a stream that the host waits for. Pinned memory that a kernel
 // ahead of the point writes stays with its owner until the kernel is done:
@@ -428,60 +494,52 @@ class HostWait {
 // num_out: rows asked for, or -1. `ahead`: the order is enqueued before the
 // host waits for the loads, so that nothing is left to do after the wait; with
 // num_out < 0 its length is not known then and src is scratch for every pair.
-// Everything whose size is known is allocated before the first launch.
-// False: a Python error is set.
-bool row_map(const Tensor& map, int64_t num_out, bool want_dest, bool ahead, RowMap* r) {
-  const int64_t T = map.size(0), E = map.size(1), chunks = omo_hip_route_chunks(T, E);
+// Everything whose size is known is allocated before the first launch. Runs
+// without the GIL.
+RowMap row_map(const Tensor& map, int64_t T, int64_t E, int64_t num_out, bool want_dest, bool ahead) {
+  RowMap r;
+  const int64_t chunks = omo_hip_route_chunks(T, E);
   const hipStream_t stream = stream_of(map);
-  const auto hip_ok = [](hipError_t e) {
-    if (e != hipSuccess) PyErr_Format(PyExc_RuntimeError, "omo_route_counts: %s", hipGetErrorString(e));
-    return e == hipSuccess;
-  };
   const Tensor counts = empty_like_device(map, {E * chunks}, at::kInt);
   // The counts also go to pinned host memory, so that the host waits for the
   // counting launch alone and no copy follows it.
   const Tensor seen = at::empty({E * chunks}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  if (want_dest) r->dest = empty_like_device(map, {T, E}, at::kInt);
-  if (ahead) r->src = empty_like_device(map, {num_out < 0 ? T * E : num_out}, at::kInt);
+  if (want_dest) r.dest = empty_like_device(map, {T, E}, at::kInt);
+  if (ahead) r.src = empty_like_device(map, {num_out < 0 ? T * E : num_out}, at::kInt);
   HostWait counted;
-  if (!hip_ok(counted.created())) return false;
-  if (!ok(omo_hip_route_counts(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks, seen.data_ptr<int32_t>(),
-                               stream)) ||
-      !hip_ok(counted.record(stream)))
-    return false;
+  if ((r.hip = counted.created()) != hipSuccess) return r;
+  r.status = omo_hip_route_counts(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
+                                  seen.data_ptr<int32_t>(), stream);
+  if (r.status != OMO_OK || (r.hip = counted.record(stream)) != hipSuccess) return r;
   const auto order = [&](bool pad) {
-    const int64_t rows = r->src.numel();
-    return ok(omo_hip_route_rows(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
-                                 rows ? r->src.data_ptr<int32_t>() : nullptr, rows, pad,
-                                 want_dest ? r->dest.data_ptr<int32_t>() : nullptr, want_dest ? T * E : 0, stream));
+    const int64_t rows = r.src.numel();
+    r.status = omo_hip_route_rows(map.data_ptr(), T, E, counts.data_ptr<int32_t>(), E * chunks,
+                                  rows ? r.src.data_ptr<int32_t>() : nullptr, rows, pad,
+                                  want_dest ? r.dest.data_ptr<int32_t>() : nullptr, want_dest ? T * E : 0, stream);
   };
-  if (ahead && !order(num_out >= 0)) return false;
-  hipError_t e;
-  Py_BEGIN_ALLOW_THREADS
-  e = counted.wait();
-  Py_END_ALLOW_THREADS
-  if (!hip_ok(e)) return false;
+  if (ahead) order(num_out >= 0);
+  if (r.status != OMO_OK || (r.hip = counted.wait()) != hipSuccess) return r;
   const int32_t* c = seen.data_ptr<int32_t>();
   int64_t routed = 0;
-  r->loads.assign((size_t)E, 0);
+  r.loads.assign((size_t)E, 0);
   for (int64_t i = 0; i < E; i++) {
-    for (int64_t k = 0; k < chunks; k++) r->loads[(size_t)i] += c[i * chunks + k];
-    routed += r->loads[(size_t)i];
+    for (int64_t k = 0; k < chunks; k++) r.loads[(size_t)i] += c[i * chunks + k];
+    routed += r.loads[(size_t)i];
   }
+  r.rows = num_out < 0 || num_out < routed ? routed : num_out;
   if (num_out >= 0 && num_out < routed) {
-    PyErr_Format(PyExc_ValueError, "num_out_tokens=%lld is smaller than the %lld routed tokens", (long long)num_out,
-                 (long long)routed);
-    return false;
+    r.wanted = num_out;
+  } else if (!ahead) {
+    r.src = empty_like_device(map, {r.rows}, at::kInt);
+    order(num_out > routed);
   }
-  r->rows = num_out < 0 ? routed : num_out;
-  if (ahead) return true;
-  r->src = empty_like_device(map, {r->rows}, at::kInt);
-  return order(num_out > routed);
+  return r;
 }
 
-const Tensor* plain_map(PyObject* o) {
-  const Tensor* t = plain_matrix(o, at::kBool);
-  return t && t->size(0) < ((int64_t)1 << 31) / t->size(1) && t->size(1) <= 4 * 65534 ? t : nullptr;
+Tensor plain_map(PyObject* o) {
+  Tensor t = plain_matrix(o, at::kBool);
+  if (t.defined() && (t.size(0) >= ((int64_t)1 << 31) / t.size(1) || t.size(1) > 4 * 65534)) t.reset();
+  return t;
 }
 
 // None (-1) or a Python int in [0, 2^31).
@@ -513,11 +571,12 @@ PyObject* make_row_map(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("make_row_map", n, 2)) return nullptr;
   int64_t num_out;
-  const Tensor* map = plain_map(a[0]);
-  if (!map || !num_out_of(a[1], &num_out) || !quiet()) return none();
-  const c10::DeviceGuard guard(map->device());
-  RowMap m;
-  if (!row_map(*map, num_out, true, false, &m)) return nullptr;
+  const Tensor map = plain_map(a[0]);
+  if (!map.defined() || !num_out_of(a[1], &num_out) || !quiet()) return none();
+  const int64_t T = map.size(0), E = map.size(1);
+  const c10::DeviceGuard guard(map.device());
+  RowMap m = unlocked([&] { return row_map(map, T, E, num_out, true, false); });
+  if (!ok(m)) return nullptr;
   PyObject* loads = list_of_ints(m.loads);
   PyObject* rest = pair_of(loads, THPVariable_Wrap(std::move(m.dest)));
   PyObject* head = rest ? THPVariable_Wrap(std::move(m.src)) : nullptr;
@@ -541,29 +600,35 @@ PyObject* permute_to_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (!arguments("permute_to_fp8", n, 4)) return nullptr;
   int64_t num_out, cspan, cstride, sspan, sstride;
-  const Tensor *codes = plain(a[0], at::kByte), *scales = plain(a[1], at::kByte), *map = plain_map(a[2]);
-  if (!codes || !scales || !map || !num_out_of(a[3], &num_out) || !rows_of(*codes, &cspan, &cstride) ||
-      !rows_of(*scales, &sspan, &sstride))
+  const Tensor codes = plain(a[0], at::kByte), scales = plain(a[1], at::kByte), map = plain_map(a[2]);
+  if (!codes.defined() || !scales.defined() || !map.defined() || !num_out_of(a[3], &num_out) ||
+      !rows_of(codes, &cspan, &cstride) || !rows_of(scales, &sspan, &sstride))
     return none();
-  const int64_t T = codes->size(0), H = 2 * codes->size(1);
-  if (scales->size(0) != T || H % 128 != 0 || scales->size(1) != H / 32 || cstride < H / 2 || sstride < H / 32 ||
-      cstride % 4 != 0 || sstride % 4 != 0 || !aligned(*codes, 4) || !aligned(*scales, 4) ||
-      codes->device() != map->device() || scales->device() != map->device() || !quiet())
+  const int64_t T = codes.size(0), H = 2 * codes.size(1), map_T = map.size(0), E = map.size(1);
+  if (scales.size(0) != T || H % 128 != 0 || scales.size(1) != H / 32 || cstride < H / 2 || sstride < H / 32 ||
+      cstride % 4 != 0 || sstride % 4 != 0 || !aligned(codes, 4) || !aligned(scales, 4) ||
+      codes.device() != map.device() || scales.device() != map.device() || !quiet())
     return none();
-  const c10::DeviceGuard guard(map->device());
+  const c10::DeviceGuard guard(map.device());
   RowMap m;
-  // The order goes ahead of the wait; the requant, which has to know the
-  // number of rows, copies it from the scratch to its own buffer.
-  if (!row_map(*map, num_out, false, true, &m)) return nullptr;
-  const int64_t N = m.rows;
-  const bool scratch = m.src.numel() != N;
-  const Tensor src = scratch ? empty_like_device(*codes, {N}, at::kInt) : m.src;
-  const Tensor q = empty_like_device(*codes, {N, H}, kFp8), s = empty_like_device(*codes, {H / 128, N}, at::kFloat);
-  if (N > 0 && !ok(omo_hip_permute_Mxfp4ToFp8_copy(
-                   codes->data_ptr(), cspan, cstride, scales->data_ptr(), sspan, sstride, T, H,
-                   m.src.data_ptr<int32_t>(), N, scratch ? src.data_ptr<int32_t>() : nullptr, q.data_ptr(), q.numel(),
-                   s.data_ptr(), s.numel(), stream_of(*codes))))
-    return nullptr;
+  Tensor src, q, s;
+  const int status = unlocked([&]() -> int {
+    // The order goes ahead of the wait; the requant, which has to know the
+    // number of rows, copies it from the scratch to its own buffer.
+    m = row_map(map, map_T, E, num_out, false, true);
+    if (m.status != OMO_OK || m.hip != hipSuccess || m.wanted >= 0) return OMO_OK;  // raised below
+    const int64_t N = m.rows;
+    const bool scratch = m.src.numel() != N;
+    src = scratch ? empty_like_device(codes, {N}, at::kInt) : m.src;
+    q = empty_like_device(codes, {N, H}, kFp8);
+    s = empty_like_device(codes, {H / 128, N}, at::kFloat);
+    if (N == 0) return OMO_OK;
+    return omo_hip_permute_Mxfp4ToFp8_copy(codes.data_ptr(), cspan, cstride, scales.data_ptr(), sspan, sstride, T, H,
+                                           m.src.data_ptr<int32_t>(), N,
+                                           scratch ? src.data_ptr<int32_t>() : nullptr, q.data_ptr(), q.numel(),
+                                           s.data_ptr(), s.numel(), stream_of(codes));
+  });
+  if (!ok(m) || !ok(status)) return nullptr;
   PyObject* loads = list_of_ints(m.loads);
   PyObject* ts = loads ? tuple_of({q, s, src}) : nullptr;
   PyObject* r = ts ? PyTuple_Pack(4, PyTuple_GET_ITEM(ts, 0), PyTuple_GET_ITEM(ts, 1), PyTuple_GET_ITEM(ts, 2), loads)

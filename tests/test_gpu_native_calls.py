@@ -241,3 +241,58 @@ def test_refused_row_order_leaves_pinned_memory_alone(dev, num_out):
     for a, b in zip(got[:3], want[:3]):
         assert torch.equal(a.cpu().view(torch.uint8), b.view(torch.uint8))
     assert got[3] == want[3]
+
+
+@pytest.mark.parametrize("name", ["quantize", "dual", "grouped", "dequant", "requant", "row_to_col", "splits", "packed",
+                                  "requant packed", "row map", "permute"])
+def test_other_threads_run_while_a_call_allocates(dev, name):
+    """A call whose outputs fit only once cached memory is freed waits for the
+    device inside its allocation; other Python threads run meanwhile."""
+    import threading
+    import time
+    mx, de, ep, pe = _apis()
+    print("threads while", name, flush=True)
+    M, K = 8192, 8192
+    x = torch.zeros((M, K), dtype=torch.bfloat16, device=dev)
+    q, s = torch.zeros((M, K // 2), dtype=torch.uint8, device=dev), torch.full((M, K // 32), 127, dtype=torch.uint8, device=dev)
+    payload, rm = torch.cat((q, s), 1), torch.zeros((M, 1024), dtype=torch.bool, device=dev)
+    rm[:, 3] = True
+    call = {"quantize": lambda: mx.omo_per_token_group_quant_mxfp4(x),
+            "dual": lambda: mx.omo_per_token_group_quant_mxfp4_dual(x),
+            "grouped": lambda: mx.omo_per_token_group_quant_mxfp4_dual_grouped([x]),
+            "dequant": lambda: de.omo_per_token_mxfp4ToBf16_dequant_wrapper(q, s, torch.float32),
+            "requant": lambda: de.omo_per_token_mxfp4ToFp8_wrapper(q, s, [M]),
+            "row_to_col": lambda: de.omo_per_token_mxfp4RowToBf16ToFp8Col_wrapper(q, s),
+            "splits": lambda: de.omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper(q, s, [M]),
+            "packed": lambda: ep.fp4_quantize_packed(x),
+            "requant packed": lambda: ep.packed_mxfp4ToFp8(payload, [M]),
+            "row map": lambda: pe.make_row_id_map(rm),
+            "permute": lambda: pe.mxfp4_permute_to_fp8(q[:, :64], s[:, :4], rm)}[name]
+    call()  # its kernels are loaded
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # 480 MB in free pieces smaller than the outputs, none beside another
+    pieces = [torch.empty(12 << 20, dtype=torch.uint8, device=dev) for _ in range(80)]
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.001):
+            ticks.append(time.perf_counter())
+
+    thread = threading.Thread(target=tick)
+    try:
+        del pieces[::2]
+        torch.cuda._sleep(200 * 2_400_000)
+        thread.start()
+        t0 = time.perf_counter()
+        call()
+        t1 = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        torch.cuda.synchronize()
+    assert t1 - t0 > 0.05, "the allocation did not wait"
+    assert sum(t0 < t < t1 for t in ticks) > 20 * (t1 - t0) / 0.1, (t1 - t0, len(ticks))
