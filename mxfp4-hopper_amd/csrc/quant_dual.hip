@@ -25,6 +25,8 @@
 // piece stored by different waves, each store instruction touched 64
 // different lines; pairing them cut the 7168 x 18432 kernel from 93 to 83 us.)
 //
+#include <algorithm>
+
 #include "omo_internal.h"
 #include "omo_quant.cuh"
 
@@ -87,7 +89,7 @@ __device__ __forceinline__ uint2 quant_half16_ref(const uint32_t (&p)[8], float 
   return make_uint2(o[0], o[1]);
 }
 
-// One 64 x 256 tile (index `logical`, M-fastest) of the [M, K] tensor x,
+// One 64 x 256 tile (tile row mt, band kt) of the [M, K] tensor x,
 // 512 threads. FULL: every tile of the tensor is whole (M % 64 == 0, K % 256
 // == 0): no clamping, no store under a bounds test (512 x 7168 4.90 -> 4.72
 // us, 2048 x 7168 11.6 -> 11.3, 8192 x 7168 35.0 -> 34.8). LINES: K % 256 ==
@@ -102,10 +104,9 @@ __device__ __forceinline__ uint2 quant_half16_ref(const uint32_t (&p)[8], float 
 template <bool FULL, bool LINES>
 __device__ __forceinline__ void dual_tile(const uint16_t* __restrict__ x, uint32_t* __restrict__ row_q,
                                           uint8_t* __restrict__ row_s, uint8_t* __restrict__ col_q,
-                                          uint8_t* __restrict__ col_s, int64_t M, int64_t K, int tiles_m,
-                                          int logical, float eps, int c_eps, uint8_t* tile, uint8_t* rs_tile) {
+                                          uint8_t* __restrict__ col_s, int64_t M, int64_t K, int64_t mt, int64_t kt,
+                                          float eps, int c_eps, uint8_t* tile, uint8_t* rs_tile) {
   const int t = threadIdx.x;
-  const int64_t mt = logical % tiles_m, kt = logical / tiles_m;
   const int64_t m0 = mt * kDualRows, k0 = kt * kDualCols;
   const int rows_valid = FULL ? kDualRows : (int)(M - m0 < kDualRows ? M - m0 : kDualRows);  // 32 or 64
   // lane t owns 16 B column chunk cc of rows r0 + 16k (k = 0..3)
@@ -224,13 +225,56 @@ __device__ __forceinline__ void dual_tile(const uint16_t* __restrict__ x, uint32
 // 68.0 us against 73.3 us for M-fastest ranges (each XCD finishing one band
 // before the next) and 73.4 us for K-fastest ones (the XCDs on different
 // stripes), which also write 10 MB more (scale lines leaving L2 partly
-// filled). Returns false past the XCD's range.
-__device__ __forceinline__ bool band_group_tile(int xcd, int j, int S, int T, int per_xcd, int* ms, int* kb) {
-  const int lo = xcd * per_xcd, hi = min(T, lo + per_xcd);
-  if (j >= hi - lo) return false;
-  const int kb0 = lo / S, ms0 = lo - kb0 * S;  // first tile of the range
+// filled).
+struct BandUnits {
+  int rows, count;  // S; S * B
+  int per_xcd;      // ceil(S * B / 8)
+  int shift;        // log2 of the tiles per unit
+  int last;         // tiles of a unit of the last row: 1 .. 1 << shift
+};
+
+static BandUnits band_units(int64_t tiles_m, int64_t bands, int shift) {
+  const int64_t rows = (tiles_m + (1 << shift) - 1) >> shift, count = rows * bands;
+  return {(int)rows, (int)count, (int)((count + kXcds - 1) / kXcds), shift,
+          (int)(tiles_m - (rows - 1) * (1 << shift))};
+}
+
+// Tiles of XCD xcd's range: hi / rows - lo / rows of its units are in the last
+// row.
+static int band_group_tiles(int xcd, const BandUnits& u) {
+  const int lo = xcd * u.per_xcd, end = lo + u.per_xcd, hi = end < u.count ? end : u.count;
+  if (hi <= lo || u.rows == 0) return 0;
+  return ((hi - lo) << u.shift) - ((1 << u.shift) - u.last) * (hi / u.rows - lo / u.rows);
+}
+
+// Tile row and band of tile j of XCD xcd's walk; false past its range. The
+// last row of units, which may hold fewer tiles each, comes last in the walk,
+// so no position is without a tile (with four positions for each of its units
+// 64 x 786432 took 67.1 us against 28.7, 576 x 196608 78.7 against 65.1, 32
+// items of 64 x 32768 109.7 against 36.0; and 32 x 2^29 passed the 2^32 - 1
+// work-items of a launch).
+// TILES: units of one tile (shift 0).
+template <bool TILES>
+__device__ __forceinline__ bool band_group_tile(int xcd, int j, const BandUnits& u, int* ms, int* kb) {
+  const int S = u.rows, lo = xcd * u.per_xcd, hi = min(u.count, lo + u.per_xcd);
+  const int kb0 = lo / S, ms0 = lo - kb0 * S;  // first unit of the range
   const int kb1 = hi / S, ms1 = hi - kb1 * S;  // one past the last
-  // tiles of the range in rows below m: band kb0 holds rows
+  if (TILES ? j >= hi - lo : hi <= lo) return false;
+  int tile = 0;
+  if (!TILES) {
+    const int upper = hi - lo - (kb1 - kb0);  // units above the last row
+    if (j < upper << u.shift) {
+      tile = j & ((1 << u.shift) - 1);
+      j >>= u.shift;
+    } else {
+      const int k = j - (upper << u.shift);
+      const int q = u.last == 3 ? k / 3 : k >> (u.last >> 1);  // k / last
+      if (q >= kb1 - kb0) return false;
+      j = upper + q;
+      tile = k - q * u.last;
+    }
+  }
+  // units of the range in rows below m: band kb0 holds rows
   // [ms0, S) (or [ms0, ms1) when kb0 == kb1), bands kb0 + 1 .. kb1 - 1 all,
   // band kb1 [0, ms1)
   auto below = [&](int m) {
@@ -243,7 +287,7 @@ __device__ __forceinline__ bool band_group_tile(int xcd, int j, int S, int T, in
     if (below(mid) <= j) a = mid;
     else b = mid;
   }
-  *ms = a;
+  *ms = TILES ? a : (a << u.shift) + tile;
   *kb = kb0 + (a >= ms0 ? 0 : 1) + (j - below(a));
   return true;
 }
@@ -258,34 +302,32 @@ __device__ __forceinline__ bool band_group_tile(int xcd, int j, int S, int T, in
 // where this one has four) took 72.3, 71.4 and 65.5 us there, 127.5 against
 // 118.9 at 28672 x 8192, and 84.3 against 79.1 at 7168 x 18432 after a 512 MB
 // fill.
-constexpr int kDualQuad = 4;
+constexpr int kDualQuadShift = 2;  // log2 of the tiles per unit
 
-// quads_m > 0: band groups over quads_m x bands units of four tiles, per_xcd
-// of them per XCD. Else each XCD takes a contiguous M-fastest range of
-// per_xcd tiles. Measured (graph replays): 8192 x 7168 37.1 us against 38.3,
-// 4096 x 7168 20.7 against 21.1; with fewer than six tiles per CU the ranges
-// are ahead (7168 x 2048 11.7 against 12.0, 2048 x 2048 5.5 against 5.9).
+// units.rows > 0: band groups over those units. Else each XCD takes a
+// contiguous M-fastest range of units.per_xcd tiles. Measured (graph
+// replays): 8192 x 7168 37.1 us against 38.3, 4096 x 7168 20.7 against 21.1;
+// with fewer than six tiles per CU the ranges are ahead (7168 x 2048 11.7
+// against 12.0, 2048 x 2048 5.5 against 5.9).
 template <bool FULL, bool LINES>
 __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(const uint16_t* __restrict__ x, uint32_t* __restrict__ row_q,
                                                          uint8_t* __restrict__ row_s, uint8_t* __restrict__ col_q,
                                                          uint8_t* __restrict__ col_s, int64_t M, int64_t K,
-                                                         int tiles_m, int tiles, int quads_m, int quads, int per_xcd,
-                                                         float eps, int c_eps) {
+                                                         int tiles_m, int tiles, BandUnits units, float eps,
+                                                         int c_eps) {
   __shared__ __attribute__((aligned(16))) uint8_t tile[kDualRows * kDualPitch];
   __shared__ __attribute__((aligned(8))) uint8_t rs_tile[kDualRows * 8];
   const int xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
-  int logical;
-  if (quads_m > 0) {
-    int ms, kb;
-    if (!band_group_tile(xcd, j / kDualQuad, quads_m, quads, per_xcd, &ms, &kb)) return;
-    ms = ms * kDualQuad + j % kDualQuad;
-    if (ms >= tiles_m) return;  // the last row of units may hold fewer than four tiles
-    logical = kb * tiles_m + ms;
+  int ms, kb;
+  if (units.rows > 0) {
+    if (!band_group_tile<false>(xcd, j, units, &ms, &kb)) return;
   } else {
-    logical = xcd * per_xcd + j;
+    const int logical = xcd * units.per_xcd + j;
     if (logical >= tiles) return;
+    ms = logical % tiles_m;
+    kb = logical / tiles_m;
   }
-  dual_tile<FULL, LINES>(x, row_q, row_s, col_q, col_s, M, K, tiles_m, logical, eps, c_eps, tile, rs_tile);
+  dual_tile<FULL, LINES>(x, row_q, row_s, col_q, col_s, M, K, ms, kb, eps, c_eps, tile, rs_tile);
 }
 
 // Grouped form: one launch over up to kDualGroupMax tensors (e.g. the weights
@@ -299,16 +341,20 @@ struct DualItem {
   uint8_t* col_q;
   uint8_t* col_s;
   int64_t M, K;
-  int tiles_m;         // the item's 64-row tile rows
-  int shift;           // log2 of the tiles per unit: 0, or 2 (kDualQuad)
-  int units_m, units;  // its units
-  int per_xcd;         // and their per-XCD share
+  BandUnits units;  // of its 64-row tiles
 };
 
 struct DualGroup {
   DualItem item[kDualGroupMax];
-  int count, tiles, per_xcd, c_eps;
+  int count, tiles, c_eps;
   float eps;
+};
+
+// With items walked in fours: each XCD's tiles of each item, counted by the
+// host (with two divisions per item in every workgroup 24 expert weights took
+// 330 us against 201).
+struct DualGroupFours : DualGroup {
+  int share[kXcds][kDualGroupMax];
 };
 
 // Each XCD takes its band-group share of each item, item after item, over
@@ -326,25 +372,36 @@ struct DualGroup {
 // 201.9 us tile by tile, 201.5 in fours; ffn 4096: 401.5 and 405.5).
 constexpr int kDualWideBands = 64;
 
-template <bool FULL, bool LINES>
-__global__ __launch_bounds__(kDualThreads) void quant_dual_grouped_kernel(const DualGroup g) {
+// Group: DualGroup where no item is walked in fours (8 of 2048 x 2048 with the
+// general walk and its table 22.1 us against 21.8).
+template <bool FULL, bool LINES, typename Group>
+__global__ __launch_bounds__(kDualThreads) void quant_dual_grouped_kernel(const Group g) {
+  constexpr bool TILES = std::is_same_v<Group, DualGroup>;
   __shared__ __attribute__((aligned(16))) uint8_t tile[kDualRows * kDualPitch];
   __shared__ __attribute__((aligned(8))) uint8_t rs_tile[kDualRows * 8];
   const int b = blockIdx.x, xcd = b % kXcds;
   int j = b / kXcds, i = 0;
   for (; i < g.count; i++) {
-    const int n = min(max(g.item[i].units - xcd * g.item[i].per_xcd, 0), g.item[i].per_xcd) << g.item[i].shift;
+    const BandUnits& u = g.item[i].units;
+    int n;
+    if constexpr (TILES) n = min(max(u.count - xcd * u.per_xcd, 0), u.per_xcd);
+    else n = g.share[xcd][i];
     if (j < n) break;
     j -= n;
   }
   if (i == g.count) return;
   const DualItem& it = g.item[i];
   int ms, kb;
-  if (!band_group_tile(xcd, j >> it.shift, it.units_m, it.units, it.per_xcd, &ms, &kb)) return;
-  ms = (ms << it.shift) + (j & ((1 << it.shift) - 1));
-  if (ms >= it.tiles_m) return;
-  dual_tile<FULL, LINES>(it.x, it.row_q, it.row_s, it.col_q, it.col_s, it.M, it.K, it.tiles_m, kb * it.tiles_m + ms, g.eps,
-                  g.c_eps, tile, rs_tile);
+  if (!band_group_tile<TILES>(xcd, j, it.units, &ms, &kb)) return;
+  dual_tile<FULL, LINES>(it.x, it.row_q, it.row_s, it.col_q, it.col_s, it.M, it.K, ms, kb, g.eps, g.c_eps, tile,
+                         rs_tile);
+}
+
+// The largest XCD's share of a tensor's tiles: the grid's positions per XCD.
+static int band_group_slots(const BandUnits& u) {
+  int n = 0;
+  for (int x = 0; x < kXcds; x++) n = std::max(n, band_group_tiles(x, u));
+  return n;
 }
 
 // Tensors of whole 64 x 256 tiles.
@@ -357,25 +414,28 @@ hipError_t launch_quant_dual(const void* x, void* row_q, void* row_s, void* col_
   const int64_t tiles_k = (K + kDualCols - 1) / kDualCols;
   const int64_t tiles = tiles_m * tiles_k;
   const bool band_group = tiles >= 6 * (int64_t)current_device_caps().cus;
-  const int64_t quads_m = band_group ? (tiles_m + kDualQuad - 1) / kDualQuad : 0, quads = quads_m * tiles_k;
-  const int64_t per_xcd = ((band_group ? quads : tiles) + kXcds - 1) / kXcds;
-  const int64_t grid = per_xcd * kXcds * (band_group ? kDualQuad : 1);
+  BandUnits units = {0, 0, (int)((tiles + kXcds - 1) / kXcds), 0, 1};
+  int64_t slots = units.per_xcd;  // of each XCD
+  if (band_group) {
+    units = band_units(tiles_m, tiles_k, kDualQuadShift);
+    slots = band_group_slots(units);
+  }
   auto kernel = dual_full(M, K)        ? quant_dual_kernel<true, true>
                 : K % kDualCols == 0 ? quant_dual_kernel<false, true>
                                      : quant_dual_kernel<false, false>;
-  return launch(kernel, dim3((unsigned)grid), dim3(kDualThreads), 0, stream, static_cast<const uint16_t*>(x),
+  return launch(kernel, dim3((unsigned)(slots * kXcds)), dim3(kDualThreads), 0, stream, static_cast<const uint16_t*>(x),
                 static_cast<uint32_t*>(row_q), static_cast<uint8_t*>(row_s), static_cast<uint8_t*>(col_q),
-                static_cast<uint8_t*>(col_s), M, K, (int)tiles_m, (int)tiles, (int)quads_m, (int)quads, (int)per_xcd,
-                eps, host_c_eps(eps, 6.0f));
+                static_cast<uint8_t*>(col_s), M, K, (int)tiles_m, (int)tiles, units, eps,
+                host_c_eps(eps, 6.0f));
 }
 
 hipError_t launch_quant_dual_grouped(const DualSpec* items, int count, float eps, hipStream_t stream) {
   for (int base = 0; base < count; base += kDualGroupMax) {
-    DualGroup g;
+    DualGroupFours g;
     memset(&g, 0, sizeof(g));
     g.count = count - base < kDualGroupMax ? count - base : kDualGroupMax;
-    bool full = true, lines = true;
-    int tiles = 0;
+    bool full = true, lines = true, single = true;
+    int tiles = 0, slots[kXcds] = {};  // of the items so far: tiles, and each XCD's share
     for (int j = 0; j < g.count; j++) {
       const DualSpec& d = items[base + j];
       DualItem& it = g.item[j];
@@ -386,25 +446,29 @@ hipError_t launch_quant_dual_grouped(const DualSpec* items, int count, float eps
       it.col_s = static_cast<uint8_t*>(d.col_s);
       it.M = d.M;
       it.K = d.K;
-      it.tiles_m = (int)((d.M + kDualRows - 1) / kDualRows);
+      const int64_t tiles_m = (d.M + kDualRows - 1) / kDualRows;
       const int bands = d.M == 0 ? 0 : (int)((d.K + kDualCols - 1) / kDualCols);
-      it.shift = bands > kDualWideBands ? 2 : 0;
-      it.units_m = (it.tiles_m + (1 << it.shift) - 1) >> it.shift;
-      it.units = it.units_m * bands;
-      it.per_xcd = (it.units + kXcds - 1) / kXcds;
-      tiles += it.tiles_m * bands;
-      g.per_xcd += it.per_xcd << it.shift;  // XCD 0 has the largest share of every item: the grid's slots per XCD
+      it.units = band_units(tiles_m, bands, bands > kDualWideBands ? kDualQuadShift : 0);
+      tiles += (int)tiles_m * bands;
+      for (int x = 0; x < kXcds; x++) slots[x] += g.share[x][j] = band_group_tiles(x, it.units);
       full = full && dual_full(d.M, d.K);
       lines = lines && d.K % kDualCols == 0;
+      single = single && it.units.shift == 0;
     }
     if (tiles == 0) continue;
     g.tiles = tiles;
     g.eps = eps;
     g.c_eps = host_c_eps(eps, 6.0f);
-    auto kernel = full    ? quant_dual_grouped_kernel<true, true>
-                  : lines ? quant_dual_grouped_kernel<false, true>
-                          : quant_dual_grouped_kernel<false, false>;
-    const hipError_t e = launch(kernel, dim3((unsigned)(g.per_xcd * kXcds)), dim3(kDualThreads), 0, stream, g);
+    const dim3 grid((unsigned)(*std::max_element(slots, slots + kXcds) * kXcds));
+    const hipError_t e =
+        single ? launch(full    ? quant_dual_grouped_kernel<true, true, DualGroup>
+                        : lines ? quant_dual_grouped_kernel<false, true, DualGroup>
+                                : quant_dual_grouped_kernel<false, false, DualGroup>,
+                        grid, dim3(kDualThreads), 0, stream, static_cast<const DualGroup&>(g))
+               : launch(full    ? quant_dual_grouped_kernel<true, true, DualGroupFours>
+                        : lines ? quant_dual_grouped_kernel<false, true, DualGroupFours>
+                                : quant_dual_grouped_kernel<false, false, DualGroupFours>,
+                        grid, dim3(kDualThreads), 0, stream, g);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -51,8 +51,11 @@ def test_whole_tiles(oracle, dev, M, K, row_shift, col_shift):
 
 # The orders of the tiles: ranges (few tiles), band groups in units of four
 # tiles with a last row of units of one to four (6 tiles per CU: 1536 tiles),
-# and grouped items of at most and of more than 64 bands side by side.
-@pytest.mark.parametrize("M,K", [(64 * 23, 256 * 67), (64 * 24, 256 * 64), (64 * 25 + 32, 256 * 62 + 32), (64 * 1538, 256)])
+# tensors of only such a row, and grouped items of at most and of more than 64
+# bands side by side.
+@pytest.mark.parametrize("M,K", [(64 * 23, 256 * 67), (64 * 24, 256 * 64), (64 * 25 + 32, 256 * 62 + 32), (64 * 1538, 256),
+                                 (32, 256 * 1537), (64 * 2, 256 * 771), (64 * 3 - 32, 256 * 512 + 64), (64 * 4, 256 * 385),
+                                 (64 * 5, 256 * 311), (64 * 7, 256 * 220)])
 def test_orders(oracle, dev, M, K):
     import omo
     print("dual order", M, K, flush=True)
@@ -60,12 +63,13 @@ def test_orders(oracle, dev, M, K):
     xd = x.to(dev)
     outs = _outs(dev, M, K, 0, 0)
     omo.omo_quant_mxfp4_dual(xd, *outs)
-    small = xd[:160, :].contiguous()
-    grouped = [_outs(dev, 160, K, 0, 0), _outs(dev, M, K, 0, 0), _outs(dev, 160, K, 0, 0)]
+    R = min(M, 160)
+    small = xd[:R, :].contiguous()
+    grouped = [_outs(dev, R, K, 0, 0), _outs(dev, M, K, 0, 0), _outs(dev, R, K, 0, 0)]
     omo.omo_quant_mxfp4_dual_grouped([small, xd, small], grouped)
     torch.cuda.synchronize()
     _check(oracle, x, outs)
     for a, b in zip(outs, grouped[1]):
         assert torch.equal(a, b)
     for o in (grouped[0], grouped[2]):
-        _check(oracle, x[:160], o)
+        _check(oracle, x[:R], o)

@@ -138,6 +138,30 @@ def test_dual_past_2_31(oracle, dev):
         np.testing.assert_array_equal(bits_u8(cs[c0:c0 + 256]).reshape(-1), es)
 
 
+@pytest.mark.parametrize("grouped", [False, True])
+def test_dual_one_tile_row_of_many_bands(oracle, dev, grouped):
+    """32 rows of 2^29 columns (34 GB): 2^21 tiles in one tile row, a quarter
+    of the workgroups of 512 lanes that a launch holds, so a grid with a
+    position for each tile of a unit of four would not launch."""
+    from omo_python_api.mxfp4 import omo_per_token_group_quant_mxfp4_dual, omo_per_token_group_quant_mxfp4_dual_grouped
+    M, K = 32, 2**29
+    _say("dual, one tile row", M, K, grouped)
+    g = torch.Generator(device=dev).manual_seed(36)
+    x = torch.randn((M, K), generator=g, device=dev, dtype=torch.bfloat16)
+    rq, rs, cq, cs = (omo_per_token_group_quant_mxfp4_dual_grouped([x])[0] if grouped
+                      else omo_per_token_group_quant_mxfp4_dual(x))
+    torch.cuda.synchronize()
+    for c0 in (0, 2**28 - 128, K - 256):
+        c1 = c0 + 256
+        xb = bits_u16(x[:, c0:c1])
+        eq, es = oracle.quant_mxfp4(np.ascontiguousarray(xb).reshape(-1))
+        np.testing.assert_array_equal(bits_u8(rq[:, c0 // 2:c1 // 2]).reshape(-1), eq)
+        np.testing.assert_array_equal(bits_u8(rs[:, c0 // 32:c1 // 32]).reshape(-1), es)
+        eq, es = oracle.quant_mxfp4(np.ascontiguousarray(xb.T).reshape(-1))
+        np.testing.assert_array_equal(bits_u8(cq[c0:c1]).reshape(-1), eq)
+        np.testing.assert_array_equal(bits_u8(cs[c0:c1]).reshape(-1), es)
+
+
 def _msplit_gpu(dev, q, s, splits):
     import omo
     from omo_python_api.mxfp4_dequant import split_metadata
