@@ -162,7 +162,8 @@ OMO_API int omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit(const void* input, i
  * copied into the launch's arguments, so no metadata is copied to the device
  * and nothing waits for the stream. output_s: sum of ceil(m_splits[i]/128)
  * rows of N. Outputs equal the device-metadata entry point's. Up to 128
- * splits, N % 32 == 0, input 16-byte aligned; OMO_ERR_UNSUPPORTED otherwise.
+ * splits, N % 32 == 0, input 16-byte aligned, fewer than 2^24 tiles of 128
+ * rows x 256 columns (2^32 - 1 work-items); OMO_ERR_UNSUPPORTED otherwise.
  * A captured launch keeps the lengths of the capture. */
 OMO_API int omo_hip_Mxfp4RowToBf16ToFp8Col_splits(const void* input, int64_t rows, int64_t row_bytes,
                                           const void* input_s, int64_t input_s_bytes, void* output_q,

@@ -372,14 +372,15 @@ PyObject* row_to_col_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (size_t i = 0; i < lens.size(); i++) rows += tiles[i] = (lens[i] + 127) / 128;
   const c10::DeviceGuard guard(x.device());
   Tensor q, qs;
-  if (!ok(unlocked([&] {
-        q = empty_like_device(x, {M * N}, kFp8);
-        qs = empty_like_device(x, {rows, N}, at::kFloat);
-        return omo_hip_Mxfp4RowToBf16ToFp8Col_splits(x.data_ptr(), M, N / 2, s.data_ptr(), scales, q.data_ptr(), M * N,
-                                                     qs.data_ptr(), rows * N, lens.data(), (int64_t)lens.size(), eps,
-                                                     stream_of(x));
-      })))
-    return nullptr;
+  const int status = unlocked([&] {
+    q = empty_like_device(x, {M * N}, kFp8);
+    qs = empty_like_device(x, {rows, N}, at::kFloat);
+    return omo_hip_Mxfp4RowToBf16ToFp8Col_splits(x.data_ptr(), M, N / 2, s.data_ptr(), scales, q.data_ptr(), M * N,
+                                                 qs.data_ptr(), rows * N, lens.data(), (int64_t)lens.size(), eps,
+                                                 stream_of(x));
+  });
+  if (status == OMO_ERR_UNSUPPORTED) return none();  // past one launch: device metadata
+  if (!ok(status)) return nullptr;
   std::vector<Tensor> blocks;
   blocks.reserve(lens.size());
   int64_t at = 0;

@@ -410,10 +410,11 @@ int omo_hip_Mxfp4RowToBf16ToFp8Col_splits(const void* input, int64_t rows, int64
   REQUIRE_BUF("output_s", output_s, output_s_elems, out_s_need);
   REQUIRE(aligned(output_s, 4), "%s: misaligned buffer", fn);
   if (M == 0 || N == 0) return ok();
-  if (!omo_hip::row_to_fp8_col_splits_ok(input, M, N, num_splits))
+  if (!omo_hip::row_to_fp8_col_splits_ok(input, M, N, m_splits, num_splits))
     return fail(OMO_ERR_UNSUPPORTED,
-                "%s: takes up to 128 splits of rows of N %% 32 == 0 elements with 16-byte aligned codes; pass device "
-                "metadata to omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit instead", fn);
+                "%s: takes up to 128 splits of rows of N %% 32 == 0 elements with 16-byte aligned codes, in one launch "
+                "of 2^32 - 1 work-items; pass device metadata to omo_hip_per_token_Mxfp4RowToBf16ToFp8Col_msplit "
+                "instead", fn);
   return from_hip(omo_hip::launch_row_to_fp8_col_splits(input, input_s, output_q, static_cast<float*>(output_s), M, N,
                                                         m_splits, num_splits, scale_rows, eps, as_stream(stream)),
                   fn);

@@ -53,7 +53,7 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
 // Splits back to back with host-known lengths; only for the forms
 // row_to_fp8_col_splits_ok accepts (at most 128 splits, N % 32 == 0, 16 B
 // aligned codes, a grid within the launch limits).
-bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, int64_t nsplits);
+bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, const int64_t* lens, int64_t nsplits);
 hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,
                                         int64_t N, const int64_t* lens, int64_t nsplits, int64_t out_s_rows, float eps,
                                         hipStream_t stream);

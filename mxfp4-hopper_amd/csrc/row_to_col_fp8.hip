@@ -1281,36 +1281,47 @@ static auto split_flat_kernel(int64_t nsplits, bool walk, bool narrow_n) {
                                  : row_to_fp8_col_msplit_flat_kernel<1, false, false, Splits>);
 }
 
-bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, int64_t nsplits) {
+// The order and the grid of splits by value: exactly the tiles there are
+// (device lengths need nsplits times the longest split's).
+struct ValueGrid {
+  int64_t row_tiles, bands, blocks;
+  bool walk;
+};
+
+static ValueGrid value_grid(int64_t N, const int64_t* lens, int64_t nsplits) {
+  ValueGrid g = {0, (N + kWideCols - 1) / kWideCols, 0, false};
+  g.walk = split_walk(nsplits, g.bands, 16);
+  int64_t per_xcd = 0;
+  for (int64_t i = 0; i < nsplits; i++) {
+    const int64_t tiles = (lens[i] + kTile - 1) / kTile;
+    g.row_tiles += tiles;
+    per_xcd += (tiles * g.bands + 7) / 8;  // XCD 0 has the largest share of every split
+  }
+  g.blocks = g.walk ? 8 * per_xcd : g.row_tiles * g.bands;
+  return g;
+}
+
+bool row_to_fp8_col_splits_ok(const void* q, int64_t total_rows, int64_t N, const int64_t* lens, int64_t nsplits) {
   return nsplits <= kFlatMaxSplits && N % 32 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0 &&
-         total_rows <= INT32_MAX && total_rows / kTile + nsplits < (int64_t)UINT32_MAX / 256 / (N / kWideCols + 1) - 8;
+         total_rows <= INT32_MAX && value_grid(N, lens, nsplits).blocks <= (int64_t)UINT32_MAX / 256;
 }
 
 // Splits back to back with lengths known to the host, in the forms that
-// row_to_fp8_col_splits_ok accepts. The grid holds exactly the tiles there
-// are (device lengths need nsplits times the longest split's).
+// row_to_fp8_col_splits_ok accepts.
 hipError_t launch_row_to_fp8_col_splits(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,
                                         int64_t N, const int64_t* lens, int64_t nsplits, int64_t out_s_rows, float eps,
                                         hipStream_t stream) {
   ValueSplits v;
   memset(&v, 0, sizeof(v));
-  const int64_t bands = (N + kWideCols - 1) / kWideCols;
-  const bool walk = split_walk(nsplits, bands, 16);
-  int64_t row_tiles = 0, per_xcd = 0;
-  for (int64_t i = 0; i < nsplits; i++) {
-    const int64_t tiles = (lens[i] + kTile - 1) / kTile;
-    v.lens[i] = (int32_t)lens[i];
-    row_tiles += tiles;
-    per_xcd += (tiles * bands + 7) / 8;  // XCD 0 has the largest share of every split
-  }
-  const int64_t grid = walk ? 8 * per_xcd : row_tiles * bands;
-  if (grid == 0) return hipSuccess;
+  const ValueGrid g = value_grid(N, lens, nsplits);
+  for (int64_t i = 0; i < nsplits; i++) v.lens[i] = (int32_t)lens[i];
+  if (g.blocks == 0) return hipSuccess;
   const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
   const bool out_line = (reinterpret_cast<uintptr_t>(out) & 127) == 0;
-  return launch(split_flat_kernel<ValueSplits>(nsplits, walk, narrow_n), dim3((unsigned)grid), dim3(256),
-                split_lds_reserve(row_tiles * bands), stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
-                static_cast<uint8_t*>(out), out_s, v, total_rows, N, out_s_rows, eps, out_line, (int)nsplits,
-                (int)row_tiles, (int)bands);
+  return launch(split_flat_kernel<ValueSplits>(nsplits, g.walk, narrow_n), dim3((unsigned)g.blocks), dim3(256),
+                split_lds_reserve(g.row_tiles * g.bands), stream, static_cast<const uint8_t*>(q),
+                static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, v, total_rows, N, out_s_rows, eps,
+                out_line, (int)nsplits, (int)g.row_tiles, (int)g.bands);
 }
 
 hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out, float* out_s, int64_t total_rows,

@@ -207,37 +207,36 @@ def omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper(data: torch.Tensor, scal
     [ceil(m_i/128), N]), one per expert split, each a view of one buffer.
 
     Up to 128 splits of 16 B aligned code rows travel by value with the
-    launch. More splits, and rows the 256-column tiles do not take, go through
-    a device copy of the metadata, for which the host waits."""
+    launch. More splits, rows the 256-column tiles do not take and tiles past
+    one launch go through a device copy of the metadata, for which the host
+    waits."""
     done = native.row_to_col_splits(data, scale, m_splits, eps)
     if done is not None:
         return done
     assert data.dim() == 2 and data.is_contiguous(), "`data` must be a contiguous 2-D tensor"
     total_m, half = data.shape
     N = half * 2
-    by_value = len(m_splits) <= MAX_VALUE_SPLITS and N % 32 == 0 and data.data_ptr() % 16 == 0 and total_m < 2**31
-    if by_value:
-        lens = [int(m) for m in m_splits]
-        if any(m < 0 for m in lens):
-            raise ValueError(f"m_splits must be non-negative, got {lens}")
-        rows, tiles = sum(lens), [(m + 127) // 128 for m in lens]
-        srows = sum(tiles)
-    else:
-        lens, offs, soffs, max_len, rows, srows = split_metadata(m_splits, data.device)
-        tiles = [(int(m) + 127) // 128 for m in m_splits]
+    lens = [int(m) for m in m_splits]
+    if any(m < 0 for m in lens):
+        raise ValueError(f"m_splits must be non-negative, got {lens}")
+    rows, tiles = sum(lens), [(m + 127) // 128 for m in lens]
     if rows != total_m:
         raise ValueError(f"sum(m_splits)={rows} does not match data rows {total_m}")
     out_q = torch.empty(total_m * N, device=data.device, dtype=fp8_type_)
-    out_s = torch.empty((srows, N), device=data.device, dtype=torch.float)
-    if len(m_splits) > 0 and N > 0 and total_m > 0:
+    out_s = torch.empty((sum(tiles), N), device=data.device, dtype=torch.float)
+    if len(lens) > 0 and N > 0 and total_m > 0:
+        scale = scale.contiguous()
+        by_value = len(lens) <= MAX_VALUE_SPLITS and N % 32 == 0 and data.data_ptr() % 16 == 0 and total_m < 2**31
         if by_value:
-            omo_Mxfp4RowToBf16ToFp8Col_splits(data, scale.contiguous(), out_q, out_s, lens, eps)
-        else:
-            omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit(data, scale.contiguous(), out_q, out_s, lens, offs, soffs,
-                                                        max_len, eps)
+            try:
+                omo_Mxfp4RowToBf16ToFp8Col_splits(data, scale, out_q, out_s, lens, eps)
+            except NotImplementedError:  # more tiles than a launch holds
+                by_value = False
+        if not by_value:
+            meta, offs, soffs, max_len, _, _ = split_metadata(lens, data.device)
+            omo_per_token_Mxfp4RowToBf16ToFp8Col_msplit(data, scale, out_q, out_s, meta, offs, soffs, max_len, eps)
     y_data, y_scale, o = [], [], 0
-    for m in m_splits:
-        m = int(m)
+    for m in lens:
         y_data.append(out_q[o * N:(o + m) * N].view(N, m))
         o += m
     y_scale = list(torch.split(out_s, tiles, dim=0))

@@ -231,3 +231,24 @@ def test_msplit_more_column_bands_than_grid_z(oracle, dev, N, empty_tail, shift)
             o += m
         np.testing.assert_array_equal(np.concatenate(got), eo)
         np.testing.assert_array_equal(outs[:, c0:c0 + w].cpu().numpy().view(np.uint32), es.view(np.uint32))
+
+
+@pytest.mark.parametrize("splits,N", [([128, 1, 77] + [0] * 125, 2**25), ([1] * 128, 2**25 + 256)])
+def test_msplit_wrapper_of_many_bands(oracle, dev, splits, N):
+    """128 splits of rows of 2^25 columns and more (131,072 bands): few row
+    tiles, which one launch holds, go by value; 128 row tiles are more than
+    the 2^24 - 1 workgroups of 256 lanes of a launch and go by device
+    metadata. Column windows at both ends against the oracle, each split's
+    scale rows included."""
+    from omo_python_api.mxfp4_dequant import omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper
+    R = sum(splits)
+    _say("msplit wrapper", R, "rows", N)
+    q, s = _gpu_codes(dev, R, N, 37)
+    ys, ss = omo_per_token_mxfp4RowToBf16ToFp8Col_msplit_wrapper(q, s, splits)
+    torch.cuda.synchronize()
+    for c0 in (0, N - 512):
+        eo, es = oracle.row_to_fp8_col_msplit(bits_u8(q[:, c0 // 2:(c0 + 512) // 2]), bits_u8(s[:, c0 // 32:(c0 + 512) // 32]),
+                                              splits)
+        np.testing.assert_array_equal(np.concatenate([bits_u8(y[c0:c0 + 512]).reshape(-1) for y in ys]), eo)
+        got = torch.cat([t[:, c0:c0 + 512] for t in ss]).cpu().numpy()
+        np.testing.assert_array_equal(got.view(np.uint32), es.view(np.uint32))
