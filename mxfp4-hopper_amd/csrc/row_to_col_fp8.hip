@@ -1229,8 +1229,11 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
     // 21.9 against 23.5; 8190 x 5120, 1280, 20.7 against 18.2). Bands fastest
     // where many CUs stay idle all the same (five tiles per eight CUs: 1000 x
     // 2880, 96 tiles, 5.2 us against 5.6 rows fastest, 1500 x 2880, 144, 5.9
-    // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1).
-    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : tiles <= 5 * cus ? kRowsFastest : kBandWalk;
+    // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1). Rows fastest too
+    // where the walk's grid, whole eighths, would pass the work-items of a
+    // launch and the tiles alone do not.
+    const bool walk = tiles > 5 * cus && (tiles + 7) / 8 * 8 <= (int64_t)UINT32_MAX / 256;
+    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : walk ? kBandWalk : kRowsFastest;
     auto kernel = narrow_n ? (whole                    ? row_to_fp8_col_wide_kernel<false, true, kBandsFastest>
                               : order == kBandsFastest ? row_to_fp8_col_wide_kernel<true, true, kBandsFastest>
                               : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, true, kRowsFastest>

@@ -94,6 +94,26 @@ def test_row_to_fp8_col_past_2_31(oracle, dev):
                                       es.view(np.uint32))
 
 
+def test_row_to_fp8_col_most_row_tiles(oracle, dev):
+    """Dense row->col FP8 of 2^24 - 1 row tiles, the most workgroups of 256
+    lanes that a launch holds, the last one ragged: an order that rounds its
+    grid up would not launch."""
+    import omo
+    M, N = 128 * (2**24 - 1) - 5, 32
+    _say("row->col dense", M, N)
+    g = torch.Generator(device=dev).manual_seed(38)
+    q = torch.randint(0, 256, (M, N // 2), generator=g, dtype=torch.uint8, device=dev)
+    s = torch.randint(120, 131, (M, N // 32), generator=g, dtype=torch.uint8, device=dev)
+    out = torch.empty((N, M), dtype=torch.float8_e4m3fn, device=dev)
+    outs = torch.empty(((M + 127) // 128, N), dtype=torch.float32, device=dev)
+    omo.omo_per_token_Mxfp4RowToBf16ToFp8Col(q, s, out, outs, 1e-10)
+    torch.cuda.synchronize()
+    for r0, r1 in ((0, 256), (2**30, 2**30 + 384), ((M - 300) // 128 * 128, M)):
+        eo, es = oracle.row_to_fp8_col(bits_u8(q[r0:r1]), bits_u8(s[r0:r1]))
+        np.testing.assert_array_equal(bits_u8(out[:, r0:r1]), eo)
+        np.testing.assert_array_equal(outs[r0 // 128:(r1 + 127) // 128].cpu().numpy().view(np.uint32), es.view(np.uint32))
+
+
 def test_row_to_fp8_col_msplit_past_2_31(oracle, dev):
     """Per-split row->col FP8 over 8 ragged splits totalling 300,001 rows x
     7168 (2.15e9 elements): the last split's output block ends past 2^31
