@@ -18,6 +18,8 @@
 // every code byte under every scale byte. Scale byte 0 (which the hardware
 // reads as 2^-127, the reference as 0.0) and 255 (hardware NaN, reference
 // inf) take the fp32 restatement.
+#include <algorithm>
+
 #include "omo_device.cuh"
 #include "omo_internal.h"
 
@@ -176,9 +178,18 @@ static hipError_t dequant_rows(const void* q, int64_t q_stride, const void* s, i
                                int64_t rows, int64_t K, hipStream_t stream) {
   constexpr int U = 4, kUnit = 32 >> Out::kBlockShift;
   const int64_t bpr = (K / kUnit + 256 * U - 1) / (256 * U);
-  return launch((dequant_rows_kernel<Out, U>), dim3((unsigned)(rows * bpr)), dim3(256), 0, stream,
-                static_cast<const uint8_t*>(q), q_stride, static_cast<const uint8_t*>(s), s_stride,
-                static_cast<u32x4*>(out), K, (int)bpr);
+  // A launch holds 2^32 - 1 work-items. fp32 rows of more than 4096 elements
+  // take two workgroups where 16-bit ones take one, so row counts that bf16
+  // and a conversion pass took in one launch need a second here.
+  const int64_t most = std::max<int64_t>(1, (int64_t)UINT32_MAX / 256 / bpr);
+  for (int64_t r = 0; r < rows; r += most) {
+    const hipError_t e = launch((dequant_rows_kernel<Out, U>), dim3((unsigned)(std::min(most, rows - r) * bpr)), dim3(256),
+                                0, stream, static_cast<const uint8_t*>(q) + r * q_stride, q_stride,
+                                static_cast<const uint8_t*>(s) + r * s_stride, s_stride,
+                                static_cast<u32x4*>(out) + r * (K / kUnit), K, (int)bpr);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_dequant_rows(const void* q, int64_t q_stride, const void* s, int64_t s_stride, void* out,

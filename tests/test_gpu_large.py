@@ -61,6 +61,25 @@ def test_quant_requant_dequant_past_2_31(oracle, dev):
     assert torch.equal(y2.view(torch.int16), y.view(torch.int16))
 
 
+def test_payload_to_fp32_past_a_launch(oracle, dev):
+    """2^23 + 3 payload rows of 4224 elements to fp32: two workgroups of 256
+    lanes a row, past the 2^32 - 1 work-items of a launch. Row windows at both
+    ends and across the second launch's first row (2^23 - 1) against the
+    oracle's bf16 values."""
+    from omo_python_api.ep_payload import packed_mxfp4ToBf16
+    T, H = 2**23 + 3, 4224
+    _say("payload to fp32", T, H)
+    g = torch.Generator(device=dev).manual_seed(39)
+    p = torch.randint(118, 136, (T, H // 32 * 17), generator=g, dtype=torch.uint8, device=dev)
+    y = packed_mxfp4ToBf16(p, torch.float32)
+    torch.cuda.synchronize()
+    for r0 in (0, 2**22, 2**23 - 8, T - 8):
+        w = bits_u8(p[r0:r0 + 8])
+        want = oracle.dequant_bf16(np.ascontiguousarray(w[:, :H // 2]).reshape(-1), np.ascontiguousarray(w[:, H // 2:]).reshape(-1))
+        got = y[r0:r0 + 8].cpu().numpy().view(np.uint32).reshape(-1)
+        np.testing.assert_array_equal(got, np.asarray(want).astype(np.uint32) << 16)
+
+
 def _gpu_codes(dev, M, N, seed):
     """MXFP4 codes and scales of a seeded N(0,1) bf16 [M, N] tensor, quantized
     on the GPU (the quantize is checked past 2^31 elements above)."""
