@@ -14,10 +14,13 @@ namespace omo_hip {
 // Enqueues `kernel` with its arguments converted to the kernel's parameter
 // types and returns the status of this launch alone (hipLaunchKernel's return
 // value), so an error left earlier on the calling thread by other code is
-// neither reported as this launch's failure nor cleared.
+// neither reported as this launch's failure nor cleared. A launch holds
+// 2^32 - 1 work-items along x; HIP runs a longer one modulo 2^32 and returns
+// success, so it is refused here.
 template <typename... P, typename... A>
 hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A&&... args) {
   static_assert(sizeof...(P) == sizeof...(A), "kernel argument count");
+  if ((uint64_t)grid.x * block.x > UINT32_MAX) return hipErrorInvalidConfiguration;
   std::tuple<std::decay_t<P>...> vals(static_cast<std::decay_t<P>>(std::forward<A>(args))...);
   return std::apply(
       [&](auto&... v) {

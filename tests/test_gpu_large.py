@@ -80,6 +80,20 @@ def test_payload_to_fp32_past_a_launch(oracle, dev):
         np.testing.assert_array_equal(got, np.asarray(want).astype(np.uint32) << 16)
 
 
+def test_more_work_items_than_a_launch_holds(dev):
+    """A quantize into 2^24 + 1 payload rows would take as many workgroups of
+    256 lanes: refused, not run modulo 2^32; the largest that fits runs."""
+    from omo_python_api.ep_payload import fp4_quantize_packed
+    T, H = 2**24 + 1, 128
+    _say("payload quantize", T, H)
+    x = torch.ones((T, H), dtype=torch.bfloat16, device=dev)
+    with pytest.raises(RuntimeError, match="invalid configuration"):
+        fp4_quantize_packed(x)
+    y = fp4_quantize_packed(x[:T - 2])
+    torch.cuda.synchronize()
+    assert torch.equal(y[-1], y[0]) and torch.equal(y[2**23], y[0]) and int(y[0, 0]) != 0
+
+
 def _gpu_codes(dev, M, N, seed):
     """MXFP4 codes and scales of a seeded N(0,1) bf16 [M, N] tensor, quantized
     on the GPU (the quantize is checked past 2^31 elements above)."""
