@@ -239,18 +239,27 @@ def floors_leg(torch, args, dev, cur, lib, _abi, wl):
         if rc:
             raise RuntimeError(f"{what} returned {rc}")
 
+    def settled(launch, n_sets):
+        """Keep the GPU at work for about 40 ms: its clocks dip 1-2 ms after a
+        load begins, for about 15 ms, and what is timed first would pay."""
+        for _ in range(2):
+            t, _ = time_launches(torch, launch, n_sets, 10, 0, graph=False)
+            for i in range(min(4000, int(40 * 10 / max(t, 1e-2)))):
+                launch(i % n_sets)
+
     def pair(name, workload, nbytes, n_sets, product, floor, steps):
-        tp, _ = time_launches(torch, product, n_sets, steps, 10)
-        tf, _ = time_launches(torch, floor, n_sets, steps, 10)
-        up, uf = tp / steps * 1e3, tf / steps * 1e3
+        """Medians of five rounds of the two in turn."""
+        settled(product, n_sets)
+        rounds = [[time_launches(torch, f, n_sets, steps, 2)[0] / steps * 1e3 for f in (product, floor)] for _ in range(5)]
+        up, uf = (sorted(r[k] for r in rounds)[2] for k in (0, 1))
         res[name] = {"workload": workload, "kernel_us": round(up, 2), "floor_us": round(uf, 2),
                      "kernel_frac_of_floor": round(uf / up, 3), "floor_frac_of_peak": round(nbytes / (uf * 1e-6) / 8e12, 3)}
 
     def alt(name, workload, nbytes, n_sets, floor, steps, against):
         """A memory-only copy of a schedule the product does not use, timed on
-        the same buffers as `against`'s pair."""
-        tf, _ = time_launches(torch, floor, n_sets, steps, 10)
-        uf = tf / steps * 1e3
+        the same buffers as `against`'s pair; median of three."""
+        settled(floor, n_sets)
+        uf = sorted(time_launches(torch, floor, n_sets, steps, 2)[0] / steps * 1e3 for _ in range(3))[1]
         res[name] = {"workload": workload, "floor_us": round(uf, 2),
                      "floor_frac_of_peak": round(nbytes / (uf * 1e-6) / 8e12, 3),
                      "vs_product_floor": round(res[against]["floor_us"] / uf, 3)}

@@ -179,10 +179,12 @@ struct FloorItem {
   uint8_t* col_q;
   uint8_t* col_s;
   int64_t M, K;
-  int tiles_m, tiles, per_xcd;
+  int rows, units, per_xcd;  // rows of units, units, and each XCD's range of them
+  int shift, last;           // log2 of the tiles per unit; tiles of a unit of the last row
 };
 
 struct FloorGroup {
+  int share[8][kFloorGroupMax];  // each XCD's tiles of each item
   FloorItem item[kFloorGroupMax];
   int count;
 };
@@ -232,8 +234,10 @@ __device__ __forceinline__ void dual_tile_floor(const FloorItem& it, int64_t m0,
   if (SCM == 1 && a0 == 0x9E3779B9u) it.row_s[t] = 1;  // keeps the LDS reads
 }
 
-// The product's grouped order: each XCD takes its band-group share of each
-// item, item after item.
+// The product's order: each XCD takes its band-group share of each item, item
+// after item, in units of one tile or (more than 64 bands, as the product's
+// grouped kernel; its kernel for one tensor from six tiles per CU) of four
+// vertically adjacent ones, the last row of units last.
 template <int SCM>
 __global__ __launch_bounds__(512) void dual_grouped_floor(const FloorGroup g) {
   __shared__ __attribute__((aligned(16))) uint8_t tile[64 * 512];
@@ -241,15 +245,19 @@ __global__ __launch_bounds__(512) void dual_grouped_floor(const FloorGroup g) {
   const int b = blockIdx.x, xcd = b % 8;
   int j = b / 8, i = 0;
   for (; i < g.count; i++) {
-    const int n = min(max(g.item[i].tiles - xcd * g.item[i].per_xcd, 0), g.item[i].per_xcd);
+    const int n = g.share[xcd][i];
     if (j < n) break;
     j -= n;
   }
   if (i == g.count) return;
   const FloorItem& it = g.item[i];
+  const int lo = xcd * it.per_xcd, hi = min(it.units, lo + it.per_xcd), lasts = hi / it.rows - lo / it.rows;
+  const int upper = (hi - lo - lasts) << it.shift;  // tiles above the last row of units
+  const int unit = j < upper ? j >> it.shift : hi - lo - lasts + (j - upper) / it.last;
+  const int sub = j < upper ? j & ((1 << it.shift) - 1) : (j - upper) % it.last;
   int ms, kb;
-  if (!floor_band_group(xcd, j, it.tiles_m, it.tiles, it.per_xcd, &ms, &kb)) return;
-  dual_tile_floor<SCM>(it, (int64_t)ms * 64, (int64_t)kb * 256, tile, rs_tile);
+  if (!floor_band_group(xcd, unit, it.rows, it.units, it.per_xcd, &ms, &kb)) return;
+  dual_tile_floor<SCM>(it, (int64_t)((ms << it.shift) + sub) * 64, (int64_t)kb * 256, tile, rs_tile);
 }
 
 // ---- row -> col FP8, 128 x 256 tiles (row_to_fp8_col_wide_kernel, row_to_fp8_col_msplit_wide_kernel)
@@ -719,7 +727,7 @@ __attribute__((visibility("default"))) int omo_floor_dual_grouped(int scm, const
   FloorGroup g;
   memset(&g, 0, sizeof(g));
   g.count = count;
-  int64_t slots = 0;
+  int64_t slots[8] = {};
   for (int i = 0; i < count; i++) {
     if (M[i] <= 0 || K[i] <= 0 || M[i] % 64 || K[i] % 256 || (M[i] / 64) * (K[i] / 256) > 0x7FFFFFFF / 8) return -1;
     FloorItem& it = g.item[i];
@@ -730,13 +738,23 @@ __attribute__((visibility("default"))) int omo_floor_dual_grouped(int scm, const
     it.col_s = static_cast<uint8_t*>(col_s[i]);
     it.M = M[i];
     it.K = K[i];
-    it.tiles_m = (int)(M[i] / 64);
-    it.tiles = it.tiles_m * (int)(K[i] / 256);
-    it.per_xcd = (it.tiles + 7) / 8;
-    slots += it.per_xcd;
+    const int tiles_m = (int)(M[i] / 64), bands = (int)(K[i] / 256);
+    it.shift = bands > 64 ? 2 : 0;
+    it.rows = (tiles_m + (1 << it.shift) - 1) >> it.shift;
+    it.last = tiles_m - ((it.rows - 1) << it.shift);
+    it.units = it.rows * bands;
+    it.per_xcd = (it.units + 7) / 8;
+    for (int x = 0; x < 8; x++) {
+      const int lo = x * it.per_xcd, hi = lo + it.per_xcd < it.units ? lo + it.per_xcd : it.units;
+      if (lo < hi)
+        g.share[x][i] = ((hi - lo) << it.shift) - ((1 << it.shift) - it.last) * (hi / it.rows - lo / it.rows);
+      slots[x] += g.share[x][i];
+    }
   }
-  if (slots > 0x7FFFFFFF / 8) return -1;
-  hipLaunchKernelGGL(scm ? dual_grouped_floor<1> : dual_grouped_floor<0>, dim3((unsigned)(slots * 8)), dim3(512), 0,
+  int64_t most = 0;
+  for (const int64_t n : slots) most = n > most ? n : most;
+  if (most * 8 * 512 > 0xFFFFFFFFll) return -1;
+  hipLaunchKernelGGL(scm ? dual_grouped_floor<1> : dual_grouped_floor<0>, dim3((unsigned)(most * 8)), dim3(512), 0,
                      stream, g);
   return (int)hipGetLastError();
 }
