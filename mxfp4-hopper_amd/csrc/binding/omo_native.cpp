@@ -650,4 +650,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_omo_native", nullptr, -1, kMetho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__omo_native() { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__omo_native() {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "torch_version", OMO_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

@@ -330,3 +330,30 @@ def test_oversized_shapes_rejected():
                                            None))
     refused(lib.omo_hip_permute_Mxfp4ToFp8(f, 1 << 20, 1 << 40, f, 1 << 20, 1 << 36, 1, 1 << 40, f, 1 << 30, f, big,
                                            f, big, None))
+
+
+def test_binding_belongs_to_the_interpreter_that_builds(monkeypatch, tmp_path):
+    """build() names the running interpreter to make, whose paths the binding
+    is compiled against; the binding's file names it too, and a binding of
+    another torch is refused at import."""
+    import importlib.metadata
+    import subprocess
+    import sys
+
+    import __graft_entry__
+    from omo import _native
+    calls = []
+    monkeypatch.setattr(__graft_entry__.subprocess, "run", lambda cmd, **_: calls.append(cmd))
+    __graft_entry__.build()
+    assert any(f"PYTHON={sys.executable}" in cmd for cmd in calls)
+    monkeypatch.undo()
+    other = tmp_path / "other-python"  # stands for another interpreter: answers what make asks it
+    other.write_text('#!/bin/sh\ncase "$2" in *EXT_SUFFIX*) echo .other.so;; *torch*) echo /other/torch;; *) echo /other/include;; esac\n')
+    other.chmod(0o755)
+    plan = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "mxfp4-hopper_amd"), f"PYTHON={other}"],
+                          check=True, capture_output=True, text=True).stdout
+    assert "-isystem /other/include" in plan and "_omo_native.other.so" in plan
+    assert os.path.basename(_native.PATH) != "_omo_native.so"
+    monkeypatch.setattr(importlib.metadata, "version", lambda _: "0.0")
+    with pytest.raises(ImportError, match="built for torch"):
+        _native._load()
