@@ -346,7 +346,7 @@ struct DualItem {
 
 struct DualGroup {
   DualItem item[kDualGroupMax];
-  int count, tiles, c_eps;
+  int count, c_eps;
   float eps;
 };
 
@@ -456,7 +456,6 @@ hipError_t launch_quant_dual_grouped(const DualSpec* items, int count, float eps
       single = single && it.units.shift == 0;
     }
     if (tiles == 0) continue;
-    g.tiles = tiles;
     g.eps = eps;
     g.c_eps = host_c_eps(eps, 6.0f);
     const dim3 grid((unsigned)(*std::max_element(slots, slots + kXcds) * kXcds));

@@ -110,11 +110,11 @@ struct StageRegs {
 // Load the staging data of tile rows [row0, row0 + rows_valid), element
 // columns [col0, col0 + 128). Missing codes become 0; missing scales 127
 // (1.0), so out-of-tensor elements dequantize to exactly 0 on the fast path.
-// vin: 16 B vector code loads are allowed (N % 32 == 0, aligned base);
-// vs: a scale row's four bytes of the tile are one aligned dword
-// (N % 128 == 0, 4 B aligned base). The byte fallbacks keep exact bounds.
+// The codes, of any alignment and width, are loaded byte by byte. vs: a scale
+// row's four bytes of the tile are one aligned dword (N % 128 == 0, 4 B aligned
+// base); the byte fallback keeps exact bounds.
 __device__ __forceinline__ StageRegs rc_load(const uint8_t* __restrict__ q, const uint8_t* __restrict__ s, int64_t N,
-                                             int64_t row0, int rows_valid, int64_t col0, bool vin, bool vs) {
+                                             int64_t row0, int rows_valid, int64_t col0, bool vs) {
   const int t = threadIdx.x;
   const int64_t half = N / 2, sstride = N / 32;
   StageRegs g;
@@ -124,12 +124,8 @@ __device__ __forceinline__ StageRegs rc_load(const uint8_t* __restrict__ q, cons
     u32x4 w = {0u, 0u, 0u, 0u};
     if (r < rows_valid && gcol < N) {
       const uint8_t* src = q + (row0 + r) * half + gcol / 2;
-      if (vin && gcol + 32 <= N) {
-        w = *reinterpret_cast<const u32x4*>(src);
-      } else {
-        const int nb = (int)((N - gcol) / 2 < 16 ? (N - gcol) / 2 : 16);
-        for (int j = 0; j < nb; j++) w[j >> 2] |= (uint32_t)src[j] << (8 * (j & 3));
-      }
+      const int nb = (int)((N - gcol) / 2 < 16 ? (N - gcol) / 2 : 16);
+      for (int j = 0; j < nb; j++) w[j >> 2] |= (uint32_t)src[j] << (8 * (j & 3));
     }
     g.codes = w;
   }
@@ -146,20 +142,6 @@ __device__ __forceinline__ StageRegs rc_load(const uint8_t* __restrict__ q, cons
       }
     }
   }
-  return g;
-}
-
-// Staging loads of an interior tile when every tile is whole and aligned
-// (M % 128 == 0, N % 128 == 0, 16 B aligned codes, 4 B aligned scales):
-// unconditional vector loads only, so the compiler can count the waits for
-// them separately from the stores still in flight. Lanes 128..511 load a
-// copy of the scale dword of row t % 128, which they do not use.
-__device__ __forceinline__ StageRegs rc_load_full(const uint8_t* __restrict__ q, const uint8_t* __restrict__ s,
-                                                  int64_t N, int64_t row0, int64_t col0) {
-  const int t = threadIdx.x;
-  StageRegs g;
-  g.codes = *reinterpret_cast<const u32x4*>(q + (row0 + (t >> 2)) * (N / 2) + col0 / 2 + (t & 3) * 16);
-  g.scales = *reinterpret_cast<const uint32_t*>(s + (row0 + (t & (kTile - 1))) * (N / 32) + col0 / 32);
   return g;
 }
 
@@ -405,26 +387,23 @@ __device__ __forceinline__ void rc_store(uint8_t* __restrict__ dst, const RowByt
 
 // Persistent over tiles (tile = blockIdx.x + k * gridDim.x, tile_m fastest):
 // the next tile's codes and scales are loaded into registers while the
-// current tile is converted, so reads and writes overlap. FULL: every tile
-// is whole and aligned, and all loads and stores are unconditional vector
-// operations.
-template <bool FULL>
+// current tile is converted, so reads and writes overlap. For codes that the
+// 256-column tiles do not take.
 __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_kernel(const uint8_t* __restrict__ q,
                                                                     const uint8_t* __restrict__ s,
                                                                     uint8_t* __restrict__ out, float* __restrict__ out_s,
                                                                     int64_t M, int64_t N, int tiles_m, int tiles,
-                                                                    float eps, bool vin, bool vs) {
+                                                                    float eps, bool vs) {
   __shared__ RowColSmem sm;
   int tile = blockIdx.x;
   if (tile >= tiles) return;
   auto rows_of = [&](int tl) {
-    if (FULL) return kTile;
     const int64_t r0 = (int64_t)(tl % tiles_m) * kTile;
     return (int)(M - r0 < kTile ? M - r0 : kTile);
   };
   auto load = [&](int tl) {
     const int64_t r0 = (int64_t)(tl % tiles_m) * kTile, c0 = (int64_t)(tl / tiles_m) * kTile;
-    return FULL ? rc_load_full(q, s, N, r0, c0) : rc_load(q, s, N, r0, rows_of(tl), c0, vin, vs);
+    return rc_load(q, s, N, r0, rows_of(tl), c0, vs);
   };
   const int t = threadIdx.x, p = t >> 3, qq = t & 7;
   rc_put(sm, load(tile));
@@ -441,10 +420,7 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_kernel(const uint8_
     LaneCols res;
     rc_tile<false>(sm, rows_valid, N, col0, eps, eps, out_s + bm * N + col0, res);
     const int64_t c = col0 + 2 * p;
-    if (FULL) {
-      __builtin_nontemporal_store(res.e0, reinterpret_cast<u32x4*>(out + c * M + row0 + 16 * qq));
-      __builtin_nontemporal_store(res.e1, reinterpret_cast<u32x4*>(out + (c + 1) * M + row0 + 16 * qq));
-    } else if (c < N) {
+    if (c < N) {
       rc_store<16>(out + c * M + row0 + 16 * qq, res.e0, 16 * qq, rows_valid);
       rc_store<16>(out + (c + 1) * M + row0 + 16 * qq, res.e1, 16 * qq, rows_valid);
     }
@@ -1146,14 +1122,14 @@ __device__ __forceinline__ void msplit_narrow_tile(RowColSmem& sm, const uint8_t
                                                    const uint8_t* __restrict__ s, uint8_t* __restrict__ out,
                                                    float* __restrict__ out_s, int64_t len, int64_t start,
                                                    int64_t sstart, int64_t bm, int64_t bn, int64_t total_rows,
-                                                   int64_t N, int64_t out_s_rows, float eps, bool vin, bool vs) {
+                                                   int64_t N, int64_t out_s_rows, float eps, bool vs) {
   if (bm * kTile >= len) return;
   // Metadata arrives on the device; tiles whose rows or scale rows fall
   // outside the buffers are skipped rather than written out of bounds.
   if (start < 0 || start + len > total_rows || sstart < 0 || sstart + bm >= out_s_rows) return;
   const int64_t row0 = start + bm * kTile, col0 = bn * kTile;
   const int rows_valid = (int)(len - bm * kTile < kTile ? len - bm * kTile : kTile);
-  rc_put(sm, rc_load(q, s, N, row0, rows_valid, col0, vin, vs));
+  rc_put(sm, rc_load(q, s, N, row0, rows_valid, col0, vs));
   __syncthreads();
   LaneCols res;
   rc_tile<true>(sm, rows_valid, N, col0, 0.0f, eps, out_s + (sstart + bm) * N + col0, res);
@@ -1169,13 +1145,12 @@ __device__ __forceinline__ void msplit_narrow_tile(RowColSmem& sm, const uint8_t
 __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_kernel(
     const uint8_t* __restrict__ q, const uint8_t* __restrict__ s, uint8_t* __restrict__ out, float* __restrict__ out_s,
     const int32_t* __restrict__ lens, const int32_t* __restrict__ offs, const int32_t* __restrict__ soffs,
-    int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vin, bool vs, int64_t bm0, int64_t bn0) {
+    int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vs, int64_t bm0, int64_t bn0) {
   __shared__ RowColSmem sm;
   const int64_t split = blockIdx.x, bm = bm0 + blockIdx.y, bn = bn0 + blockIdx.z;
   const int64_t len = lens[split];
   if (bm * kTile >= len) return;
-  msplit_narrow_tile(sm, q, s, out, out_s, len, offs[split], soffs[split], bm, bn, total_rows, N, out_s_rows, eps, vin,
-                     vs);
+  msplit_narrow_tile(sm, q, s, out, out_s, len, offs[split], soffs[split], bm, bn, total_rows, N, out_s_rows, eps, vs);
 }
 
 // The 128-column tiles on the flat grid (at most 128 splits), as the wide
@@ -1188,12 +1163,12 @@ __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_kernel(
 template <int CHUNKS>
 __global__ __launch_bounds__(kRcThreads) void row_to_fp8_col_msplit_narrow_flat_kernel(
     const uint8_t* __restrict__ q, const uint8_t* __restrict__ s, uint8_t* __restrict__ out, float* __restrict__ out_s,
-    const DeviceSplits splits, int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vin, bool vs,
+    const DeviceSplits splits, int64_t total_rows, int64_t N, int64_t out_s_rows, float eps, bool vs,
     int nsplits, int tm, int bands) {
   __shared__ RowColSmem sm;
   int64_t len, start, sstart, bm, bn;
   if (!flat_split_tile<CHUNKS, false>(splits, nsplits, tm, bands, &len, &start, &sstart, &bm, &bn)) return;
-  msplit_narrow_tile(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, vin, vs);
+  msplit_narrow_tile(sm, q, s, out, out_s, len, start, sstart, bm, bn, total_rows, N, out_s_rows, eps, vs);
 }
 
 // Dynamic LDS, unused, that caps the residency of wide tiles with ragged
@@ -1210,17 +1185,13 @@ static size_t ragged_lds_reserve() {
 hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float* out_s, int64_t M, int64_t N, float eps,
                                  hipStream_t stream) {
   if (M == 0 || N == 0) return hipSuccess;
-  const bool vin = (N % 32 == 0) && ((reinterpret_cast<uintptr_t>(q) & 15) == 0);
-  const bool vs = (N % 128 == 0) && ((reinterpret_cast<uintptr_t>(s) & 3) == 0);
-  const bool vout = (M % 16 == 0) && ((reinterpret_cast<uintptr_t>(out) & 15) == 0);
-  const bool full = vin && vs && vout && (M % kTile == 0);
-  if (vin) {
+  if (N % 32 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
     // the 256-column tiles; their scale rows are read 8 bytes at a time when
     // 8 B aligned (N % 256 == 0), else byte by byte with the last band
     // partial. 4096 x 7040: 9.5 us against 12.6 us on the 128-column tiles;
     // 16384 x 7040: 29.2 against 56.0; 4096 x 2880: 5.6 against 8.4.
     const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
-    const bool whole = vout && M % kTile == 0;
+    const bool whole = M % kTile == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     const int64_t row_tiles = (M + kTile - 1) / kTile, bands = (N + kWideCols - 1) / kWideCols;
     const int64_t tiles = row_tiles * bands, cus = current_device_caps().cus;
     // Ragged: rows fastest while the tiles are one round of resident
@@ -1252,10 +1223,10 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
   // kernel's register use (4 waves per SIMD)
   const int64_t grid_cap = 2 * (int64_t)current_device_caps().cus;
   const int64_t grid = tiles < grid_cap ? tiles : grid_cap;
-  auto kernel = full ? row_to_fp8_col_kernel<true> : row_to_fp8_col_kernel<false>;
-  return launch(kernel, dim3((unsigned)grid), dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),
-                     static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M, N, (int)tiles_m, (int)tiles,
-                     eps, vin, vs);
+  const bool vs = N % 128 == 0 && (reinterpret_cast<uintptr_t>(s) & 3) == 0;
+  return launch(row_to_fp8_col_kernel, dim3((unsigned)grid), dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),
+                static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M, N, (int)tiles_m, (int)tiles, eps,
+                vs);
 }
 
 // The same for splits, but none where there are at most about the tiles of
@@ -1333,9 +1304,9 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
                                         int64_t out_s_rows, float eps, hipStream_t stream) {
   (void)out_capacity;  // the ABI layer checks out_capacity >= total_rows * N
   if (nsplits == 0 || max_split_len <= 0 || N == 0) return hipSuccess;
-  const bool vin = (N % 32 == 0) && ((reinterpret_cast<uintptr_t>(q) & 15) == 0);
-  const bool vs = (N % 128 == 0) && ((reinterpret_cast<uintptr_t>(s) & 3) == 0);
-  const bool wide = vin;  // 256-column tiles (the last band partial where N % 256 != 0)
+  // 256-column tiles (the last band partial where N % 256 != 0)
+  const bool wide = N % 32 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
+  const bool vs = N % 128 == 0 && (reinterpret_cast<uintptr_t>(s) & 3) == 0;
   const bool narrow_n = N % kWideCols != 0 || (reinterpret_cast<uintptr_t>(s) & 7) != 0;
   const int64_t tiles_m = (max_split_len + kTile - 1) / kTile;
   const int64_t bands = wide ? (N + kWideCols - 1) / kWideCols : (N + kTile - 1) / kTile;
@@ -1355,7 +1326,7 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
     auto kernel = nsplits <= 64 ? row_to_fp8_col_msplit_narrow_flat_kernel<1> : row_to_fp8_col_msplit_narrow_flat_kernel<2>;
     return launch(kernel, grid, dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),
                   static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, splits, total_rows, N,
-                  out_s_rows, eps, vin, vs, (int)nsplits, (int)tiles_m, (int)bands);
+                  out_s_rows, eps, vs, (int)nsplits, (int)tiles_m, (int)bands);
   }
   // Grid y (row tiles) and z (column bands) hold at most 65536 each: longer
   // splits or wider rows take several launches over offset ranges.
@@ -1370,7 +1341,7 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
                         out_s, lens, offs, soffs, total_rows, N, out_s_rows, eps, out_line, bm0, bn0)
                : launch(row_to_fp8_col_msplit_kernel, grid, dim3(kRcThreads), 0, stream,
                         static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out),
-                        out_s, lens, offs, soffs, total_rows, N, out_s_rows, eps, vin, vs, bm0, bn0);
+                        out_s, lens, offs, soffs, total_rows, N, out_s_rows, eps, vs, bm0, bn0);
       if (e != hipSuccess) return e;
     }
   }

@@ -48,10 +48,6 @@ SIGNATURES = {
     "omo_hip_packed_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _P, _I64, _P],
     "omo_hip_mxfp4_permute_rows": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],
     "omo_hip_permute_Mxfp4ToFp8": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _P],
-    "omo_hip_permute_Mxfp4ToFp8_copy": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _P, _I64, _P, _I64,
-                                        _P],
-    "omo_hip_route_counts": [_P, _I64, _I64, _P, _I64, _P, _P],
-    "omo_hip_route_rows": [_P, _I64, _I64, _P, _I64, _P, _I64, _I, _P, _I64, _P],
 }
 
 
