@@ -1,7 +1,10 @@
 """The row map of a routing map by the HIP kernels against the torch
 composition of the same map on the CPU: whole numbers, so every value."""
+import numpy as np
 import pytest
 import torch
+
+from helpers import bits_u8
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +52,34 @@ def test_row_map_forms(dev):
     for T, E in ((0, 4), (4, 0)):
         src, m_splits, dest = make_row_id_map(torch.zeros((T, E), dtype=torch.bool, device=dev), 3)
         assert src.tolist() == [-1] * 3 and m_splits == [0] * E and dest.shape == (T, E)
+
+
+# The row order that the fused requant copies out of its scratch (no row count
+# given): the 8-row tile and the 32-row one (from 512 tiles), with one column
+# of workgroups and with three (only the first copies), the last tile whole and
+# of 2, 7, 12 and 13 rows; on the current stream and on another.
+@pytest.mark.parametrize("T,H,E,k", [(301, 128, 12, 3), (4099, 128, 16, 4), (4096, 128, 8, 4), (2742, 1152, 8, 3),
+                                     (2735, 1280, 64, 3)])
+@pytest.mark.parametrize("side", [False, True])
+def test_copied_row_order(oracle, dev, T, H, E, k, side):
+    from omo._native import native
+    from omo_python_api.permutation import mxfp4_permute_to_fp8
+    print("copied row order", T, H, E, k, side, flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    rm = torch.zeros((T, E), dtype=torch.bool).scatter_(1, torch.rand((T, E), generator=g).topk(k, dim=1).indices, True)
+    q = torch.randint(0, 256, (T, H // 2), generator=g, dtype=torch.uint8)
+    s = torch.randint(118, 136, (T, H // 32), generator=g, dtype=torch.uint8)
+    e_idx, t_idx = np.nonzero(rm.numpy().T)
+    eo, es = oracle.mxfp4_to_fp8(q.numpy()[t_idx], s.numpy()[t_idx])
+    qd, sd, rmd = q.to(dev), s.to(dev), rm.to(dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream() if side else torch.cuda.current_stream()):
+        assert native.permute_to_fp8(qd, sd, rmd, None) is not None
+        for _ in range(2):  # the second call finds the first one's scratch in the allocator
+            f8, f8s, src, m_splits = mxfp4_permute_to_fp8(qd, sd, rmd, split=False)
+        torch.cuda.current_stream().synchronize()
+    assert m_splits == np.bincount(e_idx, minlength=E).tolist()
+    assert src.dtype == torch.int32 and src.untyped_storage().nbytes() == 4 * src.numel()
+    np.testing.assert_array_equal(src.cpu().numpy(), t_idx)
+    np.testing.assert_array_equal(bits_u8(f8), eo)
+    np.testing.assert_array_equal(f8s.cpu().numpy().view(np.uint32), es.view(np.uint32))
