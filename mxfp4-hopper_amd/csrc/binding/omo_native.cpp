@@ -537,9 +537,21 @@ RowMap row_map(const Tensor& map, int64_t T, int64_t E, int64_t num_out, bool wa
   return r;
 }
 
+// A routing map that the two row-map launches take and are the faster for. A
+// workgroup covers four experts and one of at most 64 chunks of tokens: one or
+// two experts of very many tokens leave the chip idle (row map and loads, us,
+// against the torch composition: 2^22 x 1 289 and 269, 3 * 2^20 x 1 202 and
+// 246, 2^23 x 2 641 and 620, 2^22 x 2 328 and 383; 2^24 x 4 1341 and 1565). And each
+// sums the counts before its own, so the work grows with the square of experts
+// times chunks (4096 x 65536 8691 and 2890, 4096 x 16384 959 and 881, 512 x
+// 65536 848 and 786; 4096 x 8192 400 and 528).
 Tensor plain_map(PyObject* o) {
   Tensor t = plain_matrix(o, at::kBool);
-  if (t.defined() && (t.size(0) >= ((int64_t)1 << 31) / t.size(1) || t.size(1) > 4 * 65534)) t.reset();
+  if (!t.defined()) return t;
+  const int64_t T = t.size(0), E = t.size(1);
+  if (T >= ((int64_t)1 << 31) / E || E > 4 * 65534 || (E <= 2 && T >= E << 22) ||
+      E * omo_hip_route_chunks(T, E) >= (int64_t)1 << 17)
+    t.reset();
   return t;
 }
 

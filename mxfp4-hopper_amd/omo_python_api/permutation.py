@@ -42,7 +42,8 @@ def make_row_id_map(routing_map: torch.Tensor, num_out_tokens: Optional[int] = N
 
 def _row_map_generic(rm: torch.Tensor, num_out_tokens: Optional[int]):
     """The row map by torch operations: routing maps on the CPU, empty ones,
-    ones past 2^31 pairs, tensor subclasses."""
+    ones past 2^31 pairs, tensor subclasses, and shapes that it does faster (one
+    or two experts of millions of tokens, tens of thousands of experts)."""
     T, E = rm.shape
     e_idx, t_idx = torch.nonzero(rm.t(), as_tuple=True)  # expert-major, ascending tokens
     n = t_idx.numel()

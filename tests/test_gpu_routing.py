@@ -34,6 +34,23 @@ def test_row_map(dev, T, E, p, pad):
     assert src.untyped_storage().nbytes() == 4 * src.numel()
 
 
+# Both sides of the maps that the torch composition does faster: one and two
+# experts of very many tokens, and very many experts (3 chunks of tokens).
+@pytest.mark.parametrize("T,E,p,takes", [(2**22 - 1, 1, 0.5, True), (2**22, 1, 0.5, False), (2**23 - 1, 2, 0.3, True),
+                                         (2**23, 2, 0.3, False), (2**22, 3, 0.3, True), (700, 43690, 2e-4, True),
+                                         (700, 43691, 2e-4, False)])
+def test_row_map_routes(dev, T, E, p, takes):
+    from omo._native import native
+    from omo_python_api.permutation import make_row_id_map
+    print("row map route", T, E, flush=True)
+    rm = _map(T, E, p, T + E)
+    rmd = rm.to(dev)
+    assert (native.make_row_map(rmd, None) is not None) == takes
+    src, m_splits, dest = make_row_id_map(rmd)
+    es, em, ed = make_row_id_map(rm)
+    assert m_splits == em and torch.equal(src.cpu(), es) and torch.equal(dest.cpu(), ed)
+
+
 def test_row_map_forms(dev):
     """Strided and misaligned maps, 0/1 maps of other types, too few rows."""
     from omo_python_api.permutation import make_row_id_map
