@@ -1200,11 +1200,34 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
     // 21.9 against 23.5; 8190 x 5120, 1280, 20.7 against 18.2). Bands fastest
     // where many CUs stay idle all the same (five tiles per eight CUs: 1000 x
     // 2880, 96 tiles, 5.2 us against 5.6 rows fastest, 1500 x 2880, 144, 5.9
-    // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1). Rows fastest too
-    // where the walk's grid, whole eighths, would pass the work-items of a
-    // launch and the tiles alone do not.
-    const bool walk = tiles > 5 * cus && (tiles + 7) / 8 * 8 <= (int64_t)UINT32_MAX / 256;
-    const DenseOrder order = whole || tiles <= cus * 5 / 8 ? kBandsFastest : walk ? kBandWalk : kRowsFastest;
+    // against 6.1; 700 x 7168, 168 tiles, 6.5 against 6.1).
+    // Beyond one round the walk pays where a row tile has several bands and a
+    // band several row tiles. Inputs past the cache, walk against the order
+    // taken instead: one tile of at most 64 rows (whose lanes take fewer rows
+    // in that form) 5 x 2^20 24.0 and 13.9 us; one band 300001 x 160 25.7 and
+    // 21.9, 2^20 - 6 x 32 42.5 and 34.0 (200003 x 256 22.5 and 22.9); at most
+    // eight row tiles 500 x 131072 43.4 and 30.6, 1000 x 131072 83.5 and 67.0;
+    // at most five bands of very many tiles 300001 x 288 46.5 and 39.4, 300001
+    // x 768 113.7 and 100.1, 200001 x 1280 130.7 and 110.9, 300001 x 512 71.7
+    // and 72.3 (524289 x 256 66.4 and 68.0). Rows fastest too where the walk's
+    // grid, whole eighths, would pass the work-items of a launch and the tiles
+    // alone do not. Inputs still in the Infinity Cache want bands fastest at
+    // many more sizes (9999 x 4096 12.4 us against 17.0, 16383 x 4096 20.9
+    // against 22.5; 16383 x 7168 51.3 against 45.4), those past it do not (22.5
+    // against 20.0, 33.2 against 29.2, 63.3 against 51.0), and a launch cannot
+    // tell.
+    const bool walks = bands > 1 && row_tiles > 8 && (tiles + 7) / 8 * 8 <= (int64_t)UINT32_MAX / 256;
+    const DenseOrder order = whole || tiles <= cus * 5 / 8            ? kBandsFastest
+                             : tiles <= 5 * cus                       ? kRowsFastest
+                             : M <= 64 || (bands <= 5 && bands > 1 && tiles > 14 * cus) ? kBandsFastest
+                             : walks                                  ? kBandWalk
+                                                                      : kRowsFastest;
+    // Rows of up to 16 bands with many tiles walk without the LDS reserve:
+    // 100001 x 2048 92.0 us against 101.6, 60001 x 4096 110.7 against 123.4,
+    // 60001 x 2560 68.8 against 75.9 (50001 x 2048, 3128 tiles, 47.2 against
+    // 46.8); wider or fewer with it: 16383 x 7168 50.8 against 53.3, 30001 x
+    // 2560, 2350 tiles, 34.1 against 34.6.
+    const size_t reserve = order == kBandWalk && (bands > 16 || tiles <= 12 * cus) ? ragged_lds_reserve() : 0;
     auto kernel = narrow_n ? (whole                    ? row_to_fp8_col_wide_kernel<false, true, kBandsFastest>
                               : order == kBandsFastest ? row_to_fp8_col_wide_kernel<true, true, kBandsFastest>
                               : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, true, kRowsFastest>
@@ -1214,7 +1237,7 @@ hipError_t launch_row_to_fp8_col(const void* q, const void* s, void* out, float*
                               : order == kRowsFastest  ? row_to_fp8_col_wide_kernel<true, false, kRowsFastest>
                                                        : row_to_fp8_col_wide_kernel<true, false, kBandWalk>);
     const int64_t grid = order == kBandWalk ? (tiles + 7) / 8 * 8 : tiles;
-    return launch(kernel, dim3((unsigned)grid), dim3(256), order == kBandWalk ? ragged_lds_reserve() : 0, stream,
+    return launch(kernel, dim3((unsigned)grid), dim3(256), reserve, stream,
                   static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s, M,
                   N, eps, (int)row_tiles, (int)bands);
   }

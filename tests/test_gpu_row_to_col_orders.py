@@ -17,7 +17,13 @@ FP8 = torch.float8_e4m3fn
 # are not whole lines.
 @pytest.mark.parametrize("M,N", [(128 * 159 + 1, 256), (128 * 160 + 1, 256), (129, 128 * 257), (1000, 2880),
                                  (128 * 6 - 1, 7168), (128 * 96 + 16, 4000), (128 * 1279 + 3, 256),
-                                 (128 * 1280 + 3, 256), (128 * 768 - 5, 288), (128 * 96 + 48, 4160)])
+                                 (128 * 1280 + 3, 256), (128 * 768 - 5, 288), (128 * 96 + 48, 4160),
+                                 # past 1280 tiles: one tile of at most 64 rows bands fastest, of more and up to
+                                 # eight row tiles rows fastest; five bands past 3584 tiles bands fastest, not past:
+                                 # the walk; up to 16 bands past 3072 tiles the walk without the LDS reserve
+                                 (33, 256 * 1281), (64, 256 * 1281 + 32), (65, 256 * 1281), (1001, 256 * 161 + 96),
+                                 (1025, 256 * 143), (128 * 716 + 1, 1280), (128 * 717 + 1, 1280), (128 * 512 + 1, 1536),
+                                 (128 * 193 + 77, 4096)])
 def test_ragged_orders(oracle, dev, M, N):
     import omo
     print("ragged order", M, N, flush=True)
