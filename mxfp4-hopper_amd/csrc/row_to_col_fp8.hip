@@ -1261,12 +1261,8 @@ static size_t split_lds_reserve(int64_t tiles) {
 }
 
 // The wide flat kernel's form for a split count and width: band walk on rows
-// of more than 16 bands up to `most` splits, else contiguous ranges. With
-// device lengths up to 64 splits. With lengths by value, whose grid has no
-// empty workgroups, up to 16: at 32 splits the ranges are ahead (16431 x 7168,
-// cold buffers, 52.7 us against 55.4; 8000 x 7168 28.6 against 30.4), at 16
-// the walk (52.6 against 51.8; 20000 x 7168 67.4 against 62.5).
-static bool split_walk(int64_t nsplits, int64_t bands, int64_t most) { return nsplits <= most && bands > 16; }
+// of more than 16 bands up to 64 splits, else contiguous ranges.
+static bool split_walk(int64_t nsplits, int64_t bands) { return nsplits <= 64 && bands > 16; }
 
 template <typename Splits>
 static auto split_flat_kernel(int64_t nsplits, bool walk, bool narrow_n) {
@@ -1279,7 +1275,13 @@ static auto split_flat_kernel(int64_t nsplits, bool walk, bool narrow_n) {
 }
 
 // The order and the grid of splits by value: exactly the tiles there are
-// (device lengths need nsplits times the longest split's).
+// (device lengths need nsplits times the longest split's). Without empty
+// workgroups the ranges are ahead of the walk past 16 splits while those are
+// of at most five row tiles on average (buffers past the cache: 16431 x 7168
+// in 64 54.4 us against 58.0, in 32 55.5 and 55.4; 8000 x 7168 in 32 28.3
+// against 31.6); of more, the walk is (16431 x 7168 in 24 53.5 against 57.5,
+// 40001 x 7168 in 64 123.0 against 131.5, 100001 x 7168 in 20 298 against 351),
+// and with few splits (16 of 16431 x 7168 51.8 against 52.6).
 struct ValueGrid {
   int64_t row_tiles, bands, blocks;
   bool walk;
@@ -1287,13 +1289,13 @@ struct ValueGrid {
 
 static ValueGrid value_grid(int64_t N, const int64_t* lens, int64_t nsplits) {
   ValueGrid g = {0, (N + kWideCols - 1) / kWideCols, 0, false};
-  g.walk = split_walk(nsplits, g.bands, 16);
   int64_t per_xcd = 0;
   for (int64_t i = 0; i < nsplits; i++) {
     const int64_t tiles = (lens[i] + kTile - 1) / kTile;
     g.row_tiles += tiles;
     per_xcd += (tiles * g.bands + 7) / 8;  // XCD 0 has the largest share of every split
   }
+  g.walk = split_walk(nsplits, g.bands) && (nsplits <= 16 || g.row_tiles > 5 * nsplits);
   g.blocks = g.walk ? 8 * per_xcd : g.row_tiles * g.bands;
   return g;
 }
@@ -1342,9 +1344,10 @@ hipError_t launch_row_to_fp8_col_msplit(const void* q, const void* s, void* out,
   if (nsplits <= kFlatMaxSplits && tiles_m * bands + 7 <= (int64_t)UINT32_MAX / flat_threads / nsplits) {
     const dim3 grid((unsigned)flat_grid_blocks(nsplits, tiles_m, bands));
     if (wide) {
-      return launch(split_flat_kernel<DeviceSplits>(nsplits, split_walk(nsplits, bands, 64), narrow_n), grid, dim3(256), reserve, stream,
-                    static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s), static_cast<uint8_t*>(out), out_s,
-                    splits, total_rows, N, out_s_rows, eps, out_line, (int)nsplits, (int)tiles_m, (int)bands);
+      return launch(split_flat_kernel<DeviceSplits>(nsplits, split_walk(nsplits, bands), narrow_n), grid, dim3(256),
+                    reserve, stream, static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(s),
+                    static_cast<uint8_t*>(out), out_s, splits, total_rows, N, out_s_rows, eps, out_line, (int)nsplits,
+                    (int)tiles_m, (int)bands);
     }
     auto kernel = nsplits <= 64 ? row_to_fp8_col_msplit_narrow_flat_kernel<1> : row_to_fp8_col_msplit_narrow_flat_kernel<2>;
     return launch(kernel, grid, dim3(kRcThreads), 0, stream, static_cast<const uint8_t*>(q),

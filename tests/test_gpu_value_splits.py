@@ -28,10 +28,13 @@ def _payload(M, N, seed):
 
 # One split and one row; zero lengths at both ends; 64 and 65 splits (one and
 # two lengths per lane), 128 (the most); 16 and 17 column bands and 16 and 17
-# splits (band walk and ranges); widths with whole, partial and single-chunk last bands.
+# splits (band walk and ranges), 17 and 64 of five row tiles each and of more
+# on average (ranges and walk); widths with whole, partial and single-chunk last bands.
 @pytest.mark.parametrize("lens,N", [([1], 32), ([0, 129, 0], 256), ([0, 0, 127, 128, 300, 0], 4352),
                                     (_lens(16, 900, 6), 4352), (_lens(17, 900, 7), 4352), (_lens(64, 900, 1), 4352),
                                     (_lens(65, 900, 2), 4352), (_lens(128, 1500, 3), 288),
+                                    ([640] * 17, 4352), ([640] * 16 + [641], 4352), ([515, 640] * 32, 4384),
+                                    ([0, 1280] * 32, 4384), ([0, 1281] * 31 + [0, 1537], 4384),
                                     (_lens(7, 2100, 4), 4096), (_lens(8, 4000, 5), 7040), ([512, 256], 4608)])
 def test_value_splits_match_oracle(oracle, dev, lens, N):
     import omo
