@@ -299,9 +299,14 @@ __device__ __forceinline__ bool band_group_tile(int xcd, int j, const BandUnits&
 // 2048 x 65536 77.5 us tile by tile, 72.1 in fours; 7168 x 18432 68.8 and
 // 69.0; 16384 x 7168 63.8 and 63.5. A kernel that kept four tiles' column
 // codes in registers and wrote whole lines (80 VGPRs, three workgroups per CU
-// where this one has four) took 72.3, 71.4 and 65.5 us there, 127.5 against
-// 118.9 at 28672 x 8192, and 84.3 against 79.1 at 7168 x 18432 after a 512 MB
-// fill.
+// where this one has four) is level or up to 2% ahead on some large tensors in
+// back-to-back launches and behind on others (2048 x 65536 73.2 us, this one
+// 74.7; 12288 x 12288 80.0, 81.3; 7168 x 18432 70.7, 71.1; 16384 x 18432 180.3,
+// 179.8; 16384 x 7168 65.7, 65.0; 5120 x 20480 60.4, 58.0; 28672 x 8192 128.2,
+// 124.3), and behind on all of them after a 512 MB fill (84.8, 84.0; 97.1,
+// 89.4; 84.8, 80.0; 185.1, 183.0; 76.4, 72.0; 70.3, 64.9; 151.0, 139.0). From
+// about 1.5 to 15 ms after a load begins the GPU's clocks dip; there it was
+// 1-4% ahead at 7168 x 18432 (blocks of 20 launches: 73-77 us, 73-82).
 constexpr int kDualQuadShift = 2;  // log2 of the tiles per unit
 
 // units.rows > 0: band groups over those units. Else each XCD takes a
