@@ -42,10 +42,10 @@ __device__ __forceinline__ void dual_floor_flush(const DualFloorSmem& sm, int bu
   }
 }
 
-// The product's band-group order, over super-tiles of 256 rows:
-// numbered M-fastest (L = band * S + super-row) are cut into eight
+// The product's band-group order, over units (super-tiles of 256 rows, or the
+// product's own): numbered M-fastest (L = band * S + unit row) they are cut into eight
 // contiguous ranges of per_xcd, one per XCD, and each XCD walks its range
-// super-row by super-row. False past the XCD's range.
+// unit row by unit row. False past the XCD's range.
 __device__ __forceinline__ bool floor_band_group(int xcd, int j, int S, int T, int per_xcd, int* ms, int* kb) {
   const int lo = xcd * per_xcd, hi = min(T, lo + per_xcd);
   if (j >= hi - lo) return false;
@@ -86,13 +86,13 @@ __device__ __forceinline__ bool floor_aligned_groups(int xcd, int j, int S, int 
 }
 
 // M % 256 == 0, K % 256 == 0, 16 B aligned buffers (the shapes the bench uses).
-// SCM 0: the product's scale stores (8 B per row per tile, 8 B per column per
+// SCM 0: its scale stores (8 B per row per tile, 8 B per column per
 // super-tile, ordinary stores); SCM 1: no scale stores (the bound the code
 // traffic alone sets); SCM 2: the same scale bytes written as whole lines,
 // each workgroup's 2 KB of row scales and 2 KB of column scales contiguous at
 // its tile number * 2048 with non-temporal 16 B stores - not the output
 // layout, the bound a layout-free scale store would set. ORDER 0: the
-// product's band-group order; 1: contiguous ranges of the M-fastest
+// band-group order; 1: contiguous ranges of the M-fastest
 // numbering per XCD (each XCD finishing one band before the next); 2:
 // contiguous ranges of the K-fastest numbering; 3: aligned groups
 // (floor_aligned_groups).
@@ -189,7 +189,7 @@ struct FloorGroup {
   int count;
 };
 
-// One tile's loads and stores as the product's one-tile kernel issues them
+// One tile's loads and stores as the product issues them
 // (M % 64 == 0, K % 256 == 0): four 16 B non-temporal loads per lane, then
 // four 4 B non-temporal row-code stores, 64 rows' 8 scale bytes gathered in
 // LDS and stored after the barrier, then per column pair two 8 B code stores
