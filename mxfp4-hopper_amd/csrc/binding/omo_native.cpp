@@ -555,6 +555,18 @@ Tensor plain_map(PyObject* o) {
   return t;
 }
 
+// Raises where the map's stream is being captured: the host has to read the
+// loads, and a counting launch recorded without that would write the pinned
+// counts again on every replay, whoever holds them by then.
+bool uncaptured(const Tensor& map) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(stream_of(map), &s);
+  if (e == hipSuccess && s == hipStreamCaptureStatusNone) return true;
+  PyErr_SetString(PyExc_RuntimeError,
+                  "the host reads the expert loads of a routing map: not permitted while its stream is being captured");
+  return false;
+}
+
 // None (-1) or a Python int in [0, 2^31).
 bool num_out_of(PyObject* o, int64_t* num_out) {
   *num_out = -1;
@@ -588,6 +600,7 @@ PyObject* make_row_map(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!map.defined() || !num_out_of(a[1], &num_out) || !quiet()) return none();
   const int64_t T = map.size(0), E = map.size(1);
   const c10::DeviceGuard guard(map.device());
+  if (!uncaptured(map)) return nullptr;
   RowMap m = unlocked([&] { return row_map(map, T, E, num_out, true, false); });
   if (!ok(m)) return nullptr;
   PyObject* loads = list_of_ints(m.loads);
@@ -623,6 +636,7 @@ PyObject* permute_to_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
       codes.device() != map.device() || scales.device() != map.device() || !quiet())
     return none();
   const c10::DeviceGuard guard(map.device());
+  if (!uncaptured(map)) return nullptr;
   RowMap m;
   Tensor src, q, s;
   const int status = unlocked([&]() -> int {

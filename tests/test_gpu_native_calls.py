@@ -296,3 +296,31 @@ def test_other_threads_run_while_a_call_allocates(dev, name):
         torch.cuda.synchronize()
     assert t1 - t0 > 0.05, "the allocation did not wait"
     assert sum(t0 < t < t1 for t in ticks) > 20 * (t1 - t0) / 0.1, (t1 - t0, len(ticks))
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_row_map_refuses_a_capturing_stream(dev, fused):
+    """The row map needs the host, so a capture refuses it before anything of
+    it is recorded; the capture goes on, and its replays touch no pinned memory."""
+    from omo_python_api.permutation import make_row_id_map, mxfp4_permute_to_fp8
+    print("row map under capture", fused, flush=True)
+    T, E = 4096, 16
+    q, s = _u8(dev, 0, 256, T, 64), _u8(dev, 120, 131, T, 4)
+    rm = torch.zeros((T, E), dtype=torch.bool, device=dev)
+    rm[::3, 2] = True
+    call = (lambda: mxfp4_permute_to_fp8(q, s, rm)) if fused else (lambda: make_row_id_map(rm))
+    call()
+    x = torch.zeros(4, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1
+        with pytest.raises(RuntimeError, match="captured"):
+            call()
+        x += 1
+    pinned = torch.empty((E * 16,), dtype=torch.int32, pin_memory=True).fill_(-7)  # of the counts' size
+    for _ in range(2):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [4.0] * 4 and (pinned == -7).all()
+    call()
